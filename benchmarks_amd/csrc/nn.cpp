@@ -81,7 +81,7 @@ double dot64(const double *x, const double *y, uint64_t n, DBuf<double> &part, h
 using namespace mfx;
 
 struct mfx_nn {
-  DBuf<float> w, m, v, grad, wr;
+  DBuf<float> w, m, v, grad, wr, wa;
   DBuf<uint16_t> wb;
   uint64_t wb_off[9] = {};
   int step = 0;
@@ -91,7 +91,7 @@ struct mfx_nn {
   uint32_t lv[4][3] = {};
   DBuf<uint16_t> e0, e1, e2, e3, d2, d1, d0;
   DBuf<float> x32, y32, dy;
-  DBuf<float> gd0, gu0, gd1, gu1, gd2, gu2, ge3, t2, ge2, t1, ge1, t0, ge0, part;
+  DBuf<float> gd0, gd1, gd2, ge3, ge2, ge1, ge0, part;  // gradients in slot order
   DBuf<double> lpart, dpart;
   DBuf<double> fr, fp, fq, fz;  // flexible CG
   // two-level mode: Chebyshev smoothing around the network
@@ -145,7 +145,7 @@ struct mfx_nn {
     if (packed) return;
     for (int l = 0; l < 8; ++l)
       nn_pack_weights(w.ptr + param_offset(l), wb.ptr + wb_off[l], wr.ptr + param_offset(l),
-                      kLayers[l].cin, kLayers[l].cout, kpad(l), s);
+                      wa.ptr + param_offset(l), kLayers[l].cin, kLayers[l].cout, kpad(l), s);
     packed = true;
   }
 
@@ -170,17 +170,11 @@ struct mfx_nn {
       const uint64_t P0 = count(lv[0]), P1 = count(lv[1]), P2 = count(lv[2]), P3 = count(lv[3]);
       dy.alloc(P0);
       gd0.alloc(P0 * 16);
-      gu0.alloc(P0 * 32);
       gd1.alloc(P1 * 32);
-      gu1.alloc(P1 * 64);
       gd2.alloc(P2 * 64);
-      gu2.alloc(P2 * 64);
       ge3.alloc(P3 * 64);
-      t2.alloc(P2 * 64);
       ge2.alloc(P2 * 64);
-      t1.alloc(P1 * 32);
       ge1.alloc(P1 * 32);
-      t0.alloc(P0 * 16);
       ge0.alloc(P0 * 16);
       if (!part.ptr) part.alloc(64ull * 27 * 64 * 64);
     }
@@ -188,6 +182,7 @@ struct mfx_nn {
 
   const uint16_t *wbl(int l) const { return wb.ptr + wb_off[l]; }
   const float *wrl(int l) const { return wr.ptr + param_offset(l); }
+  const float *wal(int l) const { return wa.ptr + param_offset(l); }
   float *gl(int l) { return grad.ptr + param_offset(l); }
 
   // y32 = network(x32) on the current grid
@@ -209,40 +204,33 @@ struct mfx_nn {
 
   // grad += dL/dW for dy = dL/dy (after forward on the same x32)
   void backward(hipStream_t s) {
-    const uint64_t P0 = count(lv[0]), P1 = count(lv[1]), P2 = count(lv[2]);
     nn_conv_wgrad(1, false, d0.ptr, nullptr, dy.ptr, part.ptr, gl(7), lv[0], lv[0], 16, 1,
                   parts_for(lv[0]), s);
     nn_head_backward(dy.ptr, wrl(7), d0.ptr, gd0.ptr, lv[0], s);
     // layer g: conv over up(d1) on level 0
     nn_conv_wgrad(1, true, d1.ptr, nullptr, gd0.ptr, part.ptr, gl(6), lv[0], lv[1], 32, 16,
                   parts_for(lv[0]), s);
-    nn_conv_adjoint(1, gd0.ptr, wrl(6), gu0.ptr, lv[0], lv[0], 32, 16, s);
-    nn_up_adjoint_mask(gu0.ptr, lv[0], nullptr, d1.ptr, gd1.ptr, lv[1], 32, s);
+    nn_conv_adjoint(6, gd0.ptr, wal(6), nullptr, d1.ptr, gd1.ptr, lv[0], lv[1], s);
     // layer f: conv over up(d2) on level 1
     nn_conv_wgrad(1, true, d2.ptr, nullptr, gd1.ptr, part.ptr, gl(5), lv[1], lv[2], 64, 32,
                   parts_for(lv[1]), s);
-    nn_conv_adjoint(1, gd1.ptr, wrl(5), gu1.ptr, lv[1], lv[1], 64, 32, s);
-    nn_up_adjoint_mask(gu1.ptr, lv[1], nullptr, d2.ptr, gd2.ptr, lv[2], 64, s);
+    nn_conv_adjoint(5, gd1.ptr, wal(5), nullptr, d2.ptr, gd2.ptr, lv[1], lv[2], s);
     // layer e: conv over up(e3) on level 2
     nn_conv_wgrad(1, true, e3.ptr, nullptr, gd2.ptr, part.ptr, gl(4), lv[2], lv[3], 64, 64,
                   parts_for(lv[2]), s);
-    nn_conv_adjoint(1, gd2.ptr, wrl(4), gu2.ptr, lv[2], lv[2], 64, 64, s);
-    nn_up_adjoint_mask(gu2.ptr, lv[2], nullptr, e3.ptr, ge3.ptr, lv[3], 64, s);
+    nn_conv_adjoint(4, gd2.ptr, wal(4), nullptr, e3.ptr, ge3.ptr, lv[2], lv[3], s);
     // layer d: stride-2 conv of e2
     nn_conv_wgrad(2, false, e2.ptr, nullptr, ge3.ptr, part.ptr, gl(3), lv[3], lv[2], 64, 64,
                   parts_for(lv[3]), s);
-    nn_conv_adjoint(2, ge3.ptr, wrl(3), t2.ptr, lv[3], lv[2], 64, 64, s);
-    nn_add_mask(gd2.ptr, t2.ptr, e2.ptr, ge2.ptr, P2 * 64, s);
+    nn_conv_adjoint(3, ge3.ptr, wal(3), gd2.ptr, e2.ptr, ge2.ptr, lv[3], lv[2], s);
     // layer c: stride-2 conv of e1
     nn_conv_wgrad(2, false, e1.ptr, nullptr, ge2.ptr, part.ptr, gl(2), lv[2], lv[1], 32, 64,
                   parts_for(lv[2]), s);
-    nn_conv_adjoint(2, ge2.ptr, wrl(2), t1.ptr, lv[2], lv[1], 32, 64, s);
-    nn_add_mask(gd1.ptr, t1.ptr, e1.ptr, ge1.ptr, P1 * 32, s);
+    nn_conv_adjoint(2, ge2.ptr, wal(2), gd1.ptr, e1.ptr, ge1.ptr, lv[2], lv[1], s);
     // layer b: stride-2 conv of e0
     nn_conv_wgrad(2, false, e0.ptr, nullptr, ge1.ptr, part.ptr, gl(1), lv[1], lv[0], 16, 32,
                   parts_for(lv[1]), s);
-    nn_conv_adjoint(2, ge1.ptr, wrl(1), t0.ptr, lv[1], lv[0], 16, 32, s);
-    nn_add_mask(gd0.ptr, t0.ptr, e0.ptr, ge0.ptr, P0 * 16, s);
+    nn_conv_adjoint(1, ge1.ptr, wal(1), gd0.ptr, e0.ptr, ge0.ptr, lv[1], lv[0], s);
     // layer a: the FP32 input
     nn_conv_wgrad(1, false, nullptr, x32.ptr, ge0.ptr, part.ptr, gl(0), lv[0], lv[0], 1, 16,
                   parts_for(lv[0]), s);
@@ -424,6 +412,7 @@ mfx_status mfx_nn_create(uint64_t seed, mfx_nn **out) {
     nn->v.upload(zero.data(), n);
     nn->grad.upload(zero.data(), n);
     nn->wr.alloc(n);
+    nn->wa.alloc(n);
     uint64_t off = 0;
     for (int l = 0; l < 8; ++l) {
       nn->wb_off[l] = off;

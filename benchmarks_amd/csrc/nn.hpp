@@ -13,13 +13,15 @@ namespace mfx {
 void nn_conv_forward(int layer, const uint16_t *in, const float *in32, const uint16_t *wb,
                      const float *wr, const uint16_t *skip, uint16_t *out, float *out32,
                      const uint32_t *od, const uint32_t *id, hipStream_t s);
-void nn_conv_adjoint(int stride, const float *G, const float *W, float *dX, const uint32_t *od,
-                     const uint32_t *xd, int cin, int cout, hipStream_t s);
-void nn_up_adjoint_mask(const float *fine, const uint32_t *fd, const float *add,
-                        const uint16_t *act, float *coarse, const uint32_t *cd, int C,
-                        hipStream_t s);
-void nn_add_mask(const float *a, const float *b, const uint16_t *act, float *out, uint64_t n,
-                 hipStream_t s);
+// Data gradient of layer 1..6 in slot order (nn_kernels.hip), masked by the
+// input activation act > 0.  Layers 1-3 (stride 2; xd the input grid): out =
+// add + the transposed convolution of G.  Layers 4-6 (od the fine grid of the
+// up-sampled input, xd the coarse input grid): out = the transposed
+// convolution summed over each coarse node's children; add unused.
+// wa: the weights as nn_pack_weights orders them.
+void nn_conv_adjoint(int layer, const float *G, const float *wa, const float *add,
+                     const uint16_t *act, float *out, const uint32_t *od, const uint32_t *xd,
+                     hipStream_t s);
 // grad += dL/dW of one layer; part: scratch of n_parts * 27 * cin * cout floats
 void nn_conv_wgrad(int stride, bool up, const uint16_t *in, const float *in32, const float *G,
                    float *part, float *grad, const uint32_t *od, const uint32_t *id, int cin,
@@ -31,7 +33,7 @@ void nn_mse(const float *y, const float *target, const uint8_t *mask, float scal
             double *part, uint64_t n, hipStream_t s);
 void nn_adam(float *w, float *m, float *v, const float *g, uint32_t n, float lr, float b1, float b2,
              float eps, int step, hipStream_t s);
-void nn_pack_weights(const float *w, uint16_t *wb, float *wr, int cin, int cout, int kp,
+void nn_pack_weights(const float *w, uint16_t *wb, float *wr, float *wa, int cin, int cout, int kp,
                      hipStream_t s);
 void nn_scale_to_f32(const double *r, float *out, double scale, uint64_t n, hipStream_t s);
 void nn_scale_to_f64(const float *y, double *z, double scale, uint64_t n, hipStream_t s);

@@ -46,6 +46,16 @@ __device__ __forceinline__ void decode(uint64_t i, const Dims &d, int &x, int &y
   z = (int)(q / d.y);
 }
 
+// the same for a 32-bit node index (node counts stay below 2^32: a grid of
+// that many nodes exceeds the device's memory)
+__device__ __forceinline__ void decode32(uint32_t i, const Dims &d, int &x, int &y, int &z) {
+  const uint32_t q = i / d.x;
+  x = (int)(i - q * d.x);
+  const uint32_t r = q / d.y;
+  y = (int)(q - r * d.y);
+  z = (int)r;
+}
+
 __device__ __forceinline__ bool inside(int x, int y, int z, const Dims &d) {
   return x >= 0 && y >= 0 && z >= 0 && x < (int)d.x && y < (int)d.y && z < (int)d.z;
 }
@@ -175,60 +185,197 @@ k_conv_last(const uint16_t *__restrict__ in, const float *__restrict__ W, float 
 }
 
 // ---------------------------------------------------------------- backward
-// dX[q][c] = sum_{t,o} W[o][t][c] G[(q - off_t) / s][o] over the taps whose
-// source lands on q; thread per (q, c).  dX is on the convolution's input
-// grid (the fine grid of an up-sampled input).
-template <int STRIDE>
-__global__ void __launch_bounds__(kBlock)
-k_conv_adjoint(const float *__restrict__ G, const float *__restrict__ W, float *__restrict__ dX,
-               Dims od, Dims xd, int cin, int cout) {
-  const uint64_t n = (uint64_t)xd.x * xd.y * xd.z * cin;
-  const uint64_t i = (uint64_t)blockIdx.x * kBlock + threadIdx.x;
-  if (i >= n) return;
-  const int c = (int)(i % cin);
-  int x, y, z;
-  decode(i / cin, xd, x, y, z);
-  float a = 0.f;
-  for (int t = 0; t < 27; ++t) {
-    const int rx = x - (t % 3 - 1), ry = y - ((t / 3) % 3 - 1), rz = z - (t / 9 - 1);
-    if (STRIDE == 2 && ((rx | ry | rz) & 1)) continue;
-    const int px = rx / STRIDE, py = ry / STRIDE, pz = rz / STRIDE;
-    if (rx < 0 || ry < 0 || rz < 0 || !inside(px, py, pz, od)) continue;
-    const float *g = G + lin(px, py, pz, od) * cout;
-    const float *w = W + (uint64_t)t * cin + c;
-    for (int o = 0; o < cout; ++o) a += w[(uint64_t)o * 27 * cin] * g[o];
+// Output gradients G are FP32 channels-last with a node's channels in slot
+// order: channel o of C at slot (o % 4) (C / 4) + o / 4, so that the lane
+// group g of a wave, which multiplies the channels o = 4 s + g (s = 0, 1, ...)
+// in v_mfma_f32_16x16x4_f32, reads its channels of four consecutive steps as
+// one 16-byte load.
+__device__ __forceinline__ int slot_of(int ch, int C) { return (ch & 3) * (C / 4) + (ch >> 2); }
+
+// one tap of the data gradient: acc[n] += G[rows][o] W[o][t][16 (nt0 + n) ..]
+// over the COUT channels in ascending order.  The FP32 MFMA adds its four
+// products to the accumulator one after the other with a rounding each (an
+// FMA chain, checked on the device), so the sums are those of a scalar loop
+// over (tap, channel).
+template <int COUT, int NT>
+struct AdjTap {
+  v4f a[COUT / 16], b[NT][COUT / 16];
+  // g: this lane's row at its channel group; w: the packed weights of the tap
+  // and of the wave's first 16 input channels
+  __device__ __forceinline__ void load(const float *g, const float *w, int lane) {
+#pragma unroll
+    for (int i = 0; i < COUT / 16; ++i) {
+      a[i] = *reinterpret_cast<const v4f *>(g + 4 * i);
+#pragma unroll
+      for (int n = 0; n < NT; ++n)
+        b[n][i] = *reinterpret_cast<const v4f *>(w + ((n * (COUT / 16) + i) * 64 + lane) * 4);
+    }
   }
-  dX[i] = a;
-}
-
-// coarse[j][c] = (sum over the fine children i of j of fine[i][c]) * mask
-// (mask: coarse activation > 0), optionally plus add[j][c] before the mask
-__global__ void __launch_bounds__(kBlock)
-k_up_adjoint_mask(const float *__restrict__ fine, Dims fd, const float *__restrict__ add,
-                  const uint16_t *__restrict__ act, float *__restrict__ coarse, Dims cd, int C) {
-  const uint64_t n = (uint64_t)cd.x * cd.y * cd.z * C;
-  const uint64_t i = (uint64_t)blockIdx.x * kBlock + threadIdx.x;
-  if (i >= n) return;
-  const int c = (int)(i % C);
-  int x, y, z;
-  decode(i / C, cd, x, y, z);
-  float a = add ? add[i] : 0.f;
-  for (int dz = 0; dz < 2; ++dz)
-    for (int dy = 0; dy < 2; ++dy)
-      for (int dx = 0; dx < 2; ++dx) {
-        const int fx = 2 * x + dx, fy = 2 * y + dy, fz = 2 * z + dz;
-        if (inside(fx, fy, fz, fd)) a += fine[lin(fx, fy, fz, fd) * C + c];
+  __device__ __forceinline__ void mac(bool on, v4f *acc) const {
+#pragma unroll
+    for (int i = 0; i < COUT / 16; ++i)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const float av = on ? a[i][j] : 0.f;
+#pragma unroll
+        for (int n = 0; n < NT; ++n)
+          acc[n] = __builtin_amdgcn_mfma_f32_16x16x4f32(av, b[n][i][j], acc[n], 0, 0, 0);
       }
-  coarse[i] = bf2f(act[i]) > 0.f ? a : 0.f;
+  }
+};
+
+// Data gradient of a stride-1 convolution over an up-sampled input, summed
+// to the coarse grid and masked: out[j][c] = (act[j][c] > 0) sum over the
+// fine children q of j of sum_{t,o} W[o][t][c] G[q - off_t][o].
+// A wave's 16 rows are the 8 children of 2 coarse nodes, its columns NT tiles
+// of 16 input channels; the children's sum is taken in the registers (the
+// fine-grid gradient is never stored).  Bound by the FP32 matrix rate on
+// large grids and by the chain of 27 COUT / 4 MFMAs on small ones; the taps'
+// operands are loaded a group of GT taps ahead.  On a 33^3 grid the three
+// layers take 17.5, 12.8 and 17.7 us, against 201 us on average (plus 4.8 us
+// for the children's sum) with one thread per output on the vector units.
+template <int CIN, int COUT, int NT, int GT>
+__global__ void __launch_bounds__(kBlock)
+k_adjoint_up(const float *__restrict__ G, const float *__restrict__ wa,
+             const uint16_t *__restrict__ act, float *__restrict__ out, Dims fd, Dims cd) {
+  static_assert(27 % GT == 0 && CIN % (16 * NT) == 0, "tile shape");
+  constexpr int WPN = CIN / 16 / NT;  // waves per node tile
+  const int lane = threadIdx.x & 63;
+  const uint32_t w = blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6);
+  const uint32_t tile = w / WPN;
+  const int nt0 = (int)(w % WPN) * NT;
+  const uint32_t P = cd.x * cd.y * cd.z;
+  if (tile >= (P + 1) / 2) return;
+  const int g = lane >> 4, m = lane & 15;
+  // this lane's row: child m % 8 of coarse node 2 tile + m / 8
+  uint32_t mask = 0;
+  const float *row = G + g * (COUT / 4);
+  {
+    const uint32_t j = 2 * tile + (m >> 3);
+    int X, Y, Z;
+    decode32(j, cd, X, Y, Z);
+    const int x = 2 * X + (m & 1), y = 2 * Y + ((m >> 1) & 1), z = 2 * Z + ((m >> 2) & 1);
+    if (j < P && inside(x, y, z, fd)) {
+      row += lin(x, y, z, fd) * COUT;
+#pragma unroll
+      for (int t = 0; t < 27; ++t)
+        if (inside(x - (t % 3 - 1), y - (t / 3 % 3 - 1), z - (t / 9 - 1), fd)) mask |= 1u << t;
+    }
+  }
+  const int64_t sy = (int64_t)fd.x * COUT, sz = sy * fd.y;
+  auto src = [&](int t) -> const float * {
+    const int64_t off = (t % 3 - 1) * COUT + (t / 3 % 3 - 1) * sy + (t / 9 - 1) * sz;
+    return (mask >> t & 1) ? row - off : row;  // an outside tap reads the row itself, unused
+  };
+  auto wgt = [&](int t) { return wa + (size_t)(t * (CIN / 16) + nt0) * COUT * 16; };
+  v4f acc[NT];
+#pragma unroll
+  for (int n = 0; n < NT; ++n) acc[n] = v4f{0.f, 0.f, 0.f, 0.f};
+  AdjTap<COUT, NT> cur[GT], nxt[GT];
+#pragma unroll
+  for (int k = 0; k < GT; ++k) cur[k].load(src(k), wgt(k), lane);
+#pragma unroll
+  for (int t = 0; t < 27; t += GT) {
+    if (t + GT < 27) {
+#pragma unroll
+      for (int k = 0; k < GT; ++k) nxt[k].load(src(t + GT + k), wgt(t + GT + k), lane);
+      __builtin_amdgcn_sched_barrier(0);  // keeps the loads ahead of the products
+    }
+#pragma unroll
+    for (int k = 0; k < GT; ++k) cur[k].mac(mask >> (t + k) & 1, acc);
+    if (t + GT < 27) {
+#pragma unroll
+      for (int k = 0; k < GT; ++k) cur[k] = nxt[k];
+    }
+  }
+  // rows 4 g .. 4 g + 3 are children 0-3 (even g) or 4-7 (odd g) of coarse
+  // node 2 tile + g / 2: summed in child order, the even group first
+  const uint32_t j = 2 * tile + (g >> 1);
+  int X, Y, Z;
+  decode32(j, cd, X, Y, Z);
+  const bool xi = 2 * X + 1 < (int)fd.x, yi = 2 * Y + 1 < (int)fd.y;
+  const bool zi = !(g & 1) || 2 * Z + 1 < (int)fd.z;
+#pragma unroll
+  for (int n = 0; n < NT; ++n) {
+    const bool in[4] = {zi, zi && xi, zi && yi, zi && xi && yi};
+    float s = 0.f;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) s = in[r] ? s + acc[n][r] : s;
+    s = __shfl(s, lane & 47, 64);  // odd groups: the even group's sum
+#pragma unroll
+    for (int r = 0; r < 4; ++r) s = in[r] ? s + acc[n][r] : s;
+    const int ch = (nt0 + n) * 16 + m;
+    if ((g & 1) && j < P)
+      out[(uint64_t)j * CIN + slot_of(ch, CIN)] =
+          bf2f(act[(uint64_t)j * CIN + ch]) > 0.f ? s : 0.f;
+  }
 }
 
-// out = (a + b) * (act > 0), elementwise (b optional)
-__global__ void k_add_mask(const float *__restrict__ a, const float *__restrict__ b,
-                           const uint16_t *__restrict__ act, float *__restrict__ out, uint64_t n) {
-  const uint64_t i = (uint64_t)blockIdx.x * kBlock + threadIdx.x;
-  if (i >= n) return;
-  const float v = a[i] + (b ? b[i] : 0.f);
-  out[i] = bf2f(act[i]) > 0.f ? v : 0.f;
+// Data gradient of a stride-2 convolution, added to `add` and masked:
+// out[q][c] = (act[q][c] > 0) (add[q][c] + sum_{t,o} W[o][t][c]
+// G[(q - off_t) / 2][o]) over the taps whose source lands on q.  A node's
+// taps depend on the parity of its coordinates only: even takes the middle
+// tap of its axis, odd the two outer ones.  blockIdx.y is the parity class,
+// so a wave's 16 rows share their 1, 2, 4 or 8 taps.  On a 33^3 grid 9.7-9.9
+// us per layer, against 119 us on average (plus 4.8 us for the masked sum)
+// with one thread per output on the vector units.
+template <int CIN, int COUT, int NT>
+__global__ void __launch_bounds__(kBlock)
+k_adjoint_down(const float *__restrict__ G, const float *__restrict__ wa,
+               const float *__restrict__ add, const uint16_t *__restrict__ act,
+               float *__restrict__ out, Dims od, Dims xd) {
+  constexpr int WPN = CIN / 16 / NT;
+  const int cx = blockIdx.y & 1, cy = blockIdx.y >> 1 & 1, cz = blockIdx.y >> 2;
+  const Dims kd{(xd.x + 1 - cx) / 2, (xd.y + 1 - cy) / 2, (xd.z + 1 - cz) / 2};  // class grid
+  const uint32_t P = kd.x * kd.y * kd.z;
+  const int lane = threadIdx.x & 63;
+  const uint32_t w = blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6);
+  const uint32_t tile = w / WPN;
+  const int nt0 = (int)(w % WPN) * NT;
+  if (tile >= (P + 15) / 16) return;
+  const int g = lane >> 4, m = lane & 15;
+  int ix, iy, iz;
+  const bool valid = tile * 16 + m < P;
+  decode32(valid ? tile * 16 + m : 0, kd, ix, iy, iz);
+  const int n_taps = (1 + cx) << (cy + cz);
+  // tap i of the class, ascending: along an odd axis first tap 0 (source
+  // node i + 1), then tap 2 (source i); along an even one tap 1 (source i)
+  bool on_cur, on_nxt = false;
+  AdjTap<COUT, NT> cur, nxt;
+  auto load = [&](int i, AdjTap<COUT, NT> &v) -> bool {
+    const int kx = cx ? i & 1 : 1, ky = cy ? (i >> cx) & 1 : 1, kz = cz ? i >> (cx + cy) : 1;
+    const int px = ix + 1 - kx, py = iy + 1 - ky, pz = iz + 1 - kz;
+    const int t = (cx ? 2 * kx : 1) + 3 * (cy ? 2 * ky : 1) + 9 * (cz ? 2 * kz : 1);
+    const bool on = valid && inside(px, py, pz, od);
+    v.load(G + (on ? lin(px, py, pz, od) : 0) * COUT + g * (COUT / 4),
+           wa + (size_t)(t * (CIN / 16) + nt0) * COUT * 16, lane);
+    return on;
+  };
+  v4f acc[NT];
+#pragma unroll
+  for (int n = 0; n < NT; ++n) acc[n] = v4f{0.f, 0.f, 0.f, 0.f};
+  on_cur = load(0, cur);
+  for (int i = 0; i < n_taps; ++i) {
+    if (i + 1 < n_taps) on_nxt = load(i + 1, nxt);
+    __builtin_amdgcn_sched_barrier(0);
+    cur.mac(on_cur, acc);
+    cur = nxt;
+    on_cur = on_nxt;
+  }
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    const uint32_t i = tile * 16 + 4 * g + r;
+    if (i >= P) continue;
+    decode32(i, kd, ix, iy, iz);
+    const uint64_t q = lin(2 * ix + cx, 2 * iy + cy, 2 * iz + cz, xd) * CIN;
+#pragma unroll
+    for (int n = 0; n < NT; ++n) {
+      const int ch = (nt0 + n) * 16 + m;
+      const uint64_t at = q + slot_of(ch, CIN);
+      const float v = add[at] + acc[n][r];
+      out[at] = bf2f(act[q + ch]) > 0.f ? v : 0.f;
+    }
+  }
 }
 
 // partial weight gradients: block (t, part) sums over its node range
@@ -263,7 +410,7 @@ k_conv_wgrad(const uint16_t *__restrict__ in, const float *__restrict__ in32,
           const int64_t s = tap_source<STRIDE, UP>(x, y, z, t, od, id);
           if (s >= 0) xv = in32 ? in32[s] : bf2f(in[(uint64_t)s * cin + c]);
         }
-        if (c < cout) gv = G[p * cout + c];
+        if (c < cout) gv = G[p * cout + (cout % 4 ? c : slot_of(c, cout))];
       }
       sX[j][c] = xv;
       sG[j][c] = gv;
@@ -344,7 +491,7 @@ k_conv_wgrad_mfma(const uint16_t *__restrict__ in, const float *__restrict__ G,
     for (int a = 0; a < OT; ++a) {
       uint16_t h[8];
 #pragma unroll
-      for (int q = 0; q < 8; ++q) h[q] = pt[q] < p1 ? f2bf(G[pt[q] * COUT + a * 16 + li]) : 0;
+      for (int q = 0; q < 8; ++q) h[q] = pt[q] < p1 ? f2bf(G[pt[q] * COUT + slot_of(a * 16 + li, COUT)]) : 0;
       const uint4 raw = make_uint4(h[0] | (uint32_t)h[1] << 16, h[2] | (uint32_t)h[3] << 16,
                                    h[4] | (uint32_t)h[5] << 16, h[6] | (uint32_t)h[7] << 16);
       ag[a] = __builtin_bit_cast(v8bf, raw);
@@ -406,7 +553,7 @@ k_conv_wgrad_thin(const uint16_t *__restrict__ in, const float *__restrict__ in3
       const float xv = in32[src];
       const float *g = G + p * 16;
 #pragma unroll
-      for (int k = 0; k < 16; ++k) acc[k] += g[k] * xv;
+      for (int k = 0; k < 16; ++k) acc[k] += g[slot_of(k, 16)] * xv;
     }
   }
 #pragma unroll
@@ -442,22 +589,37 @@ __global__ void k_wgrad_reduce(const float *__restrict__ part, float *__restrict
   grad[w] += s;
 }
 
-// head backward: g[p][c] = (sum_t W[t][c] dy[p - off_t]) * (act[p][c] > 0)
+// head backward: g[p][c] = (sum_t W[t][c] dy[p - off_t]) * (act[p][c] > 0),
+// stored in slot order.  A wave holds 64 nodes and the four channels c = 4 j +
+// wave (one 16-byte store), with the weights in scalar registers; the taps
+// outside the grid are left out of the sum.
 __global__ void __launch_bounds__(kBlock)
 k_head_backward(const float *__restrict__ dy, const float *__restrict__ W,
                 const uint16_t *__restrict__ act, float *__restrict__ g, Dims d) {
-  const uint64_t n = (uint64_t)d.x * d.y * d.z * 16;
-  const uint64_t i = (uint64_t)blockIdx.x * kBlock + threadIdx.x;
-  if (i >= n) return;
-  const int c = (int)(i % 16);
+  const uint32_t P = d.x * d.y * d.z;
+  const uint32_t i = blockIdx.x * 64 + (threadIdx.x & 63);
+  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  if (i >= P) return;
   int x, y, z;
-  decode(i / 16, d, x, y, z);
-  float a = 0.f;
+  decode32(i, d, x, y, z);
+  float v[27];
+  uint32_t mask = 0;
+#pragma unroll
   for (int t = 0; t < 27; ++t) {
     const int px = x - (t % 3 - 1), py = y - ((t / 3) % 3 - 1), pz = z - (t / 9 - 1);
-    if (inside(px, py, pz, d)) a += W[t * 16 + c] * dy[lin(px, py, pz, d)];
+    const bool on = inside(px, py, pz, d);
+    mask |= (uint32_t)on << t;
+    v[t] = dy[on ? lin(px, py, pz, d) : i];
   }
-  g[i] = bf2f(act[i]) > 0.f ? a : 0.f;
+  v4f o;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    float a = 0.f;
+#pragma unroll
+    for (int t = 0; t < 27; ++t) a = (mask >> t & 1) ? a + W[t * 16 + 4 * j + wv] * v[t] : a;
+    o[j] = bf2f(act[(uint64_t)i * 16 + 4 * j + wv]) > 0.f ? a : 0.f;
+  }
+  *reinterpret_cast<v4f *>(g + (uint64_t)i * 16 + 4 * wv) = o;
 }
 
 // loss pieces: dy = scale (y - target) on free nodes (0 on masked nodes),
@@ -499,9 +661,12 @@ __global__ void k_adam(float *__restrict__ w, float *__restrict__ m, float *__re
 }
 
 // layer weights [o][t][c] FP32 -> bf16 [o][KP] (k = t cin + c, zero padded)
-// and the FP32 value of each bf16 weight [o][t][c]
+// and the FP32 value of each bf16 weight [o][t][c]; with wa (channel counts
+// that are multiples of 16) also the FP32 value in the order AdjTap reads it:
+// [t][c / 16][o / 16][lane 16 (o % 4) + c % 16][(o / 4) % 4]
 __global__ void k_pack_weights(const float *__restrict__ w, uint16_t *__restrict__ wb,
-                               float *__restrict__ wr, int cin, int cout, int kp) {
+                               float *__restrict__ wr, float *__restrict__ wa, int cin, int cout,
+                               int kp) {
   const int n = cout * kp;
   const int i = blockIdx.x * kBlock + threadIdx.x;
   if (i >= n) return;
@@ -511,6 +676,11 @@ __global__ void k_pack_weights(const float *__restrict__ w, uint16_t *__restrict
   if (k < K) {
     h = f2bf(w[o * K + k]);
     wr[o * K + k] = bf2f(h);
+    if (wa) {
+      const int t = k / cin, c = k - t * cin;
+      wa[((((t * (cin / 16) + c / 16) * (cout / 16) + o / 16) * 64 + (o & 3) * 16 + c % 16) * 4) +
+         ((o >> 2) & 3)] = bf2f(h);
+    }
   }
   wb[i] = h;
 }
@@ -564,30 +734,38 @@ void nn_conv_forward(int layer, const uint16_t *in, const float *in32, const uin
   MFX_HIP(hipGetLastError());
 }
 
-void nn_conv_adjoint(int stride, const float *G, const float *W, float *dX, const uint32_t *od,
-                     const uint32_t *xd, int cin, int cout, hipStream_t s) {
-  const uint64_t n = (uint64_t)xd[0] * xd[1] * xd[2] * cin;
-  if (stride == 1)
-    hipLaunchKernelGGL(k_conv_adjoint<1>, dim3(blocks(n)), dim3(kBlock), 0, s, G, W, dX, D3(od),
-                       D3(xd), cin, cout);
-  else
-    hipLaunchKernelGGL(k_conv_adjoint<2>, dim3(blocks(n)), dim3(kBlock), 0, s, G, W, dX, D3(od),
-                       D3(xd), cin, cout);
-  MFX_HIP(hipGetLastError());
+namespace {
+template <int CIN, int COUT, int NT, int GT>
+void adjoint_up(const float *G, const float *wa, const uint16_t *act, float *out,
+                const uint32_t *fd, const uint32_t *cd, hipStream_t s) {
+  const uint64_t tiles = ((uint64_t)cd[0] * cd[1] * cd[2] + 1) / 2;
+  hipLaunchKernelGGL((k_adjoint_up<CIN, COUT, NT, GT>), dim3(blocks(tiles * (CIN / 16 / NT) * 64)),
+                     dim3(kBlock), 0, s, G, wa, act, out, D3(fd), D3(cd));
 }
-
-void nn_up_adjoint_mask(const float *fine, const uint32_t *fd, const float *add,
-                        const uint16_t *act, float *coarse, const uint32_t *cd, int C,
-                        hipStream_t s) {
-  const uint64_t n = (uint64_t)cd[0] * cd[1] * cd[2] * C;
-  hipLaunchKernelGGL(k_up_adjoint_mask, dim3(blocks(n)), dim3(kBlock), 0, s, fine, D3(fd), add, act,
-                     coarse, D3(cd), C);
-  MFX_HIP(hipGetLastError());
+template <int CIN, int COUT, int NT>
+void adjoint_down(const float *G, const float *wa, const float *add, const uint16_t *act,
+                  float *out, const uint32_t *od, const uint32_t *xd, hipStream_t s) {
+  // the all-even parity class is the largest
+  const uint64_t n = (uint64_t)((xd[0] + 1) / 2) * ((xd[1] + 1) / 2) * ((xd[2] + 1) / 2);
+  hipLaunchKernelGGL((k_adjoint_down<CIN, COUT, NT>),
+                     dim3(blocks((n + 15) / 16 * (CIN / 16 / NT) * 64), 8), dim3(kBlock), 0, s, G,
+                     wa, add, act, out, D3(od), D3(xd));
 }
+}  // namespace
 
-void nn_add_mask(const float *a, const float *b, const uint16_t *act, float *out, uint64_t n,
-                 hipStream_t s) {
-  hipLaunchKernelGGL(k_add_mask, dim3(blocks(n)), dim3(kBlock), 0, s, a, b, act, out, n);
+void nn_conv_adjoint(int layer, const float *G, const float *wa, const float *add,
+                     const uint16_t *act, float *out, const uint32_t *od, const uint32_t *xd,
+                     hipStream_t s) {
+  // input-channel tiles per wave (NT): two where the grid has waves enough
+  switch (layer) {
+    case 1: adjoint_down<16, 32, 1>(G, wa, add, act, out, od, xd, s); break;
+    case 2: adjoint_down<32, 64, 1>(G, wa, add, act, out, od, xd, s); break;
+    case 3: adjoint_down<64, 64, 1>(G, wa, add, act, out, od, xd, s); break;
+    case 4: adjoint_up<64, 64, 1, 1>(G, wa, act, out, od, xd, s); break;
+    case 5: adjoint_up<64, 32, 2, 1>(G, wa, act, out, od, xd, s); break;
+    case 6: adjoint_up<32, 16, 2, 3>(G, wa, act, out, od, xd, s); break;
+    default: throw Error{MFX_ERR_INVALID_ARG, "layer has no data gradient"};
+  }
   MFX_HIP(hipGetLastError());
 }
 
@@ -644,8 +822,8 @@ void nn_conv_wgrad(int stride, bool up, const uint16_t *in, const float *in32, c
 
 void nn_head_backward(const float *dy, const float *W, const uint16_t *act, float *g,
                       const uint32_t *d, hipStream_t s) {
-  const uint64_t n = (uint64_t)d[0] * d[1] * d[2] * 16;
-  hipLaunchKernelGGL(k_head_backward, dim3(blocks(n)), dim3(kBlock), 0, s, dy, W, act, g, D3(d));
+  const uint64_t n = (uint64_t)d[0] * d[1] * d[2];
+  hipLaunchKernelGGL(k_head_backward, dim3((unsigned)((n + 63) / 64)), dim3(kBlock), 0, s, dy, W, act, g, D3(d));
   MFX_HIP(hipGetLastError());
 }
 
@@ -668,10 +846,11 @@ void nn_adam(float *w, float *m, float *v, const float *g, uint32_t n, float lr,
   MFX_HIP(hipGetLastError());
 }
 
-void nn_pack_weights(const float *w, uint16_t *wb, float *wr, int cin, int cout, int kp,
+void nn_pack_weights(const float *w, uint16_t *wb, float *wr, float *wa, int cin, int cout, int kp,
                      hipStream_t s) {
+  if (cin % 16 || cout % 16) wa = nullptr;
   hipLaunchKernelGGL(k_pack_weights, dim3(blocks((uint64_t)cout * kp)), dim3(kBlock), 0, s, w, wb,
-                     wr, cin, cout, kp);
+                     wr, wa, cin, cout, kp);
   MFX_HIP(hipGetLastError());
 }
 
