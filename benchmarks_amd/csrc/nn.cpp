@@ -52,9 +52,10 @@ struct LayerDesc {
 constexpr LayerDesc kLayers[8] = {{1, 16}, {16, 32}, {32, 64}, {64, 64},
                                   {64, 64}, {64, 32}, {32, 16}, {16, 1}};
 
+uint64_t n_weights(int l) { return 27ull * kLayers[l].cin * kLayers[l].cout; }
 uint64_t param_offset(int l) {
   uint64_t o = 0;
-  for (int k = 0; k < l; ++k) o += 27ull * kLayers[k].cin * kLayers[k].cout;
+  for (int k = 0; k < l; ++k) o += n_weights(k);
   return o;
 }
 uint64_t n_params_total() { return param_offset(8); }
@@ -176,14 +177,13 @@ struct mfx_nn {
       ge2.alloc(P2 * 64);
       ge1.alloc(P1 * 32);
       ge0.alloc(P0 * 16);
-      if (!part.ptr) part.alloc(64ull * 27 * 64 * 64);
+      if (part.n < part_floats()) part.alloc(part_floats());
     }
   }
 
   const uint16_t *wbl(int l) const { return wb.ptr + wb_off[l]; }
   const float *wrl(int l) const { return wr.ptr + param_offset(l); }
   const float *wal(int l) const { return wa.ptr + param_offset(l); }
-  float *gl(int l) { return grad.ptr + param_offset(l); }
 
   // y32 = network(x32) on the current grid
   void forward(hipStream_t s) {
@@ -198,42 +198,37 @@ struct mfx_nn {
     nn_conv_forward(7, d0.ptr, nullptr, nullptr, wrl(7), nullptr, nullptr, y32.ptr, lv[0], lv[0], s);
   }
 
-  static uint32_t parts_for(const uint32_t *d) {
-    return (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>(64, count(d) / 2048));
+  // output grid level of each layer
+  static constexpr int kOut[8] = {0, 1, 2, 3, 2, 1, 0, 0};
+  // partial weight gradients of all layers
+  uint64_t part_floats() const {
+    uint64_t n = 0;
+    for (int l = 0; l < 8; ++l) n += nn_wgrad_parts(l, lv[kOut[l]]) * n_weights(l);
+    return n;
   }
 
   // grad += dL/dW for dy = dL/dy (after forward on the same x32)
   void backward(hipStream_t s) {
-    nn_conv_wgrad(1, false, d0.ptr, nullptr, dy.ptr, part.ptr, gl(7), lv[0], lv[0], 16, 1,
-                  parts_for(lv[0]), s);
+    // data gradients, from the head down to the input layer's output
     nn_head_backward(dy.ptr, wrl(7), d0.ptr, gd0.ptr, lv[0], s);
-    // layer g: conv over up(d1) on level 0
-    nn_conv_wgrad(1, true, d1.ptr, nullptr, gd0.ptr, part.ptr, gl(6), lv[0], lv[1], 32, 16,
-                  parts_for(lv[0]), s);
     nn_conv_adjoint(6, gd0.ptr, wal(6), nullptr, d1.ptr, gd1.ptr, lv[0], lv[1], s);
-    // layer f: conv over up(d2) on level 1
-    nn_conv_wgrad(1, true, d2.ptr, nullptr, gd1.ptr, part.ptr, gl(5), lv[1], lv[2], 64, 32,
-                  parts_for(lv[1]), s);
     nn_conv_adjoint(5, gd1.ptr, wal(5), nullptr, d2.ptr, gd2.ptr, lv[1], lv[2], s);
-    // layer e: conv over up(e3) on level 2
-    nn_conv_wgrad(1, true, e3.ptr, nullptr, gd2.ptr, part.ptr, gl(4), lv[2], lv[3], 64, 64,
-                  parts_for(lv[2]), s);
     nn_conv_adjoint(4, gd2.ptr, wal(4), nullptr, e3.ptr, ge3.ptr, lv[2], lv[3], s);
-    // layer d: stride-2 conv of e2
-    nn_conv_wgrad(2, false, e2.ptr, nullptr, ge3.ptr, part.ptr, gl(3), lv[3], lv[2], 64, 64,
-                  parts_for(lv[3]), s);
     nn_conv_adjoint(3, ge3.ptr, wal(3), gd2.ptr, e2.ptr, ge2.ptr, lv[3], lv[2], s);
-    // layer c: stride-2 conv of e1
-    nn_conv_wgrad(2, false, e1.ptr, nullptr, ge2.ptr, part.ptr, gl(2), lv[2], lv[1], 32, 64,
-                  parts_for(lv[2]), s);
     nn_conv_adjoint(2, ge2.ptr, wal(2), gd1.ptr, e1.ptr, ge1.ptr, lv[2], lv[1], s);
-    // layer b: stride-2 conv of e0
-    nn_conv_wgrad(2, false, e0.ptr, nullptr, ge1.ptr, part.ptr, gl(1), lv[1], lv[0], 16, 32,
-                  parts_for(lv[1]), s);
     nn_conv_adjoint(1, ge1.ptr, wal(1), gd0.ptr, e0.ptr, ge0.ptr, lv[1], lv[0], s);
-    // layer a: the FP32 input
-    nn_conv_wgrad(1, false, nullptr, x32.ptr, ge0.ptr, part.ptr, gl(0), lv[0], lv[0], 1, 16,
-                  parts_for(lv[0]), s);
+    // weight gradients: input and output gradient of each layer
+    const uint16_t *in[8] = {nullptr, e0.ptr, e1.ptr, e2.ptr, e3.ptr, d2.ptr, d1.ptr, d0.ptr};
+    const float *G[8] = {ge0.ptr, ge1.ptr, ge2.ptr, ge3.ptr, gd2.ptr, gd1.ptr, gd0.ptr, dy.ptr};
+    const int in_level[8] = {0, 0, 1, 2, 3, 2, 1, 0};
+    NnWgrad l[8];
+    float *p = part.ptr;
+    for (int k = 0; k < 8; ++k) {
+      l[k] = NnWgrad{in[k], G[k], p, lv[kOut[k]], lv[in_level[k]],
+                     nn_wgrad_parts(k, lv[kOut[k]]), (uint32_t)n_weights(k)};
+      p += l[k].n_parts * n_weights(k);
+    }
+    nn_wgrad(l, x32.ptr, grad.ptr, s);
   }
 
   // z = ||r|| s y(r / ||r||) on a box operator's node grid; constrained rows

@@ -22,10 +22,18 @@ void nn_conv_forward(int layer, const uint16_t *in, const float *in32, const uin
 void nn_conv_adjoint(int layer, const float *G, const float *wa, const float *add,
                      const uint16_t *act, float *out, const uint32_t *od, const uint32_t *xd,
                      hipStream_t s);
-// grad += dL/dW of one layer; part: scratch of n_parts * 27 * cin * cout floats
-void nn_conv_wgrad(int stride, bool up, const uint16_t *in, const float *in32, const float *G,
-                   float *part, float *grad, const uint32_t *od, const uint32_t *id, int cin,
-                   int cout, uint32_t n_parts, hipStream_t s);
+// grad += dL/dW of all layers (G: output gradients in slot order, layer 7:
+// dy; in: the layer's bf16 input, layer 0: nullptr with x32).  part: scratch
+// of n_parts x n_weights floats per layer, n_parts = nn_wgrad_parts.
+struct NnWgrad {
+  const uint16_t *in;
+  const float *G;
+  float *part;
+  const uint32_t *od, *id;
+  uint32_t n_parts, n_weights;
+};
+uint32_t nn_wgrad_parts(int layer, const uint32_t *od);
+void nn_wgrad(const NnWgrad (&l)[8], const float *x32, float *grad, hipStream_t s);
 void nn_head_backward(const float *dy, const float *W, const uint16_t *act, float *g,
                       const uint32_t *d, hipStream_t s);
 uint32_t nn_mse_blocks(uint64_t n);

@@ -9,11 +9,12 @@
 // and, with up-sampling, in = up(v), up(v)[i] = v[i >> 1] per direction.
 //
 // Forward (implicit GEMM on v_mfma_f32_16x16x32_bf16): a wavefront owns 16
-// consecutive output nodes and all output channels; the K dimension
+// consecutive output nodes and NT tiles of 16 output channels; the K dimension
 // (t, c) runs in chunks of 32: lane l gathers 8 consecutive channels of one
 // tap of node l % 16 (one 16-byte load, channels-last) as the A operand and
-// 8 consecutive k of output channel l % 16 of the weights [o][k] as the B
-// operand.  D register r of lane l is node 4 (l / 16) + r, channel l % 16.
+// 8 consecutive k of output channel l % 16 as the B operand, whose weights are
+// stored in lane order.  D register r of lane l is node 4 (l / 16) + r,
+// channel l % 16.
 #include <algorithm>
 
 #include "mfx_internal.hpp"
@@ -39,16 +40,9 @@ struct Dims {
   uint32_t x, y, z;
 };
 
-__device__ __forceinline__ void decode(uint64_t i, const Dims &d, int &x, int &y, int &z) {
-  x = (int)(i % d.x);
-  const uint64_t q = i / d.x;
-  y = (int)(q % d.y);
-  z = (int)(q / d.y);
-}
-
-// the same for a 32-bit node index (node counts stay below 2^32: a grid of
-// that many nodes exceeds the device's memory)
-__device__ __forceinline__ void decode32(uint32_t i, const Dims &d, int &x, int &y, int &z) {
+// coordinates of node i (node counts stay below 2^32: a grid of that many
+// nodes exceeds the device's memory)
+__device__ __forceinline__ void decode(uint32_t i, const Dims &d, int &x, int &y, int &z) {
   const uint32_t q = i / d.x;
   x = (int)(i - q * d.x);
   const uint32_t r = q / d.y;
@@ -79,61 +73,136 @@ __device__ __forceinline__ int64_t tap_source(int x, int y, int z, int t, const 
   return (int64_t)lin(qx, qy, qz, id);
 }
 
-template <int CIN, int COUT, int STRIDE, bool UP, bool SKIP>
+// The chunks' operands are loaded in groups of GC, one group ahead of the
+// products (the sums keep one accumulator per output and the order of k).  On
+// the grids the preconditioner uses a layer has few waves, each a chain of
+// 27 CIN / 32 products: what bounds it is the latency of the gathered loads,
+// so NT = 1 spreads the channels over waves and the groups keep 2 GC loads
+// in flight.  33^3 grid: the six layers take 4.2, 6.3, 10.9, 7.7, 8.3 and 9.9
+// us, against 9, 15, 31, 33, 22 and 15 us with all channel tiles in one wave
+// and one chunk's loads at a time.
+template <int CIN, int COUT, int STRIDE, bool UP, int NT>
 __global__ void __launch_bounds__(kBlock)
 k_conv_mfma(const uint16_t *__restrict__ in, const uint16_t *__restrict__ W,
             const uint16_t *__restrict__ skip, uint16_t *__restrict__ out, Dims od, Dims id) {
-  static_assert(CIN % 16 == 0 && COUT % 16 == 0, "channel counts must be multiples of 16");
-  constexpr int K = 27 * CIN, KP = (K + 31) / 32 * 32, NT = COUT / 16;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const uint64_t P = (uint64_t)od.x * od.y * od.z;
-  const uint64_t base = ((uint64_t)blockIdx.x * (kBlock / 64) + wave) * 16;
-  if (base >= P) return;
-  const uint64_t node = base + (lane & 15);
-  int x = 0, y = 0, z = 0;
-  const bool valid = node < P;
-  if (valid) decode(node, od, x, y, z);
-  const int kl = 8 * (lane >> 4);
+  static_assert(CIN % 16 == 0 && CIN <= 64 && COUT % (16 * NT) == 0, "channel tiles");
+  constexpr int NC = (27 * CIN + 31) / 32;           // chunks of 32 k
+  constexpr int GC = CIN == 16 ? (NT == 1 ? 7 : 2) : (NT == 1 ? 9 : 3), WPN = COUT / 16 / NT;
+  static_assert(NC % GC == 0, "chunk groups");
+  const int lane = threadIdx.x & 63, g = lane >> 4, li = lane & 15;
+  const uint32_t w = blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6);
+  const uint32_t P = od.x * od.y * od.z, tile = w / WPN;
+  const int nt0 = (int)(w % WPN) * NT;
+  if (tile >= (P + 15) / 16) return;
+  const uint32_t node = tile * 16 + li;
+  // the lane's input rows: element offsets of the three taps per axis and the
+  // mask of the taps inside the grid
+  const Dims bd = UP ? od : id;
+  int xo[3];
+  int64_t yo[3], zo[3];
+  uint32_t mask = 0;
+  {
+    int x, y, z;
+    decode(node < P ? node : 0, od, x, y, z);
+    bool vx[3], vy[3], vz[3];
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+      const int qx = STRIDE * x + k - 1, qy = STRIDE * y + k - 1, qz = STRIDE * z + k - 1;
+      vx[k] = qx >= 0 && qx < (int)bd.x;
+      vy[k] = qy >= 0 && qy < (int)bd.y;
+      vz[k] = qz >= 0 && qz < (int)bd.z;
+      xo[k] = (vx[k] ? UP ? qx >> 1 : qx : 0) * CIN;
+      yo[k] = (int64_t)(vy[k] ? UP ? qy >> 1 : qy : 0) * id.x * CIN;
+      zo[k] = (int64_t)(vz[k] ? UP ? qz >> 1 : qz : 0) * id.x * id.y * CIN;
+    }
+#pragma unroll
+    for (int t = 0; t < 27; ++t)
+      mask |= (uint32_t)(vx[t % 3] && vy[t / 3 % 3] && vz[t / 9]) << t;
+    if (node >= P) mask = 0;
+  }
+  auto off = [&](int t) { return xo[t % 3] + yo[t / 3 % 3] + zo[t / 9]; };
+  // chunk i of the lane: tap and channels (CIN = 16: two taps per chunk, the
+  // upper half of the wave on the second one)
+  auto load_a = [&](int i, bool &on) -> uint4 {
+    int64_t o;
+    if constexpr (CIN == 16) {
+      const int t0 = 2 * i, t1 = 2 * i + 1;
+      const bool hi = g >> 1;
+      const int64_t o0 = off(t0), d = t1 < 27 ? off(t1 < 27 ? t1 : 26) - o0 : 0;
+      o = o0 + (hi ? d : 0) + 8 * (g & 1);
+      on = hi ? (t1 < 27 && (mask >> t1 & 1)) : (mask >> t0 & 1);
+    } else {
+      const int t = i * 32 / CIN;
+      o = off(t) + i * 32 % CIN + 8 * g;
+      on = mask >> t & 1;
+    }
+    return *reinterpret_cast<const uint4 *>(in + o);
+  };
+  // weights of chunk i, channel tile n: [chunk][tile][lane][8]
+  auto load_b = [&](int i, int n) {
+    return *reinterpret_cast<const uint4 *>(
+        W + ((size_t)(i * (COUT / 16) + nt0 + n) * 64 + lane) * 8);
+  };
   v4f acc[NT];
 #pragma unroll
   for (int n = 0; n < NT; ++n) acc[n] = v4f{0.f, 0.f, 0.f, 0.f};
-  for (int kc = 0; kc < KP; kc += 32) {
-    const int k = kc + kl;
-    uint4 araw = make_uint4(0, 0, 0, 0);
-    if (valid && k < K) {
-      const int t = k / CIN, c = k - t * CIN;
-      const int64_t src = tap_source<STRIDE, UP>(x, y, z, t, od, id);
-      if (src >= 0) araw = *reinterpret_cast<const uint4 *>(in + (uint64_t)src * CIN + c);
-    }
-    const v8bf a = __builtin_bit_cast(v8bf, araw);
+  uint16_t sk[NT][4];
+  if (UP) {
 #pragma unroll
-    for (int n = 0; n < NT; ++n) {
-      const uint4 braw =
-          *reinterpret_cast<const uint4 *>(W + (uint64_t)(n * 16 + (lane & 15)) * KP + k);
-      acc[n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, __builtin_bit_cast(v8bf, braw), acc[n], 0,
-                                                       0, 0);
+    for (int n = 0; n < NT; ++n)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const uint32_t o = min(tile * 16 + 4 * g + r, P - 1);
+        sk[n][r] = skip[(uint64_t)o * COUT + (nt0 + n) * 16 + li];
+      }
+  }
+  uint4 a[2][GC], b[2][GC][NT];
+  bool on[2][GC];
+  auto load = [&](int i0, int buf) {
+#pragma unroll
+    for (int k = 0; k < GC; ++k) {
+      a[buf][k] = load_a(i0 + k, on[buf][k]);
+#pragma unroll
+      for (int n = 0; n < NT; ++n) b[buf][k][n] = load_b(i0 + k, n);
+    }
+  };
+  load(0, 0);
+#pragma unroll
+  for (int i0 = 0; i0 < NC; i0 += GC) {
+    const int cur = i0 / GC & 1;
+    if (i0 + GC < NC) load(i0 + GC, cur ^ 1);
+    __builtin_amdgcn_sched_barrier(0);  // keeps the loads ahead of the products
+#pragma unroll
+    for (int k = 0; k < GC; ++k) {
+      const uint4 z = a[cur][k];
+      const bool v = on[cur][k];
+      const uint4 av = make_uint4(v ? z.x : 0, v ? z.y : 0, v ? z.z : 0, v ? z.w : 0);
+#pragma unroll
+      for (int n = 0; n < NT; ++n)
+        acc[n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+            __builtin_bit_cast(v8bf, av), __builtin_bit_cast(v8bf, b[cur][k][n]), acc[n], 0, 0, 0);
     }
   }
-  // epilogue: node base + 4 (lane / 16) + r, channel n * 16 + lane % 16
 #pragma unroll
   for (int n = 0; n < NT; ++n)
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
-      const uint64_t o = base + 4 * (lane >> 4) + r;
+      const uint32_t o = tile * 16 + 4 * g + r;
       if (o >= P) continue;
-      const int ch = n * 16 + (lane & 15);
       float v = acc[n][r];
-      if (SKIP) v += bf2f(skip[o * COUT + ch]);
-      out[o * COUT + ch] = f2bf(fmaxf(v, 0.f));
+      if (UP) v += bf2f(sk[n][r]);
+      out[(uint64_t)o * COUT + (nt0 + n) * 16 + li] = f2bf(fmaxf(v, 0.f));
     }
 }
 
-// first layer: one FP32 input channel -> 16, ReLU; thread per node
+// first layer: one FP32 input channel -> 16, ReLU; a wave holds 64 nodes and
+// four of the channels (one 8-byte store), weights in scalar registers
 __global__ void __launch_bounds__(kBlock)
 k_conv_first(const float *__restrict__ in, const float *__restrict__ W, uint16_t *__restrict__ out,
              Dims d) {
-  const uint64_t P = (uint64_t)d.x * d.y * d.z;
-  const uint64_t i = (uint64_t)blockIdx.x * kBlock + threadIdx.x;
+  const uint32_t P = d.x * d.y * d.z;
+  const uint32_t i = blockIdx.x * 64 + (threadIdx.x & 63);
+  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   if (i >= P) return;
   int x, y, z;
   decode(i, d, x, y, z);
@@ -141,44 +210,58 @@ k_conv_first(const float *__restrict__ in, const float *__restrict__ W, uint16_t
 #pragma unroll
   for (int t = 0; t < 27; ++t) {
     const int64_t s = tap_source<1, false>(x, y, z, t, d, d);
-    v[t] = s >= 0 ? in[s] : 0.f;
+    v[t] = in[s >= 0 ? s : (int64_t)i];
+    v[t] = s >= 0 ? v[t] : 0.f;
   }
-  uint16_t o[16];
+  uint16_t o[4];
 #pragma unroll
-  for (int c = 0; c < 16; ++c) {
+  for (int c = 0; c < 4; ++c) {
     float a = 0.f;
 #pragma unroll
-    for (int t = 0; t < 27; ++t) a += W[c * 27 + t] * v[t];
+    for (int t = 0; t < 27; ++t) a += W[(4 * wv + c) * 27 + t] * v[t];
     o[c] = f2bf(fmaxf(a, 0.f));
   }
-  uint32_t pk[8];
-#pragma unroll
-  for (int c = 0; c < 8; ++c) pk[c] = (uint32_t)o[2 * c] | ((uint32_t)o[2 * c + 1] << 16);
-  uint4 *dst = reinterpret_cast<uint4 *>(out + i * 16);
-  dst[0] = make_uint4(pk[0], pk[1], pk[2], pk[3]);
-  dst[1] = make_uint4(pk[4], pk[5], pk[6], pk[7]);
+  *reinterpret_cast<uint2 *>(out + (uint64_t)i * 16 + 4 * wv) =
+      make_uint2((uint32_t)o[0] | (uint32_t)o[1] << 16, (uint32_t)o[2] | (uint32_t)o[3] << 16);
 }
 
-// last layer: 16 -> 1 FP32 output, no activation; thread per node
+// last layer: 16 -> 1 FP32 output, no activation; thread per node, a plane of
+// nine taps loaded ahead of its products (one FMA chain over taps and channels;
+// taps outside the grid are left out)
 __global__ void __launch_bounds__(kBlock)
 k_conv_last(const uint16_t *__restrict__ in, const float *__restrict__ W, float *__restrict__ out,
             Dims d) {
-  const uint64_t P = (uint64_t)d.x * d.y * d.z;
-  const uint64_t i = (uint64_t)blockIdx.x * kBlock + threadIdx.x;
+  const uint32_t P = d.x * d.y * d.z;
+  const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
   if (i >= P) return;
   int x, y, z;
   decode(i, d, x, y, z);
   float a = 0.f;
-  for (int t = 0; t < 27; ++t) {
-    const int64_t s = tap_source<1, false>(x, y, z, t, d, d);
-    if (s < 0) continue;
-    const uint4 *src = reinterpret_cast<const uint4 *>(in + (uint64_t)s * 16);
-    const uint4 lo = src[0], hi = src[1];
-    const uint32_t w32[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
+  uint4 v[2][9][2];
+  auto load = [&](int tz, int buf) {
 #pragma unroll
-    for (int c = 0; c < 16; ++c) {
-      const uint16_t h = (uint16_t)(w32[c >> 1] >> (16 * (c & 1)));
-      a += W[t * 16 + c] * bf2f(h);
+    for (int t = 0; t < 9; ++t) {
+      const int64_t s = tap_source<1, false>(x, y, z, 9 * tz + t, d, d);
+      const uint4 *src = reinterpret_cast<const uint4 *>(in + (s >= 0 ? s : (int64_t)i) * 16);
+      v[buf][t][0] = src[0];
+      v[buf][t][1] = src[1];
+    }
+  };
+  load(0, 0);
+#pragma unroll
+  for (int tz = 0; tz < 3; ++tz) {
+    if (tz < 2) load(tz + 1, (tz + 1) & 1);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int t = 0; t < 9; ++t) {
+      const uint4 lo = v[tz & 1][t][0], hi = v[tz & 1][t][1];
+      const uint32_t w32[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
+      float s = a;
+#pragma unroll
+      for (int c = 0; c < 16; ++c)
+        s += W[(9 * tz + t) * 16 + c] *
+             bf2f((uint16_t)(w32[c >> 1] >> (16 * (c & 1))));
+      a = tap_source<1, false>(x, y, z, 9 * tz + t, d, d) >= 0 ? s : a;
     }
   }
   out[i] = a;
@@ -253,7 +336,7 @@ k_adjoint_up(const float *__restrict__ G, const float *__restrict__ wa,
   {
     const uint32_t j = 2 * tile + (m >> 3);
     int X, Y, Z;
-    decode32(j, cd, X, Y, Z);
+    decode(j, cd, X, Y, Z);
     const int x = 2 * X + (m & 1), y = 2 * Y + ((m >> 1) & 1), z = 2 * Z + ((m >> 2) & 1);
     if (j < P && inside(x, y, z, fd)) {
       row += lin(x, y, z, fd) * COUT;
@@ -292,7 +375,7 @@ k_adjoint_up(const float *__restrict__ G, const float *__restrict__ wa,
   // node 2 tile + g / 2: summed in child order, the even group first
   const uint32_t j = 2 * tile + (g >> 1);
   int X, Y, Z;
-  decode32(j, cd, X, Y, Z);
+  decode(j, cd, X, Y, Z);
   const bool xi = 2 * X + 1 < (int)fd.x, yi = 2 * Y + 1 < (int)fd.y;
   const bool zi = !(g & 1) || 2 * Z + 1 < (int)fd.z;
 #pragma unroll
@@ -336,7 +419,7 @@ k_adjoint_down(const float *__restrict__ G, const float *__restrict__ wa,
   const int g = lane >> 4, m = lane & 15;
   int ix, iy, iz;
   const bool valid = tile * 16 + m < P;
-  decode32(valid ? tile * 16 + m : 0, kd, ix, iy, iz);
+  decode(valid ? tile * 16 + m : 0, kd, ix, iy, iz);
   const int n_taps = (1 + cx) << (cy + cz);
   // tap i of the class, ascending: along an odd axis first tap 0 (source
   // node i + 1), then tap 2 (source i); along an even one tap 1 (source i)
@@ -366,7 +449,7 @@ k_adjoint_down(const float *__restrict__ G, const float *__restrict__ wa,
   for (int r = 0; r < 4; ++r) {
     const uint32_t i = tile * 16 + 4 * g + r;
     if (i >= P) continue;
-    decode32(i, kd, ix, iy, iz);
+    decode(i, kd, ix, iy, iz);
     const uint64_t q = lin(2 * ix + cx, 2 * iy + cy, 2 * iz + cz, xd) * CIN;
 #pragma unroll
     for (int n = 0; n < NT; ++n) {
@@ -378,180 +461,161 @@ k_adjoint_down(const float *__restrict__ G, const float *__restrict__ wa,
   }
 }
 
-// partial weight gradients: block (t, part) sums over its node range
-//   dW[o][t][c] += G[p][o] * in(s p + off_t)[c]
-// in: bf16 channels-last (or FP32 when cin == 1 and in32 is set)
-template <int STRIDE, bool UP>
-__global__ void __launch_bounds__(kBlock)
-k_conv_wgrad(const uint16_t *__restrict__ in, const float *__restrict__ in32,
-             const float *__restrict__ G, float *__restrict__ part, Dims od, Dims id, int cin,
-             int cout, uint32_t n_parts) {
-  constexpr int PC = 16;  // nodes staged per round
-  __shared__ float sX[PC][64];
-  __shared__ float sG[PC][64];
-  const int t = blockIdx.x;
-  const uint32_t pi = blockIdx.y;
-  const uint64_t P = (uint64_t)od.x * od.y * od.z;
-  const uint64_t p0 = P * pi / n_parts, p1 = P * (pi + 1) / n_parts;
-  const int nout = cin * cout;  // <= 4096: up to 16 per thread
-  float acc[16];
-#pragma unroll
-  for (int k = 0; k < 16; ++k) acc[k] = 0.f;
-  for (uint64_t pb = p0; pb < p1; pb += PC) {
-    __syncthreads();
-    for (int e = threadIdx.x; e < PC * 64; e += kBlock) {
-      const int j = e / 64, c = e % 64;
-      const uint64_t p = pb + j;
-      float xv = 0.f, gv = 0.f;
-      if (p < p1) {
-        int x, y, z;
-        decode(p, od, x, y, z);
-        if (c < cin) {
-          const int64_t s = tap_source<STRIDE, UP>(x, y, z, t, od, id);
-          if (s >= 0) xv = in32 ? in32[s] : bf2f(in[(uint64_t)s * cin + c]);
-        }
-        if (c < cout) gv = G[p * cout + (cout % 4 ? c : slot_of(c, cout))];
-      }
-      sX[j][c] = xv;
-      sG[j][c] = gv;
-    }
-    __syncthreads();
-#pragma unroll
-    for (int k = 0; k < 16; ++k) {
-      const int idx = threadIdx.x + k * kBlock;
-      if (idx >= nout) break;
-      const int o = idx / cin, c = idx - o * cin;
-      float s = acc[k];
-#pragma unroll
-      for (int j = 0; j < PC; ++j) s += sG[j][o] * sX[j][c];
-      acc[k] = s;
-    }
-  }
-#pragma unroll
-  for (int k = 0; k < 16; ++k) {
-    const int idx = threadIdx.x + k * kBlock;
-    if (idx >= nout) break;
-    const int o = idx / cin, c = idx - o * cin;
-    part[((uint64_t)pi * cout + o) * 27 * cin + (uint64_t)t * cin + c] = acc[k];
-  }
-}
+// Weight gradients dW[o][t][c] = sum_p G[p][o] X(s p + off_t)[c] of all layers
+// in one launch (WgradArgs: per layer its operands, block range and parts;
+// the layers are independent once the data gradients are known, and alone
+// none of them has waves enough for the device).  Every unit writes a partial
+// [part][o][t][c]; k_wgrad_reduce sums the parts in a fixed order.
+struct WgradLayer {
+  const uint16_t *in;  // bf16 activations (layer 0: nullptr)
+  const float *G;      // output gradients, slot order (layer 7: dy)
+  float *part;
+  Dims od, id;
+  uint32_t n_parts, block0;  // first block of this layer
+};
+struct WgradArgs {
+  WgradLayer l[8];
+  const float *x32;  // input of layer 0
+};
 
-// The same weight gradient on MFMA (bf16 inputs, FP32 accumulation), for
-// channel counts that are multiples of 16: per tap t an implicit GEMM
-// dW_t[o][c] = sum_p G[p][o] X[src(p, t)][c] with M = output channels,
-// N = input channels and K = grid points, 32 points per
-// v_mfma_f32_16x16x32_bf16.  Each wave owns every (o, c) tile and a
-// strided share of the part's 32-point chunks; the output gradients G are
-// rounded to bf16 (the activations X are stored in bf16 already).  The four
-// waves are summed in LDS into the same per-part partials as k_conv_wgrad.
-template <int CIN, int COUT, int STRIDE, bool UP>
-__global__ void __launch_bounds__(kBlock)
-k_conv_wgrad_mfma(const uint16_t *__restrict__ in, const float *__restrict__ G,
-                  float *__restrict__ part, Dims od, Dims id, uint32_t n_parts) {
-  static_assert(CIN % 16 == 0 && COUT % 16 == 0, "channel counts must be multiples of 16");
-  constexpr int OT = COUT / 16, CT = CIN / 16, NW = kBlock / 64;
-  __shared__ float red[NW][OT * CT * 4][64];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int t = blockIdx.x;
-  const uint32_t pi = blockIdx.y;
-  const uint64_t P = (uint64_t)od.x * od.y * od.z;
-  const uint64_t p0 = P * pi / n_parts, p1 = P * (pi + 1) / n_parts;
-  const int kq = 8 * (lane >> 4), li = lane & 15;
-  v4f acc[OT][CT];
+// Layers 1-6 on MFMA (bf16 operands, FP32 accumulation), one unit per wave: 16
+// output channels (rows) x CTW tiles of 16 input channels (columns) for the
+// three taps of one x-row of the stencil, K = grid points, 32 per
+// v_mfma_f32_16x16x32_bf16.  The output gradients are rounded to bf16 and
+// loaded once for the three taps; with an up-sampled input the taps share
+// two inputs per point, lo = (x - 1) / 2 and lo + 1.  A lane holds 8
+// consecutive points, decoded once.  Bound by the latency of the gathered
+// 2-byte and 4-byte loads: 38 us for all eight layers on a 33^3 grid, against
+// 430 us in one launch per layer with one tap per workgroup, the loads of each
+// tap by themselves and a 64-bit index division per point.
+template <int CIN, int COUT, int STRIDE, bool UP, int CTW>
+__device__ __forceinline__ void wgrad_mfma(const WgradLayer &L, uint32_t unit) {
+  static_assert(CIN % (16 * CTW) == 0 && COUT % 16 == 0, "channel tiles");
+  static_assert(UP == (STRIDE == 1), "the stride-1 layers read an up-sampled input");
+  constexpr int OT = COUT / 16, CG = CIN / 16 / CTW;
+  constexpr int NX = UP ? 2 : 3;  // inputs per point
+  const int lane = threadIdx.x & 63, g = lane >> 4, li = lane & 15;
+  const int ot = unit % OT, cg = unit / OT % CG, zy = unit / (OT * CG) % 9;
+  const uint32_t pi = unit / (OT * CG * 9);
+  if (pi >= L.n_parts) return;
+  const int oy = zy % 3 - 1, oz = zy / 3 - 1;
+  const uint32_t P = L.od.x * L.od.y * L.od.z, chunks = (P + 31) / 32;
+  const uint32_t k0 = (uint64_t)chunks * pi / L.n_parts,
+                 k1 = (uint64_t)chunks * (pi + 1) / L.n_parts;
+  const int slot = slot_of(ot * 16 + li, COUT);
+  const uint16_t *in = L.in + cg * CTW * 16 + li;
+  v4f acc[3][CTW];
 #pragma unroll
-  for (int a = 0; a < OT; ++a)
+  for (int t = 0; t < 3; ++t)
 #pragma unroll
-    for (int b = 0; b < CT; ++b) acc[a][b] = v4f{0.f, 0.f, 0.f, 0.f};
-  for (uint64_t cb = p0 + 32 * (uint64_t)wave; cb < p1; cb += 32 * NW) {
-    // this lane's 8 points of the chunk: k = kq .. kq + 7
-    int64_t src[8];
-    uint64_t pt[8];
+    for (int b = 0; b < CTW; ++b) acc[t][b] = v4f{0.f, 0.f, 0.f, 0.f};
+  for (uint32_t k = k0; k < k1; ++k) {
+    const uint32_t p0 = k * 32 + 8 * g;
+    int x, y, z;
+    decode(p0 < P ? p0 : 0, L.od, x, y, z);
+    uint16_t h[NX][CTW][8];
+    float gv[8];
+    uint32_t row_on = 0, left = 0, right = 0, odd = 0;  // per point
 #pragma unroll
     for (int q = 0; q < 8; ++q) {
-      pt[q] = cb + kq + q;
-      src[q] = -1;
-      if (pt[q] < p1) {
-        int x, y, z;
-        decode(pt[q], od, x, y, z);
-        src[q] = tap_source<STRIDE, UP>(x, y, z, t, od, id);
+      const bool live = p0 + q < P;
+      gv[q] = L.G[(uint64_t)(live ? p0 + q : 0) * COUT + slot];
+      gv[q] = live ? gv[q] : 0.f;
+      const int ry = STRIDE * y + oy, rz = STRIDE * z + oz;
+      // the grid the taps are bounded by: the fine grid of an up-sampled input
+      const Dims bd = UP ? L.od : L.id;
+      const bool row = live && ry >= 0 && rz >= 0 && ry < (int)bd.y && rz < (int)bd.z;
+      row_on |= (uint32_t)row << q;
+      left |= (uint32_t)(STRIDE * x > 0) << q;
+      right |= (uint32_t)(STRIDE * x + 1 < (int)bd.x) << q;
+      odd |= (uint32_t)(x & 1) << q;
+      const uint64_t base = row ? lin(0, UP ? ry >> 1 : ry, UP ? rz >> 1 : rz, L.id) : 0;
+      const int lo = UP ? (x - 1) >> 1 : 2 * x - 1;
+#pragma unroll
+      for (int j = 0; j < NX; ++j) {
+        const int xs = min(max(lo + j, 0), (int)L.id.x - 1);  // outside: read, not used
+#pragma unroll
+        for (int b = 0; b < CTW; ++b) h[j][b][q] = in[(base + xs) * CIN + b * 16];
+      }
+      if (++x == (int)L.od.x) {
+        x = 0;
+        if (++y == (int)L.od.y) {
+          y = 0;
+          ++z;
+        }
       }
     }
-    v8bf bx[CT], ag[OT];
+    __builtin_amdgcn_sched_barrier(0);  // all loads of the chunk are in flight
+    uint32_t gw[4];
 #pragma unroll
-    for (int b = 0; b < CT; ++b) {
-      uint16_t h[8];
+    for (int q = 0; q < 4; ++q)
+      gw[q] = (uint32_t)f2bf(gv[2 * q]) | (uint32_t)f2bf(gv[2 * q + 1]) << 16;
+    const v8bf ag = __builtin_bit_cast(v8bf, make_uint4(gw[0], gw[1], gw[2], gw[3]));
 #pragma unroll
-      for (int q = 0; q < 8; ++q)
-        h[q] = src[q] >= 0 ? in[(uint64_t)src[q] * CIN + b * 16 + li] : (uint16_t)0;
-      const uint4 raw = make_uint4(h[0] | (uint32_t)h[1] << 16, h[2] | (uint32_t)h[3] << 16,
-                                   h[4] | (uint32_t)h[5] << 16, h[6] | (uint32_t)h[7] << 16);
-      bx[b] = __builtin_bit_cast(v8bf, raw);
+    for (int t = 0; t < 3; ++t) {
+      const uint32_t on = row_on & (t == 0 ? left : t == 2 ? right : ~0u);
+#pragma unroll
+      for (int b = 0; b < CTW; ++b) {
+        uint32_t xw[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          uint32_t v[2];
+#pragma unroll
+          for (int e = 0; e < 2; ++e) {
+            const int i = 2 * q + e;
+            // up-sampled middle tap: x / 2 is lo for odd x, lo + 1 for even x
+            const uint16_t raw = !UP      ? h[t][b][i]
+                                 : t == 0 ? h[0][b][i]
+                                 : t == 2 ? h[1][b][i]
+                                          : (odd >> i & 1 ? h[0][b][i] : h[1][b][i]);
+            v[e] = (on >> i & 1) ? raw : 0u;
+          }
+          xw[q] = v[0] | v[1] << 16;
+        }
+        acc[t][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+            ag, __builtin_bit_cast(v8bf, make_uint4(xw[0], xw[1], xw[2], xw[3])), acc[t][b], 0, 0,
+            0);
+      }
     }
-#pragma unroll
-    for (int a = 0; a < OT; ++a) {
-      uint16_t h[8];
-#pragma unroll
-      for (int q = 0; q < 8; ++q) h[q] = pt[q] < p1 ? f2bf(G[pt[q] * COUT + slot_of(a * 16 + li, COUT)]) : 0;
-      const uint4 raw = make_uint4(h[0] | (uint32_t)h[1] << 16, h[2] | (uint32_t)h[3] << 16,
-                                   h[4] | (uint32_t)h[5] << 16, h[6] | (uint32_t)h[7] << 16);
-      ag[a] = __builtin_bit_cast(v8bf, raw);
-    }
-#pragma unroll
-    for (int a = 0; a < OT; ++a)
-#pragma unroll
-      for (int b = 0; b < CT; ++b)
-        acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ag[a], bx[b], acc[a][b], 0, 0, 0);
   }
+  // D layout: register r of a lane holds (o, c) = (16 ot + 4 g + r, 16 b + li)
 #pragma unroll
-  for (int a = 0; a < OT; ++a)
+  for (int t = 0; t < 3; ++t)
 #pragma unroll
-    for (int b = 0; b < CT; ++b)
+    for (int b = 0; b < CTW; ++b)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) red[wave][(a * CT + b) * 4 + r][lane] = acc[a][b][r];
-  __syncthreads();
-  // D layout: register r of lane l holds (o, c) = (16 a + 4 (l / 16) + r, 16 b + l % 16)
-  for (int e = threadIdx.x; e < OT * CT * 4 * 64; e += kBlock) {
-    const int tr = e / 64, l = e % 64;
-    float v = 0.f;
-#pragma unroll
-    for (int w = 0; w < NW; ++w) v += red[w][tr][l];
-    const int tile = tr / 4, r = tr % 4, a = tile / CT, b = tile % CT;
-    const int o = a * 16 + 4 * (l >> 4) + r, c = b * 16 + (l & 15);
-    part[((uint64_t)pi * COUT + o) * 27 * CIN + (uint64_t)t * CIN + c] = v;
-  }
+      for (int r = 0; r < 4; ++r) {
+        const int o = ot * 16 + 4 * g + r, c = (cg * CTW + b) * 16 + li;
+        L.part[(((uint64_t)pi * COUT + o) * 27 + zy * 3 + t) * CIN + c] = acc[t][b][r];
+      }
 }
 
-// Weight gradient of the two 1-channel layers (stride 1, no up-sampling):
-// the input layer (1 -> 16, FP32 input in32) and the head (16 -> 1, bf16
-// input in, output gradient with one channel).  Per tap only 16 weights, so
-// every thread accumulates all 16 over its share of the part's points; the
-// sums go through wave shuffles and LDS into the same per-part partials.
+// The two 1-channel layers (stride 1, FP32 products): the input layer (1 ->
+// 16, input x32) and the head (16 -> 1, bf16 input, output gradient with one
+// channel).  Per tap only 16 weights, so every thread accumulates all 16 over
+// its share of the part's points; the sums go through wave shuffles and LDS.
 template <bool HEAD>
-__global__ void __launch_bounds__(kBlock)
-k_conv_wgrad_thin(const uint16_t *__restrict__ in, const float *__restrict__ in32,
-                  const float *__restrict__ G, float *__restrict__ part, Dims od,
-                  uint32_t n_parts) {
-  __shared__ float red[kBlock / 64][16];
-  const int t = blockIdx.x;
-  const uint32_t pi = blockIdx.y;
-  const uint64_t P = (uint64_t)od.x * od.y * od.z;
-  const uint64_t p0 = P * pi / n_parts, p1 = P * (pi + 1) / n_parts;
+__device__ __forceinline__ void wgrad_thin(const WgradLayer &L, const float *x32, uint32_t unit,
+                                           float (*red)[16]) {
+  const int t = unit % 27;
+  const uint32_t pi = unit / 27, P = L.od.x * L.od.y * L.od.z;
+  const uint32_t p0 = (uint64_t)P * pi / L.n_parts, p1 = (uint64_t)P * (pi + 1) / L.n_parts;
   float acc[16];
 #pragma unroll
   for (int k = 0; k < 16; ++k) acc[k] = 0.f;
-  for (uint64_t p = p0 + threadIdx.x; p < p1; p += kBlock) {
+  for (uint32_t p = p0 + threadIdx.x; p < p1; p += kBlock) {
     int x, y, z;
-    decode(p, od, x, y, z);
-    const int64_t src = tap_source<1, false>(x, y, z, t, od, od);
+    decode(p, L.od, x, y, z);
+    const int64_t src = tap_source<1, false>(x, y, z, t, L.od, L.od);
     if (src < 0) continue;
     if constexpr (HEAD) {  // dW[0][t][c] = sum_p dy[p] act[p + off_t][c]
-      const float g = G[p];
-      const uint16_t *a = in + (uint64_t)src * 16;
+      const float g = L.G[p];
+      const uint16_t *a = L.in + (uint64_t)src * 16;
 #pragma unroll
       for (int k = 0; k < 16; ++k) acc[k] += g * bf2f(a[k]);
     } else {  // dW[o][t][0] = sum_p G[p][o] x[p + off_t]
-      const float xv = in32[src];
-      const float *g = G + p * 16;
+      const float xv = x32[src];
+      const float *g = L.G + (uint64_t)p * 16;
 #pragma unroll
       for (int k = 0; k < 16; ++k) acc[k] += g[slot_of(k, 16)] * xv;
     }
@@ -573,20 +637,51 @@ k_conv_wgrad_thin(const uint16_t *__restrict__ in, const float *__restrict__ in3
 #pragma unroll
     for (int w = 0; w < kBlock / 64; ++w) v += red[w][k];
     // HEAD: cout 1, cin 16 (c = k); else cout 16 (o = k), cin 1
-    const uint64_t idx = HEAD ? ((uint64_t)pi * 27 + t) * 16 + k
-                              : ((uint64_t)pi * 16 + k) * 27 + t;
-    part[idx] = v;
+    L.part[HEAD ? ((uint64_t)pi * 27 + t) * 16 + k : ((uint64_t)pi * 16 + k) * 27 + t] = v;
   }
 }
 
-// grad[w] += sum over parts of part[part][w] (fixed order)
-__global__ void k_wgrad_reduce(const float *__restrict__ part, float *__restrict__ grad, uint32_t nw,
-                               uint32_t n_parts) {
-  const uint32_t w = blockIdx.x * kBlock + threadIdx.x;
-  if (w >= nw) return;
+// block ranges in the order of the layers below (longest units first)
+constexpr int kWgradOrder[8] = {6, 5, 1, 4, 2, 3, 7, 0};
+
+__global__ void __launch_bounds__(kBlock) k_wgrad(WgradArgs a) {
+  __shared__ float red[kBlock / 64][16];
+  const uint32_t b = blockIdx.x;
+  auto wave_unit = [&](int l) {
+    return (b - a.l[l].block0) * (kBlock / 64) + (threadIdx.x >> 6);
+  };
+  if (b < a.l[5].block0) return wgrad_mfma<32, 16, 1, true, 2>(a.l[6], wave_unit(6));
+  if (b < a.l[1].block0) return wgrad_mfma<64, 32, 1, true, 2>(a.l[5], wave_unit(5));
+  if (b < a.l[4].block0) return wgrad_mfma<16, 32, 2, false, 1>(a.l[1], wave_unit(1));
+  if (b < a.l[2].block0) return wgrad_mfma<64, 64, 1, true, 2>(a.l[4], wave_unit(4));
+  if (b < a.l[3].block0) return wgrad_mfma<32, 64, 2, false, 2>(a.l[2], wave_unit(2));
+  if (b < a.l[7].block0) return wgrad_mfma<64, 64, 2, false, 2>(a.l[3], wave_unit(3));
+  if (b < a.l[0].block0) return wgrad_thin<true>(a.l[7], nullptr, b - a.l[7].block0, red);
+  wgrad_thin<false>(a.l[0], a.x32, b - a.l[0].block0, red);
+}
+
+// grad[w] += sum over its layer's parts of part[part][w], in a fixed order:
+// four strided sums per weight, then their sum
+struct ReduceArgs {
+  const float *part[8];
+  uint32_t n_parts[8], w0[9];  // first weight of each layer
+};
+__global__ void __launch_bounds__(kBlock) k_wgrad_reduce(ReduceArgs a, float *__restrict__ grad) {
+  __shared__ float red[4][64];
+  const int j = threadIdx.x >> 6, i = threadIdx.x & 63;
+  const uint32_t w = blockIdx.x * 64 + i;
   float s = 0.f;
-  for (uint32_t k = 0; k < n_parts; ++k) s += part[(uint64_t)k * nw + w];
-  grad[w] += s;
+  if (w < a.w0[8]) {
+    int l = 0;
+    while (w >= a.w0[l + 1]) ++l;
+    const uint32_t nw = a.w0[l + 1] - a.w0[l];
+    const float *p = a.part[l] + (w - a.w0[l]);
+#pragma unroll 4
+    for (uint32_t k = j; k < a.n_parts[l]; k += 4) s += p[(uint64_t)k * nw];
+  }
+  red[j][i] = s;
+  __syncthreads();
+  if (j == 0 && w < a.w0[8]) grad[w] += ((red[0][i] + red[1][i]) + red[2][i]) + red[3][i];
 }
 
 // head backward: g[p][c] = (sum_t W[t][c] dy[p - off_t]) * (act[p][c] > 0),
@@ -601,7 +696,7 @@ k_head_backward(const float *__restrict__ dy, const float *__restrict__ W,
   const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   if (i >= P) return;
   int x, y, z;
-  decode32(i, d, x, y, z);
+  decode(i, d, x, y, z);
   float v[27];
   uint32_t mask = 0;
 #pragma unroll
@@ -660,10 +755,11 @@ __global__ void k_adam(float *__restrict__ w, float *__restrict__ m, float *__re
   w[i] -= lr * (mi / c1) / (sqrtf(vi / c2) + eps);
 }
 
-// layer weights [o][t][c] FP32 -> bf16 [o][KP] (k = t cin + c, zero padded)
-// and the FP32 value of each bf16 weight [o][t][c]; with wa (channel counts
-// that are multiples of 16) also the FP32 value in the order AdjTap reads it:
-// [t][c / 16][o / 16][lane 16 (o % 4) + c % 16][(o / 4) % 4]
+// layer weights [o][t][c] FP32 -> bf16 (k = t cin + c, zero padded to kp) in
+// the order k_conv_mfma reads them, [k / 32][o / 16][lane 16 (k / 8 % 4) + o %
+// 16][k % 8], and the FP32 value of each bf16 weight in the order AdjTap reads
+// it, wa[t][c / 16][o / 16][lane 16 (o % 4) + c % 16][(o / 4) % 4] (both where
+// the channel counts are multiples of 16, wa given) and as wr[o][t][c]
 __global__ void k_pack_weights(const float *__restrict__ w, uint16_t *__restrict__ wb,
                                float *__restrict__ wr, float *__restrict__ wa, int cin, int cout,
                                int kp) {
@@ -682,7 +778,7 @@ __global__ void k_pack_weights(const float *__restrict__ w, uint16_t *__restrict
          ((o >> 2) & 3)] = bf2f(h);
     }
   }
-  wb[i] = h;
+  if (wa) wb[((size_t)(k / 32 * (cout / 16) + o / 16) * 64 + (k >> 3 & 3) * 16 + o % 16) * 8 + k % 8] = h;
 }
 
 __global__ void k_scale_to_f32(const double *__restrict__ r, float *__restrict__ out, double s,
@@ -702,16 +798,27 @@ __global__ void k_axpy_f32(float *__restrict__ x, float a, const float *__restri
   if (i < n) x[i] += a * y[i];
 }
 
+constexpr uint64_t kSpreadWaves = 4096;  // four waves per SIMD
+
 inline unsigned blocks(uint64_t n) { return (unsigned)std::max<uint64_t>(1, (n + kBlock - 1) / kBlock); }
 inline Dims D3(const uint32_t *d) { return Dims{d[0], d[1], d[2]}; }
 
-template <int CIN, int COUT, int STRIDE, bool UP, bool SKIP>
+// Channel tiles per wave: one while the waves do not fill the device (each
+// then waits for its own loads only), all of them on larger grids, where the
+// gathered rows are then loaded once for all channels.  The whole network
+// against the form with all tiles in a wave and no loads ahead: 63 us / 146 on
+// 33^3 nodes, 145 / 241 on 65^3, 5.6 ms / 7.3 on 257^3.
+template <int CIN, int COUT, int STRIDE, bool UP>
 void mfma_launch(const uint16_t *in, const uint16_t *W, const uint16_t *skip, uint16_t *out,
                  const uint32_t *od, const uint32_t *id, hipStream_t s) {
-  const uint64_t P = (uint64_t)od[0] * od[1] * od[2];
-  const uint64_t waves = (P + 15) / 16;
-  hipLaunchKernelGGL((k_conv_mfma<CIN, COUT, STRIDE, UP, SKIP>), dim3(blocks(waves * 64)),
-                     dim3(kBlock), 0, s, in, W, skip, out, D3(od), D3(id));
+  constexpr int NT = COUT / 16;
+  const uint64_t tiles = ((uint64_t)od[0] * od[1] * od[2] + 15) / 16;
+  if (NT == 1 || tiles * NT <= kSpreadWaves)
+    hipLaunchKernelGGL((k_conv_mfma<CIN, COUT, STRIDE, UP, 1>), dim3(blocks(tiles * NT * 64)),
+                       dim3(kBlock), 0, s, in, W, skip, out, D3(od), D3(id));
+  else
+    hipLaunchKernelGGL((k_conv_mfma<CIN, COUT, STRIDE, UP, NT>), dim3(blocks(tiles * 64)),
+                       dim3(kBlock), 0, s, in, W, skip, out, D3(od), D3(id));
 }
 
 }  // namespace
@@ -721,13 +828,13 @@ void nn_conv_forward(int layer, const uint16_t *in, const float *in32, const uin
                      const uint32_t *od, const uint32_t *id, hipStream_t s) {
   const uint64_t P = (uint64_t)od[0] * od[1] * od[2];
   switch (layer) {
-    case 0: hipLaunchKernelGGL(k_conv_first, dim3(blocks(P)), dim3(kBlock), 0, s, in32, wr, out, D3(od)); break;
-    case 1: mfma_launch<16, 32, 2, false, false>(in, wb, nullptr, out, od, id, s); break;
-    case 2: mfma_launch<32, 64, 2, false, false>(in, wb, nullptr, out, od, id, s); break;
-    case 3: mfma_launch<64, 64, 2, false, false>(in, wb, nullptr, out, od, id, s); break;
-    case 4: mfma_launch<64, 64, 1, true, true>(in, wb, skip, out, od, id, s); break;
-    case 5: mfma_launch<64, 32, 1, true, true>(in, wb, skip, out, od, id, s); break;
-    case 6: mfma_launch<32, 16, 1, true, true>(in, wb, skip, out, od, id, s); break;
+    case 0: hipLaunchKernelGGL(k_conv_first, dim3((unsigned)((P + 63) / 64)), dim3(kBlock), 0, s, in32, wr, out, D3(od)); break;
+    case 1: mfma_launch<16, 32, 2, false>(in, wb, nullptr, out, od, id, s); break;
+    case 2: mfma_launch<32, 64, 2, false>(in, wb, nullptr, out, od, id, s); break;
+    case 3: mfma_launch<64, 64, 2, false>(in, wb, nullptr, out, od, id, s); break;
+    case 4: mfma_launch<64, 64, 1, true>(in, wb, skip, out, od, id, s); break;
+    case 5: mfma_launch<64, 32, 1, true>(in, wb, skip, out, od, id, s); break;
+    case 6: mfma_launch<32, 16, 1, true>(in, wb, skip, out, od, id, s); break;
     case 7: hipLaunchKernelGGL(k_conv_last, dim3(blocks(P)), dim3(kBlock), 0, s, in, wr, out32, D3(od)); break;
     default: throw Error{MFX_ERR_INVALID_ARG, "layer out of range"};
   }
@@ -769,54 +876,38 @@ void nn_conv_adjoint(int layer, const float *G, const float *wa, const float *ad
   MFX_HIP(hipGetLastError());
 }
 
-// the MFMA weight gradient for the layer shapes of the U-Net; false if the
-// shape has no MFMA instance (then the VALU kernel runs)
-template <int CI, int CO, int ST, bool UPF>
-bool wgrad_mfma_if(int stride, bool up, const uint16_t *in, const float *G, float *part,
-                   const uint32_t *od, const uint32_t *id, int cin, int cout, uint32_t n_parts,
-                   hipStream_t s) {
-  if (!(in && cin == CI && cout == CO && stride == ST && up == UPF)) return false;
-  hipLaunchKernelGGL((k_conv_wgrad_mfma<CI, CO, ST, UPF>), dim3(27, n_parts), dim3(kBlock), 0, s,
-                     in, G, part, D3(od), D3(id), n_parts);
-  return true;
-}
-bool wgrad_mfma(int stride, bool up, const uint16_t *in, const float *G, float *part,
-                const uint32_t *od, const uint32_t *id, int cin, int cout, uint32_t n_parts,
-                hipStream_t s) {
-  return wgrad_mfma_if<32, 16, 1, true>(stride, up, in, G, part, od, id, cin, cout, n_parts, s) ||
-         wgrad_mfma_if<64, 32, 1, true>(stride, up, in, G, part, od, id, cin, cout, n_parts, s) ||
-         wgrad_mfma_if<64, 64, 1, true>(stride, up, in, G, part, od, id, cin, cout, n_parts, s) ||
-         wgrad_mfma_if<64, 64, 2, false>(stride, up, in, G, part, od, id, cin, cout, n_parts, s) ||
-         wgrad_mfma_if<32, 64, 2, false>(stride, up, in, G, part, od, id, cin, cout, n_parts, s) ||
-         wgrad_mfma_if<16, 32, 2, false>(stride, up, in, G, part, od, id, cin, cout, n_parts, s);
+uint32_t nn_wgrad_parts(int layer, const uint32_t *od) {
+  const uint64_t P = (uint64_t)od[0] * od[1] * od[2];
+  // MFMA layers: units of at least four 32-point chunks; the 1-channel ones:
+  // blocks of at least four points per thread
+  const uint64_t n = (layer == 0 || layer == 7) ? P / (4 * kBlock) : (P + 31) / 32 / 4;
+  return (uint32_t)std::min<uint64_t>(std::max<uint64_t>(n, 1), 128);
 }
 
-void nn_conv_wgrad(int stride, bool up, const uint16_t *in, const float *in32, const float *G,
-                   float *part, float *grad, const uint32_t *od, const uint32_t *id, int cin,
-                   int cout, uint32_t n_parts, hipStream_t s) {
-  MFX_REQUIRE(cin <= 64 && cout <= 64 && cin * cout <= 16 * kBlock, "weight tile too large");
-  const dim3 grid(27, n_parts);
-  // the U-Net's layers with 16-multiple channel counts run on MFMA, the two
-  // 1-channel layers on the thin kernel
-  if (stride == 1 && !up && cin == 16 && cout == 1 && in) {
-    hipLaunchKernelGGL(k_conv_wgrad_thin<true>, grid, dim3(kBlock), 0, s, in, nullptr, G, part,
-                       D3(od), n_parts);
-  } else if (stride == 1 && !up && cin == 1 && cout == 16 && in32) {
-    hipLaunchKernelGGL(k_conv_wgrad_thin<false>, grid, dim3(kBlock), 0, s, nullptr, in32, G,
-                       part, D3(od), n_parts);
-  } else if (!wgrad_mfma(stride, up, in, G, part, od, id, cin, cout, n_parts, s)) {
-    if (stride == 2)
-      hipLaunchKernelGGL((k_conv_wgrad<2, false>), grid, dim3(kBlock), 0, s, in, in32, G, part,
-                         D3(od), D3(id), cin, cout, n_parts);
-    else if (up)
-      hipLaunchKernelGGL((k_conv_wgrad<1, true>), grid, dim3(kBlock), 0, s, in, in32, G, part,
-                         D3(od), D3(id), cin, cout, n_parts);
-    else
-      hipLaunchKernelGGL((k_conv_wgrad<1, false>), grid, dim3(kBlock), 0, s, in, in32, G, part,
-                         D3(od), D3(id), cin, cout, n_parts);
+void nn_wgrad(const NnWgrad (&l)[8], const float *x32, float *grad, hipStream_t s) {
+  // units (waves) per part of the MFMA layers: 9 x-rows of taps x output tiles
+  // x input tile groups, as the instances in k_wgrad split them
+  const uint32_t units[8] = {0, 9 * 2, 9 * 4, 9 * 4 * 2, 9 * 4 * 2, 9 * 2 * 2, 9, 0};
+  WgradArgs a;
+  ReduceArgs r;
+  a.x32 = x32;
+  uint32_t block = 0;
+  for (int k : kWgradOrder) {
+    const bool thin = k == 0 || k == 7;
+    a.l[k] = WgradLayer{l[k].in, l[k].G, l[k].part, D3(l[k].od), D3(l[k].id), l[k].n_parts, block};
+    block += thin ? 27 * l[k].n_parts
+                  : (units[k] * l[k].n_parts + kBlock / 64 - 1) / (kBlock / 64);
   }
-  const uint32_t nw = 27u * cin * cout;
-  hipLaunchKernelGGL(k_wgrad_reduce, dim3(blocks(nw)), dim3(kBlock), 0, s, part, grad, nw, n_parts);
+  uint32_t w = 0;
+  for (int k = 0; k < 8; ++k) {
+    r.part[k] = l[k].part;
+    r.n_parts[k] = l[k].n_parts;
+    r.w0[k] = w;
+    w += l[k].n_weights;
+  }
+  r.w0[8] = w;
+  hipLaunchKernelGGL(k_wgrad, dim3(block), dim3(kBlock), 0, s, a);
+  hipLaunchKernelGGL(k_wgrad_reduce, dim3((w + 63) / 64), dim3(kBlock), 0, s, r, grad);
   MFX_HIP(hipGetLastError());
 }
 
