@@ -19,6 +19,8 @@ void set_error(const std::string &msg) { g_last_error = msg; }
 using namespace mfx;
 
 static void finish_setup(mfx_op *op, int with_fp32, hipStream_t s) {
+  op->cmask.alloc((op->N + 31) / 32);
+  launch_bitmask(op->cons.ptr, op->n_cons, op->cmask.ptr, op->N, s);
   const uint64_t nq3 = (uint64_t)op->nq * op->nq * op->nq;
   if (op->geometry == MFX_GEOM_STORED) {
     op->G.alloc((uint64_t)op->E * 6 * nq3);
@@ -146,9 +148,7 @@ void cg_run(mfx_op &op, double *x, const double *b, const double *inv_diag, int 
 
   const auto t0 = std::chrono::steady_clock::now();
   // r = A x
-  launch_fill(w.r, 0.0, N, s);
-  op.apply64(x, w.r, s);
-  launch_copy_listed<double>(w.r, x, op.cons.ptr, op.n_cons, s);
+  op.vmult64(x, w.r, s);
   cg_init(w.st, b, w.r, inv_diag, N, w.part, abs_tol, rel_tol, max_steps, s);
   const int *done = &w.st->done;
   int h_local = 0;
@@ -363,6 +363,7 @@ mfx_status mfx_op_create(const mfx_op_desc *d, mfx_op **out) {
     op->cellX.upload(d->cell_vertices, (uint64_t)d->n_cells * 24);
     op->cons.upload(d->constrained, d->n_constrained);
     finish_setup(op.get(), d->with_fp32, nullptr);
+    op->cons_in_map = any_masked(op->map.ptr, nmap, op->cmask.ptr, nullptr);
     *out = op.release();
   });
 }
@@ -430,10 +431,7 @@ mfx_status mfx_op_vmult(mfx_op *op, double *dst, const double *src, void *stream
   return guard([&] {
     MFX_REQUIRE(op && dst && src, "null pointer argument");
     MFX_REQUIRE(dst != src, "vmult: src and dst must not alias");
-    hipStream_t s = as_stream(stream);
-    launch_fill(dst, 0.0, op->N, s);
-    op->apply64(src, dst, s);
-    launch_copy_listed<double>(dst, src, op->cons.ptr, op->n_cons, s);
+    op->vmult64(src, dst, as_stream(stream));
   });
 }
 
@@ -450,10 +448,7 @@ mfx_status mfx_op_vmult_f32(mfx_op *op, float *dst, const float *src, void *stre
     MFX_REQUIRE(op && dst && src, "null pointer argument");
     MFX_REQUIRE(dst != src, "vmult: src and dst must not alias");
     MFX_REQUIRE(op->D32.ptr, "operator created without with_fp32");
-    hipStream_t s = as_stream(stream);
-    launch_fill_f32(dst, 0.0f, op->N, s);
-    op->apply32(src, dst, s);
-    launch_copy_listed<float>(dst, src, op->cons.ptr, op->n_cons, s);
+    op->vmult32(src, dst, as_stream(stream));
   });
 }
 

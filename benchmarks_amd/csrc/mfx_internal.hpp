@@ -102,6 +102,15 @@ void launch_fill_f32(float *x, float v, uint64_t n, hipStream_t s);
 template <typename T>
 void launch_copy_listed(T *dst, const T *src, const uint32_t *list, uint64_t n,
                         hipStream_t s);
+// dst = src on the listed rows, 0 elsewhere; mask: the list as a bitmask
+template <typename T>
+void launch_start(T *dst, const T *src, const uint32_t *mask, const uint32_t *list,
+                  uint64_t n_list, uint64_t n, hipStream_t s);
+// bitmask of n rows (ceil(n / 32) words) with the listed rows set
+void launch_bitmask(const uint32_t *list, uint64_t n_list, uint32_t *mask, uint64_t n,
+                    hipStream_t s);
+// whether a valid map entry is a row of the bitmask (synchronizes the stream)
+bool any_masked(const uint32_t *map, uint64_t n, const uint32_t *mask, hipStream_t s);
 void launch_set_listed(double *dst, double v, const uint32_t *list, uint64_t n,
                        hipStream_t s);
 void launch_gather(const uint32_t *map, uint64_t n, const double *src, double *evec,

@@ -53,14 +53,10 @@ double dot(const double *x, const double *y, uint64_t n, DBuf<double> &part, hip
 }  // namespace
 
 void vmult64(mfx_op &op, double *dst, const double *src, hipStream_t s) {
-  launch_fill(dst, 0.0, op.N, s);
-  op.apply64(src, dst, s);
-  launch_copy_listed<double>(dst, src, op.cons.ptr, op.n_cons, s);
+  op.vmult64(src, dst, s);
 }
 void vmult32(mfx_op &op, float *dst, const float *src, hipStream_t s) {
-  launch_fill_f32(dst, 0.0f, op.N, s);
-  op.apply32(src, dst, s);
-  launch_copy_listed<float>(dst, src, op.cons.ptr, op.n_cons, s);
+  op.vmult32(src, dst, s);
 }
 
 // Chebyshev iteration for A x = b with the Jacobi preconditioner on the

@@ -102,6 +102,10 @@ struct mfx_op {
   uint64_t N = 0;
   uint64_t n_cons = 0;
   DBuf<uint32_t> map, cons;
+  DBuf<uint32_t> cmask;  // bit i: DoF i is constrained
+  // a caller's map gathers constrained DoFs: their rows then receive the
+  // cells' contributions, which vmult overwrites afterwards
+  bool cons_in_map = false;
   DBuf<double> G, B, D, xq, wq, support, cellX;
   DBuf<float> G32, B32, D32, xq32, wq32;
   // Gauss quadrature: the even-odd tables of B, B^T, D and D^T (eo_tab
@@ -189,6 +193,31 @@ struct mfx_op {
     else
       launch_apply<float>(p, nq, colloc, B32.ptr, D32.ptr, G32.ptr, src, dst, map.ptr, E, s,
                           nullptr, nullptr, row_cells());
+  }
+  // dst = A src with identity on the constrained rows
+  void vmult64(const double *src, double *dst, hipStream_t s) const {
+    if (patch && det) {
+      launch_patch<double>(patch_op64(), src, dst, s, nullptr, nullptr, true);
+    } else if (cons_in_map) {
+      launch_fill(dst, 0.0, N, s);
+      apply64(src, dst, s);
+      launch_copy_listed<double>(dst, src, cons.ptr, n_cons, s);
+    } else {
+      launch_start<double>(dst, src, cmask.ptr, cons.ptr, n_cons, N, s);
+      apply64(src, dst, s);
+    }
+  }
+  void vmult32(const float *src, float *dst, hipStream_t s) const {
+    if (patch && det) {
+      launch_patch<float>(patch_op32(), src, dst, s, nullptr, nullptr, true);
+    } else if (cons_in_map) {
+      launch_fill_f32(dst, 0.0f, N, s);
+      apply32(src, dst, s);
+      launch_copy_listed<float>(dst, src, cons.ptr, n_cons, s);
+    } else {
+      launch_start<float>(dst, src, cmask.ptr, cons.ptr, n_cons, N, s);
+      apply32(src, dst, s);
+    }
   }
 };
 

@@ -700,15 +700,17 @@ __global__ void k_patch_map(PatchLayout lay, int p, int bx, int by, int bz, uint
 // (pbuf[patch][local], from k_patch in deterministic mode) in ascending patch
 // order -- up to two patches per direction, the lower one first when the
 // node lies on their shared face -- to dst.  Constrained nodes (invalid in
-// the patch map) are left alone.  Workgroups cover x-runs of one node row
+// the patch map) are left alone.  ASSIGN: dst is set instead (constrained
+// nodes to src), which spares the vmult its start pass and the read of dst.
+// Workgroups cover x-runs of one node row
 // (y, z) at a time, so the only divisions are by the compile-time patch
 // spans and one per row.
 constexpr int kGatherX = 128;  // nodes of one row per workgroup
 
-template <typename T, int P, int BX, int BY, int BZ>
+template <typename T, int P, int BX, int BY, int BZ, bool ASSIGN>
 __global__ void __launch_bounds__(kGatherX)
 k_patch_gather(PatchLayout lay, const uint32_t *__restrict__ pmap, const T *__restrict__ pbuf,
-               T *__restrict__ dst, const int *__restrict__ skip) {
+               const T *__restrict__ src, T *__restrict__ dst, const int *__restrict__ skip) {
   if (skip && *skip) return;  // converged CG: the patch kernel stored nothing
   constexpr int SX = BX * P, SY = BY * P, SZ = BZ * P;
   constexpr int PX = SX + 1, PY = SY + 1, PZ = SZ + 1;
@@ -727,7 +729,11 @@ k_patch_gather(PatchLayout lay, const uint32_t *__restrict__ pmap, const T *__re
     // the lower patch along an axis holds the node as its last one
     const int x0 = (qx > 0 && lx == 0) ? 0 : 1, y0 = (qy > 0 && ly == 0) ? 0 : 1,
               z0 = (qz > 0 && lz == 0) ? 0 : 1;
-    if (pmap[at] == kInvalid) continue;  // constrained
+    const size_t node = (size_t)row * Nx + gx;
+    if (pmap[at] == kInvalid) {  // constrained
+      if (ASSIGN) dst[node] = src[node];
+      continue;
+    }
     // offsets to the same node in the lower patch along x, y, z
     const long dx = -(long)P3 + SX;
     const long dy = -(long)lay.np[0] * P3 + (long)SY * PX;
@@ -737,7 +743,7 @@ k_patch_gather(PatchLayout lay, const uint32_t *__restrict__ pmap, const T *__re
       for (int iy = y0; iy < 2; ++iy)
         for (int ix = x0; ix < 2; ++ix)
           sum += pbuf[(long)at + (iz ? 0 : dz) + (iy ? 0 : dy) + (ix ? 0 : dx)];
-    dst[(size_t)row * Nx + gx] += sum;
+    dst[node] = ASSIGN ? sum : dst[node] + sum;
   }
 }
 
@@ -794,7 +800,8 @@ void launch_patch_v(const PatchOp<T> &o, const T *src, T *dst, hipStream_t s, do
 
 template <typename T, class C>
 void launch_patch_t(const PatchOp<T> &o, const T *src, T *dst, hipStream_t s, double *partials,
-                    const int *skip) {
+                    const int *skip, bool assign) {
+  MFX_REQUIRE(!assign || (o.pbuf && !skip), "assigning apply: deterministic scatter only");
   // the kernel indexes the patch map with its compile-time patch size: the
   // map must have been built for exactly this shape
   MFX_REQUIRE(o.shape.bx == C::BX && o.shape.by == C::BY && o.shape.bz == C::BZ,
@@ -813,8 +820,12 @@ void launch_patch_t(const PatchOp<T> &o, const T *src, T *dst, hipStream_t s, do
     const uint32_t nx = o.lay.n[0] * C::P + 1;
     const uint64_t rows = ((uint64_t)o.lay.n[1] * C::P + 1) * ((uint64_t)o.lay.n[2] * C::P + 1);
     const dim3 grid((nx + kGatherX - 1) / kGatherX, (unsigned)std::min<uint64_t>(rows, 65535));
-    hipLaunchKernelGGL((k_patch_gather<T, C::P, C::BX, C::BY, C::BZ>), grid, dim3(kGatherX), 0, s,
-                       o.lay, o.pmap, o.pbuf, dst, skip);
+    if (assign)
+      hipLaunchKernelGGL((k_patch_gather<T, C::P, C::BX, C::BY, C::BZ, true>), grid,
+                         dim3(kGatherX), 0, s, o.lay, o.pmap, o.pbuf, src, dst, skip);
+    else
+      hipLaunchKernelGGL((k_patch_gather<T, C::P, C::BX, C::BY, C::BZ, false>), grid,
+                         dim3(kGatherX), 0, s, o.lay, o.pmap, o.pbuf, src, dst, skip);
     MFX_HIP(hipGetLastError());
   }
 }
@@ -853,13 +864,14 @@ template PatchGrid patch_grid<float>(int, const PatchLayout &, bool);
 
 template <typename T>
 void launch_patch(const PatchOp<T> &o, const T *src, T *dst, hipStream_t s, double *partials,
-                  const int *skip) {
-  with_cfg(o.p, [&](auto c) { launch_patch_t<T, decltype(c)>(o, src, dst, s, partials, skip); });
+                  const int *skip, bool assign) {
+  with_cfg(o.p,
+           [&](auto c) { launch_patch_t<T, decltype(c)>(o, src, dst, s, partials, skip, assign); });
 }
 template void launch_patch<double>(const PatchOp<double> &, const double *, double *, hipStream_t,
-                                   double *, const int *);
+                                   double *, const int *, bool);
 template void launch_patch<float>(const PatchOp<float> &, const float *, float *, hipStream_t,
-                                  double *, const int *);
+                                  double *, const int *, bool);
 
 uint32_t patch_batch_grid(int p, uint32_t n_patches, bool dot) {
   return with_cfg(p, [&](auto c) {

@@ -77,9 +77,11 @@ uint32_t patch_count(const PatchLayout &lay);
 // grids of the kernels with the metric from the vertices or (stored) from G
 template <typename T>
 PatchGrid patch_grid(int p, const PatchLayout &lay, bool stored);
+// dst += A src over the free rows.  assign (deterministic scatter only): dst =
+// A src, the constrained rows taking src, without a start value.
 template <typename T>
 void launch_patch(const PatchOp<T> &o, const T *src, T *dst, hipStream_t s,
-                  double *partials = nullptr, const int *skip = nullptr);
+                  double *partials = nullptr, const int *skip = nullptr, bool assign = false);
 void launch_patch_map(const PatchLayout &lay, int p, PatchShape sh, uint32_t *pmap, hipStream_t s);
 // The stored metric terms G [cell][6][nq^3] permuted into the patch order the
 // kernel with stored geometry reads (patch_geometry_size elements).
