@@ -19,7 +19,7 @@ void set_error(const std::string &msg) { g_last_error = msg; }
 using namespace mfx;
 
 static void finish_setup(mfx_op *op, int with_fp32, hipStream_t s) {
-  op->cmask.alloc((op->N + 31) / 32);
+  op->cmask.alloc((op->N + 31) / 32 + 1);  // the last word: scratch of any_masked
   launch_bitmask(op->cons.ptr, op->n_cons, op->cmask.ptr, op->N, s);
   const uint64_t nq3 = (uint64_t)op->nq * op->nq * op->nq;
   if (op->geometry == MFX_GEOM_STORED) {
@@ -363,7 +363,8 @@ mfx_status mfx_op_create(const mfx_op_desc *d, mfx_op **out) {
     op->cellX.upload(d->cell_vertices, (uint64_t)d->n_cells * 24);
     op->cons.upload(d->constrained, d->n_constrained);
     finish_setup(op.get(), d->with_fp32, nullptr);
-    op->cons_in_map = any_masked(op->map.ptr, nmap, op->cmask.ptr, nullptr);
+    op->cons_in_map = any_masked(op->map.ptr, nmap, op->cmask.ptr,
+                                 op->cmask.ptr + op->cmask.n - 1, nullptr);
     *out = op.release();
   });
 }

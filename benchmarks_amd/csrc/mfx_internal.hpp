@@ -109,8 +109,10 @@ void launch_start(T *dst, const T *src, const uint32_t *mask, const uint32_t *li
 // bitmask of n rows (ceil(n / 32) words) with the listed rows set
 void launch_bitmask(const uint32_t *list, uint64_t n_list, uint32_t *mask, uint64_t n,
                     hipStream_t s);
-// whether a valid map entry is a row of the bitmask (synchronizes the stream)
-bool any_masked(const uint32_t *map, uint64_t n, const uint32_t *mask, hipStream_t s);
+// whether a valid map entry is a row of the bitmask; found: one device word of
+// scratch (synchronizes the stream)
+bool any_masked(const uint32_t *map, uint64_t n, const uint32_t *mask, uint32_t *found,
+                hipStream_t s);
 void launch_set_listed(double *dst, double v, const uint32_t *list, uint64_t n,
                        hipStream_t s);
 void launch_gather(const uint32_t *map, uint64_t n, const double *src, double *evec,

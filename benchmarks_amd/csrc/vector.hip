@@ -424,17 +424,14 @@ void launch_bitmask(const uint32_t *list, uint64_t n_list, uint32_t *mask, uint6
     hipLaunchKernelGGL(k_mark_bits, dim3(vec_grid(n_list)), dim3(kBlock), 0, s, list, n_list, mask);
   MFX_HIP(hipGetLastError());
 }
-bool any_masked(const uint32_t *map, uint64_t n, const uint32_t *mask, hipStream_t s) {
+bool any_masked(const uint32_t *map, uint64_t n, const uint32_t *mask, uint32_t *found,
+                hipStream_t s) {
   if (!n) return false;
-  uint32_t *found = nullptr, h = 0;
-  MFX_HIP(hipMalloc(reinterpret_cast<void **>(&found), sizeof(uint32_t)));
+  uint32_t h = 0;
   hipLaunchKernelGGL(k_zero_words, dim3(1), dim3(kBlock), 0, s, found, (uint64_t)1);
   hipLaunchKernelGGL(k_any_masked, dim3(vec_grid(n)), dim3(kBlock), 0, s, map, n, mask, found);
-  const hipError_t e1 = hipMemcpyAsync(&h, found, sizeof(uint32_t), hipMemcpyDeviceToHost, s);
-  const hipError_t e2 = hipStreamSynchronize(s);
-  (void)hipFree(found);
-  MFX_HIP(e1);
-  MFX_HIP(e2);
+  MFX_HIP(hipMemcpyAsync(&h, found, sizeof(uint32_t), hipMemcpyDeviceToHost, s));
+  MFX_HIP(hipStreamSynchronize(s));
   return h != 0;
 }
 void launch_set_listed(double *dst, double v, const uint32_t *list, uint64_t n, hipStream_t s) {
