@@ -126,8 +126,19 @@ static void lexicographic_G(const mfx_op *op, GeometryView &v, hipStream_t s) {
 
 namespace mfx {
 
+// Whether a CG step runs in three launches (cg_direction_small): every
+// workgroup of the vector passes then sums all partials, which pays while
+// the workgroups and the partials are few (the sums cost a workgroup about a
+// microsecond, the three launches they replace 8 us; at 512 workgroups and
+// 2048 partials their reads are 8 MB from the L2s).
+static bool cg_small(const mfx_op &op) {
+  const uint32_t nb_vec = cg_vec_blocks(op.N);
+  return !op.cons_in_map && nb_vec <= 512 && op.apply_blocks() + nb_vec <= 2048;
+}
+
 size_t cg_partial_count(const mfx_op &op) {
   const uint32_t nb_apply = op.apply_blocks();
+  if (cg_small(op)) return (size_t)nb_apply + 3 * (size_t)cg_vec_blocks(op.N);
   const uint32_t nb_cons = cg_cons_blocks(op.n_cons);
   const uint32_t nb_vec = cg_vec_blocks(op.N);
   const size_t na = (size_t)nb_apply + nb_cons;
@@ -143,19 +154,31 @@ void cg_run(mfx_op &op, double *x, const double *b, const double *inv_diag, int 
   const uint32_t nb_apply = op.apply_blocks();
   const uint32_t nb_cons = cg_cons_blocks(op.n_cons);
   const uint32_t nb_vec = cg_vec_blocks(N);
-  CgState init{};
-  MFX_HIP(hipMemcpyAsync(w.st, &init, sizeof(CgState), hipMemcpyHostToDevice, s));
+  // small: the alternating states st[0] (written by the direction pass) and
+  // st[1] (by the update pass), partials [apply][constrained rows][r.r, r.Pr]
+  const bool small = cg_small(op);
+  CgState *sb = w.st, *sa = small ? w.st + 1 : w.st;
+  double *part_r = small ? w.part + nb_apply + nb_vec : w.part;
+  CgState init[2]{};
+  MFX_HIP(hipMemcpyAsync(w.st, init, sizeof(init), hipMemcpyHostToDevice, s));
 
   const auto t0 = std::chrono::steady_clock::now();
   // r = A x
   op.vmult64(x, w.r, s);
-  cg_init(w.st, b, w.r, inv_diag, N, w.part, abs_tol, rel_tol, max_steps, s);
+  cg_init(w.st, b, w.r, inv_diag, N, part_r, abs_tol, rel_tol, max_steps, s);
   const int *done = &w.st->done;
   int h_local = 0;
   int *h_done = w.h_done ? w.h_done : &h_local;
   int batch = 4;
   for (int it = 0;;) {
-    for (int k = 0; k < batch; ++k, ++it) {
+    for (int k = 0; small && k < batch; ++k, ++it) {
+      cg_direction_small(sa, sb, part_r, it == 0, w.r, inv_diag, op.cmask.ptr, w.p, w.ap, x,
+                         w.part + nb_apply, N, s);
+      op.apply64(w.p, w.ap, s, w.part, done);
+      cg_update_small(sb, sa, w.part, nb_apply + nb_vec, w.r, w.ap, inv_diag, N, part_r, s);
+    }
+    if (small) cg_test(sa, sb, part_r, N, s);
+    for (int k = 0; !small && k < batch; ++k, ++it) {
       cg_direction(w.st, w.r, inv_diag, w.p, w.ap, x, N, s);
       op.apply64(w.p, w.ap, s, w.part, done);
       cg_constrained(w.st, op.cons.ptr, op.n_cons, w.p, w.ap, w.part + nb_apply, s);
@@ -170,7 +193,7 @@ void cg_run(mfx_op &op, double *x, const double *b, const double *inv_diag, int 
     if (it > max_steps + 8) break;  // device enforces max_steps; this bounds the host loop
     batch = std::min(batch * 2, 64);
   }
-  cg_finish(w.st, x, w.p, N, s);
+  cg_finish(sb, sa, x, w.p, N, s);
   CgState fin{};
   MFX_HIP(hipMemcpyAsync(&fin, w.st, sizeof(CgState), hipMemcpyDeviceToHost, s));
   MFX_HIP(hipStreamSynchronize(s));
@@ -506,7 +529,7 @@ mfx_status mfx_cg_solve(mfx_op *op, double *x, const double *b, const double *in
       op->ap.alloc(N);
     }
     if (op->part.n < npart) op->part.alloc(npart);
-    if (!op->st.ptr) op->st.alloc(1);
+    if (!op->st.ptr) op->st.alloc(2);
     if (!op->h_done) MFX_HIP(hipHostMalloc(reinterpret_cast<void **>(&op->h_done), sizeof(int)));
     const CgWork w{op->r.ptr, op->pdir.ptr, op->ap.ptr, op->part.ptr, op->st.ptr, op->h_done};
     cg_run(*op, x, b, inv_diag, max_steps, abs_tol, rel_tol, w, res, as_stream(stream));

@@ -51,7 +51,21 @@ uint32_t cg_alpha_extra(uint32_t n);
 void cg_update(const CgState *st, double *r, const double *ap, const double *invd, uint64_t n,
                double *part, hipStream_t s);
 void cg_check(CgState *st, const double *part, uint32_t nb, hipStream_t s);
-// the last step's x += alpha p (nothing if no step was taken)
-void cg_finish(const CgState *st, double *x, const double *p, uint64_t n, hipStream_t s);
+// the last step's x += alpha p (nothing if no step was taken), alpha from sa
+void cg_finish(const CgState *st, const CgState *sa, double *x, const double *p, uint64_t n,
+               hipStream_t s);
+// A step in three launches (direction, apply, update) for systems with few
+// partials: the direction pass tests the previous step's convergence (not on
+// the first) and starts Ap on the constrained rows (bitmask `mask`, partials
+// of p^2 in part_c), the update pass forms alpha from the n_pap partials.
+// sa / sb: the alternating states (vector.hip); part: 2 cg_vec_blocks(n)
+// partials of the update pass.  cg_test: the convergence test alone.
+void cg_direction_small(const CgState *sa, CgState *sb, const double *part, bool first,
+                        const double *r, const double *invd, const uint32_t *mask, double *p,
+                        double *ap, double *x, double *part_c, uint64_t n, hipStream_t s);
+void cg_update_small(const CgState *sb, CgState *sa, const double *pap, uint32_t n_pap, double *r,
+                     const double *ap, const double *invd, uint64_t n, double *part,
+                     hipStream_t s);
+void cg_test(const CgState *sa, CgState *sb, const double *part, uint64_t n, hipStream_t s);
 
 }  // namespace mfx

@@ -22,7 +22,7 @@ namespace {
 
 constexpr uint64_t kNoAllocMaxDofs = 1ull << 21;        // 2,097,152 DoFs
 constexpr uint64_t kNoAllocMaxPartials = 1ull << 17;    // partial sums of one reduction
-constexpr uint64_t kStateDoubles = (sizeof(CgState) + 7) / 8;
+constexpr uint64_t kStateDoubles = (2 * sizeof(CgState) + 7) / 8;
 constexpr uint64_t kScratchDoubles = 3 * kNoAllocMaxDofs + kNoAllocMaxPartials + kStateDoubles;
 
 static __device__ __align__(256) double scratch[kScratchDoubles];

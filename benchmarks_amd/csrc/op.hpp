@@ -126,7 +126,7 @@ struct mfx_op {
   DBuf<float> pbuf32;
   // CG scratch, allocated on first use
   DBuf<double> r, pdir, ap, part;
-  DBuf<CgState> st;
+  DBuf<CgState> st;  // two (cg_run)
   int *h_done = nullptr;  // pinned
   ~mfx_op() {
     if (h_done) (void)hipHostFree(h_done);
@@ -224,7 +224,7 @@ struct mfx_op {
 namespace mfx {
 
 // Work buffers of one CG solve: three N-vectors, cg_partial_count(op)
-// partial sums, the device state, and a host word for the `done` flag
+// partial sums, two device states, and a host word for the `done` flag
 // (pinned, or nullptr to read it into pageable host memory).
 struct CgWork {
   double *r, *p, *ap, *part;
