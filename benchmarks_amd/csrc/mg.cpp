@@ -67,24 +67,36 @@ void vmult32(mfx_op &op, float *dst, const float *src, hipStream_t s) {
 // `degree` updates in all, so the error is multiplied by the scaled
 // Chebyshev polynomial T_degree((theta - lambda) / delta) / T_degree(theta / delta).
 // A is applied degree - 1 times from a zero x, degree times otherwise.
-// t and d are scratch vectors of the operator's size.
+// t and d are scratch vectors of the operator's size.  A step reads t = A x and
+// writes the start value of the next A x in its place (identity rows and
+// zeros), so every apply but the first adds to t without a start pass.
+bool cheb_starts(const mfx_op &op) { return !op.cons_in_map; }
+
 void chebyshev(mfx_op &op, float *x, const float *b, const float *dinv, float *t, float *d,
-               int degree, double lmin, double lmax, bool zero_initial, hipStream_t s) {
+               int degree, double lmin, double lmax, bool zero_initial, hipStream_t s, bool started,
+               bool leave_start) {
   const double theta = 0.5 * (lmax + lmin), delta = 0.5 * (lmax - lmin);
   const uint64_t N = op.N;
-  if (zero_initial) {
-    launch_cheb_step(x, d, b, nullptr, dinv, 0.0f, (float)(1.0 / theta), true, N, s);
-  } else {
-    vmult32(op, t, x, s);
-    launch_cheb_step(x, d, b, t, dinv, 0.0f, (float)(1.0 / theta), false, N, s);
-  }
+  const bool starts = cheb_starts(op);
+  MFX_REQUIRE(starts || (!started && !leave_start), "Chebyshev: operator needs its own start");
   double rho_old = delta / theta;
-  for (int k = 1; k < degree; ++k) {
-    vmult32(op, t, x, s);
-    const double rho = 1.0 / (2.0 * theta / delta - rho_old);
-    launch_cheb_step(x, d, b, t, dinv, (float)(rho * rho_old), (float)(2.0 * rho / delta), false,
-                     N, s);
-    rho_old = rho;
+  for (int k = 0; k < degree; ++k) {
+    const bool apply = k > 0 || !zero_initial;
+    if (apply) {
+      if (starts && (k > 0 || started))
+        op.apply32(x, t, s);
+      else
+        op.vmult32(x, t, s);
+    }
+    double c1 = 0.0, c2 = 1.0 / theta;
+    if (k > 0) {
+      const double rho = 1.0 / (2.0 * theta / delta - rho_old);
+      c1 = rho * rho_old;
+      c2 = 2.0 * rho / delta;
+      rho_old = rho;
+    }
+    launch_cheb_step(x, d, b, t, dinv, (float)c1, (float)c2, apply, k == 0 && zero_initial,
+                     starts && (k + 1 < degree || leave_start) ? op.cmask.ptr : nullptr, N, s);
   }
 }
 
@@ -244,38 +256,41 @@ struct mfx_mg {
   // outer CG scratch (FP64)
   DBuf<double> r, z, p, ap, part;
 
-  void smooth(Level &L, bool zero_initial, hipStream_t s) {
+  // first: pre-smoothing from zero, which leaves t as the start value of the
+  // residual's A x; otherwise post-smoothing, t started by the prolongation
+  void smooth(Level &L, bool first, hipStream_t s) {
     chebyshev(L.sm(), L.x.ptr, L.b.ptr, L.dinv.ptr, L.t.ptr, L.d.ptr, degree, L.lmin, L.lmax,
-              zero_initial, s);
+              first, s, !first, first);
   }
 
-  // x_l = V-cycle(b_l), zero initial guess
+  // x_l = V-cycle(b_l), zero initial guess.  Between the applies a level runs
+  // the Chebyshev steps and six transfer passes only: the residual b - A x is
+  // formed by the first restriction pass, the coarse constrained rows are
+  // zeroed by the last one, and the last prolongation pass adds to x and
+  // starts the next A x.
   void vcycle(size_t l, hipStream_t s) {
     Level &L = lv[l];
-    if (l + 1 == lv.size()) {
-      launch_fill_f32(L.x.ptr, 0.0f, L.op->N, s);
+    if (l + 1 == lv.size()) {  // (the constrained rows of x are zero from the start)
       launch_dense_solve(Ainv.ptr, free_idx.ptr, n_free, L.b.ptr, L.x.ptr, s);
       return;
     }
     Level &Cl = lv[l + 1];
     smooth(L, true, s);
-    vmult32(L.sm(), L.t.ptr, L.x.ptr, s);
-    launch_residual_f32(L.t.ptr, L.b.ptr, L.t.ptr, L.op->N, s);
-    restrict_<float>(L.to_coarse.R32, L.dims, Cl.dims, L.t.ptr, L.d.ptr, L.t.ptr, Cl.b.ptr, s);
-    launch_set_listed_f32(Cl.b.ptr, 0.0f, Cl.op->cons.ptr, Cl.op->n_cons, s);
+    L.sm().apply32(L.x.ptr, L.t.ptr, s);
+    restrict_<float>(L.to_coarse.R32, L.dims, Cl.dims, L.t.ptr, L.d.ptr, L.t.ptr, Cl.b.ptr, s,
+                     L.b.ptr, Cl.op->cmask.ptr);
     vcycle(l + 1, s);
-    prolongate<float>(L.to_coarse.P32, L.dims, Cl.dims, Cl.x.ptr, L.t.ptr, L.d.ptr, L.x.ptr, true, s);
+    prolongate<float>(L.to_coarse.P32, L.dims, Cl.dims, Cl.x.ptr, L.t.ptr, L.d.ptr, L.x.ptr, true, s,
+                      L.t.ptr, L.op->cmask.ptr);
     smooth(L, false, s);
   }
 
   // z = M r in FP64: constrained rows pass through, the rest is one FP32 V-cycle
   void precondition(double *z64, const double *r64, hipStream_t s) {
     Level &L = lv[0];
-    launch_to_float(r64, L.b.ptr, L.op->N, s);
-    launch_set_listed_f32(L.b.ptr, 0.0f, L.op->cons.ptr, L.op->n_cons, s);
+    launch_to_float_free(r64, L.b.ptr, L.op->cmask.ptr, L.op->N, s);
     vcycle(0, s);
-    launch_to_double(L.x.ptr, z64, L.op->N, s);
-    launch_copy_listed<double>(z64, r64, L.op->cons.ptr, L.op->n_cons, s);
+    launch_to_double_free(L.x.ptr, r64, z64, L.op->cmask.ptr, L.op->N, s);
   }
 };
 
@@ -406,6 +421,7 @@ mfx_status mfx_mg_create(const mfx_mg_desc *d, mfx_mg **out) {
       L.b.alloc(N);
       L.t.alloc(N);
       L.d.alloc(N);
+      launch_fill_f32(L.x.ptr, 0.0f, N, s);
       if (&L != &mg->lv.back()) {
         L.lmax = safety * estimate_lambda_max(L.sm(), inv.ptr, eig_its, s);
         L.lmin = L.lmax / range;
@@ -553,10 +569,12 @@ mfx_status mfx_chebyshev_f32(mfx_op *op, const float *inv_diag, float *x, const 
     MFX_REQUIRE(degree >= 1 && degree <= 32, "degree must be in 1..32");
     MFX_REQUIRE(lambda_max > lambda_min && lambda_min > 0.0, "need 0 < lambda_min < lambda_max");
     hipStream_t s = as_stream(stream);
-    DBuf<float> t, dd;
-    t.alloc(op->N);
-    dd.alloc(op->N);
-    chebyshev(*op, x, b, inv_diag, t.ptr, dd.ptr, degree, lambda_min, lambda_max, x_is_zero != 0, s);
+    // scratch of the handle: allocating it and freeing it on every call took
+    // ~100 us of a 740 us smoothing at 7.2M DoFs
+    if (op->cheb_t.n != op->N) op->cheb_t.alloc(op->N);
+    if (op->cheb_d.n != op->N) op->cheb_d.alloc(op->N);
+    chebyshev(*op, x, b, inv_diag, op->cheb_t.ptr, op->cheb_d.ptr, degree, lambda_min, lambda_max,
+              x_is_zero != 0, s);
     MFX_HIP(hipStreamSynchronize(s));
   });
 }

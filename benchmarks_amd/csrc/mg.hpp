@@ -13,33 +13,59 @@ namespace mfx {
 void vmult64(mfx_op &op, double *dst, const double *src, hipStream_t s);
 void vmult32(mfx_op &op, float *dst, const float *src, hipStream_t s);
 // `degree` Chebyshev(Jacobi) steps towards A x = b in FP32 on [lmin, lmax]
-// (t, d: scratch vectors of the operator's size)
+// (t, d: scratch vectors of the operator's size).  started: t already holds
+// the start value of A x (chebyshev_start's rows); leave_start: t is left as the
+// start value of A x for the final x.  Both only where
+// cheb_starts(op): the apply then adds to t without a start pass of its own.
 void chebyshev(mfx_op &op, float *x, const float *b, const float *dinv, float *t, float *d,
-               int degree, double lmin, double lmax, bool zero_initial, hipStream_t s);
+               int degree, double lmin, double lmax, bool zero_initial, hipStream_t s,
+               bool started = false, bool leave_start = false);
+bool cheb_starts(const mfx_op &op);
 // largest eigenvalue of D^-1 A from `iters` CG (Lanczos) steps, FP64
 double estimate_lambda_max(mfx_op &op, const double *inv_diag, int iters, hipStream_t s);
 
-// A 1D transfer matrix in CSR form (device arrays), applied along one axis of
-// a lexicographic (x fastest) node grid.
+// A 1D transfer matrix (device arrays), applied along one axis of a
+// lexicographic (x fastest) node grid: row i has span[i].y entries val[i width
+// ...] in the consecutive columns from span[i].x.
 template <typename T>
 struct AxisMatrix {
-  int rows = 0, cols = 0;
-  const int *rowptr = nullptr;
-  const int *col = nullptr;
+  int rows = 0, cols = 0, width = 0;
+  const int2 *span = nullptr;
   const T *val = nullptr;
+};
+
+// Operands of one pass: out = M in, or M (minuend - in); the rows of zero_rows
+// (bitmask) are set to zero; add: out += instead; start: beside out, out on
+// the rows of start_rows and 0 elsewhere.
+template <typename T>
+struct AxisIO {
+  const T *in = nullptr;
+  T *out = nullptr;
+  const T *minuend = nullptr;
+  const uint32_t *zero_rows = nullptr;
+  bool add = false;
+  T *start = nullptr;
+  const uint32_t *start_rows = nullptr;
 };
 
 // out[i0,i1,i2] (+)= sum_k M[i_axis][k] in[..k..]: `out_dims` are the output
 // grid's node counts, the input has M.cols nodes along `axis`.
 template <typename T>
-void launch_axis_pass(const AxisMatrix<T> &M, int axis, const uint32_t out_dims[3], const T *in,
-                      T *out, bool add, hipStream_t s);
+void launch_axis_pass(const AxisMatrix<T> &M, int axis, const uint32_t out_dims[3],
+                      const AxisIO<T> &io, hipStream_t s);
 
 // One Chebyshev step on FP32 vectors:
-//   r = b - t (r = b when t is null), d = c1 d + c2 dinv r, x = x + d
+//   r = b - t (r = b without has_t), d = c1 d + c2 dinv r, x = x + d
 // (x = d when x_zero: the iterate was zero).  c1 = 0 starts the recurrence.
-void launch_cheb_step(float *x, float *d, const float *b, const float *t, const float *dinv,
-                      float c1, float c2, bool x_zero, uint64_t n, hipStream_t s);
+// start (bitmask, optional): t = the new x on its rows, 0 elsewhere.
+void launch_cheb_step(float *x, float *d, const float *b, float *t, const float *dinv, float c1,
+                      float c2, bool has_t, bool x_zero, const uint32_t *start, uint64_t n,
+                      hipStream_t s);
+// b = r, 0 on the rows of the bitmask; z = x, r on the rows of the bitmask
+void launch_to_float_free(const double *r, float *b, const uint32_t *mask, uint64_t n,
+                          hipStream_t s);
+void launch_to_double_free(const float *x, const double *r, double *z, const uint32_t *mask,
+                           uint64_t n, hipStream_t s);
 // r = b - t
 void launch_residual_f32(float *r, const float *b, const float *t, uint64_t n, hipStream_t s);
 void launch_to_double(const float *in, double *out, uint64_t n, hipStream_t s);

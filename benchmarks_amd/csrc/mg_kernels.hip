@@ -24,50 +24,64 @@ inline unsigned grid_for(uint64_t n) {
   return (unsigned)std::max<uint64_t>(1, std::min<uint64_t>((n + kBlock - 1) / kBlock, 65536));
 }
 
-template <typename T, bool ADD>
-__global__ void k_axis_pass(const T *__restrict__ in, T *__restrict__ out, uint32_t n0, uint32_t n1,
-                            uint32_t n2, int axis, uint32_t in_len, const int *__restrict__ rowptr,
-                            const int *__restrict__ col, const T *__restrict__ val) {
-  const uint64_t total = (uint64_t)n0 * n1 * n2;
-  for (uint64_t t = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; t < total;
-       t += (uint64_t)gridDim.x * blockDim.x) {
-    const uint32_t i0 = (uint32_t)(t % n0);
-    const uint64_t q = t / n0;
-    const uint32_t i1 = (uint32_t)(q % n1), i2 = (uint32_t)(q / n1);
-    uint32_t row;
-    uint64_t base, stride;
+// One thread per output; the row's entries are consecutive inputs along the
+// axis (begin, count), so the loads of the inputs wait for one load only.
+// The fused ends of a V-cycle's transfers (AxisIO): the input as a residual
+// minuend - in, rows of the output set to zero, the output added to and the
+// start of the next A x written beside it.
+template <typename T>
+__global__ void __launch_bounds__(kBlock)
+k_axis_pass(AxisIO<T> io, uint32_t n0, uint32_t n1, uint32_t total, int axis, uint32_t in_len,
+            const int2 *__restrict__ span, const T *__restrict__ val, int width) {
+  const T *__restrict__ in = io.in;
+  const T *__restrict__ minuend = io.minuend;
+  for (uint32_t t = blockIdx.x * kBlock + threadIdx.x; t < total; t += gridDim.x * kBlock) {
+    const uint32_t q = t / n0, i0 = t - q * n0;
+    const uint32_t i2 = q / n1, i1 = q - i2 * n1;
+    uint32_t row, base, stride;
     if (axis == 0) {
       row = i0;
-      base = (uint64_t)in_len * q;
+      base = in_len * q;
       stride = 1;
     } else if (axis == 1) {
       row = i1;
-      base = i0 + (uint64_t)n0 * in_len * i2;
+      base = i0 + n0 * in_len * i2;
       stride = n0;
     } else {
       row = i2;
-      base = i0 + (uint64_t)n0 * i1;
-      stride = (uint64_t)n0 * n1;
+      base = i0 + n0 * i1;
+      stride = n0 * n1;
     }
+    const int2 sp = span[row];
+    const T *w = val + (size_t)row * width;
+    base += stride * (uint32_t)sp.x;
     T acc = 0;
-    for (int k = rowptr[row]; k < rowptr[row + 1]; ++k) acc += val[k] * in[base + stride * col[k]];
-    if (ADD)
-      out[t] += acc;
-    else
-      out[t] = acc;
+    for (int k = 0; k < sp.y; ++k) {
+      const uint32_t at = base + stride * (uint32_t)k;
+      acc += w[k] * (minuend ? minuend[at] - in[at] : in[at]);
+    }
+    if (io.zero_rows && (io.zero_rows[t >> 5] >> (t & 31) & 1)) acc = 0;
+    if (io.add) acc += io.out[t];
+    io.out[t] = acc;
+    if (io.start) io.start[t] = (io.start_rows[t >> 5] >> (t & 31) & 1) ? acc : T(0);
   }
 }
 
+// start (optional): also the start value of the next A x in t -- the new x on
+// the rows of the bitmask (identity rows), 0 elsewhere -- which spares the
+// apply its own start pass over x and t.
 __global__ void k_cheb_step(float *__restrict__ x, float *__restrict__ d,
-                            const float *__restrict__ b, const float *__restrict__ t,
-                            const float *__restrict__ dinv, float c1, float c2, int x_zero,
-                            uint64_t n) {
+                            const float *__restrict__ b, float *__restrict__ t,
+                            const float *__restrict__ dinv, float c1, float c2, int has_t,
+                            int x_zero, const uint32_t *__restrict__ start, uint64_t n) {
   for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
        i += (uint64_t)gridDim.x * blockDim.x) {
-    const float r = t ? b[i] - t[i] : b[i];
+    const float r = has_t ? b[i] - t[i] : b[i];
     const float dn = (c1 != 0.0f ? c1 * d[i] : 0.0f) + c2 * dinv[i] * r;
     d[i] = dn;
-    x[i] = x_zero ? dn : x[i] + dn;
+    const float xn = x_zero ? dn : x[i] + dn;
+    x[i] = xn;
+    if (start) t[i] = (start[i >> 5] >> (i & 31) & 1) ? xn : 0.0f;
   }
 }
 
@@ -82,6 +96,25 @@ __global__ void k_to_double(const float *__restrict__ in, double *__restrict__ o
   for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
        i += (uint64_t)gridDim.x * blockDim.x)
     out[i] = (double)in[i];
+}
+
+// FP64 <-> FP32 ends of the V-cycle: b = r with the constrained rows
+// (bitmask) zero; z = x with the constrained rows of r
+__global__ void k_to_float_free(const double *__restrict__ r, float *__restrict__ b,
+                                const uint32_t *__restrict__ mask, uint64_t n) {
+  for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
+       i += (uint64_t)gridDim.x * blockDim.x)
+    b[i] = (mask[i >> 5] >> (i & 31) & 1) ? 0.0f : (float)r[i];
+}
+__global__ void k_to_double_free(const float *__restrict__ x, const double *__restrict__ r,
+                                 double *__restrict__ z, const uint32_t *__restrict__ mask,
+                                 uint64_t n) {
+  for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
+       i += (uint64_t)gridDim.x * blockDim.x) {
+    double v = (double)x[i];
+    if (mask[i >> 5] >> (i & 31) & 1) v = r[i];
+    z[i] = v;
+  }
 }
 
 __global__ void k_set_listed_f32(float *__restrict__ dst, float v, const uint32_t *__restrict__ list,
@@ -152,33 +185,31 @@ __global__ void k_residual_f64(double *__restrict__ r, const double *__restrict_
 }  // namespace
 
 template <typename T>
-void launch_axis_pass(const AxisMatrix<T> &M, int axis, const uint32_t out_dims[3], const T *in,
-                      T *out, bool add, hipStream_t s) {
+void launch_axis_pass(const AxisMatrix<T> &M, int axis, const uint32_t out_dims[3],
+                      const AxisIO<T> &io, hipStream_t s) {
   MFX_REQUIRE(axis >= 0 && axis < 3, "axis must be 0, 1 or 2");
-  MFX_REQUIRE(M.rowptr && M.col && M.val && in && out, "transfer pass: null pointer");
+  MFX_REQUIRE(M.span && M.val && io.in && io.out, "transfer pass: null pointer");
   MFX_REQUIRE((uint32_t)M.rows == out_dims[axis], "transfer pass: matrix rows != output length");
+  MFX_REQUIRE(!io.start || io.start_rows, "transfer pass: start value without its rows");
   const uint64_t n = (uint64_t)out_dims[0] * out_dims[1] * out_dims[2];
+  const uint64_t n_in = n / out_dims[axis] * (uint64_t)M.cols;
+  MFX_REQUIRE(n < (1ull << 31) && n_in < (1ull << 31), "transfer pass: grid too large");
   if (n == 0) return;
-  if (add)
-    hipLaunchKernelGGL((k_axis_pass<T, true>), dim3(grid_for(n)), dim3(kBlock), 0, s, in, out,
-                       out_dims[0], out_dims[1], out_dims[2], axis, (uint32_t)M.cols, M.rowptr,
-                       M.col, M.val);
-  else
-    hipLaunchKernelGGL((k_axis_pass<T, false>), dim3(grid_for(n)), dim3(kBlock), 0, s, in, out,
-                       out_dims[0], out_dims[1], out_dims[2], axis, (uint32_t)M.cols, M.rowptr,
-                       M.col, M.val);
+  hipLaunchKernelGGL((k_axis_pass<T>), dim3(grid_for(n)), dim3(kBlock), 0, s, io, out_dims[0],
+                     out_dims[1], (uint32_t)n, axis, (uint32_t)M.cols, M.span, M.val, M.width);
   MFX_HIP(hipGetLastError());
 }
 template void launch_axis_pass<float>(const AxisMatrix<float> &, int, const uint32_t[3],
-                                      const float *, float *, bool, hipStream_t);
+                                      const AxisIO<float> &, hipStream_t);
 template void launch_axis_pass<double>(const AxisMatrix<double> &, int, const uint32_t[3],
-                                       const double *, double *, bool, hipStream_t);
+                                       const AxisIO<double> &, hipStream_t);
 
-void launch_cheb_step(float *x, float *d, const float *b, const float *t, const float *dinv,
-                      float c1, float c2, bool x_zero, uint64_t n, hipStream_t s) {
+void launch_cheb_step(float *x, float *d, const float *b, float *t, const float *dinv, float c1,
+                      float c2, bool has_t, bool x_zero, const uint32_t *start, uint64_t n,
+                      hipStream_t s) {
   if (n == 0) return;
   hipLaunchKernelGGL(k_cheb_step, dim3(grid_for(n)), dim3(kBlock), 0, s, x, d, b, t, dinv, c1, c2,
-                     (int)x_zero, n);
+                     (int)has_t, (int)x_zero, start, n);
   MFX_HIP(hipGetLastError());
 }
 
@@ -191,6 +222,20 @@ void launch_residual_f32(float *r, const float *b, const float *t, uint64_t n, h
 void launch_to_double(const float *in, double *out, uint64_t n, hipStream_t s) {
   if (n == 0) return;
   hipLaunchKernelGGL(k_to_double, dim3(grid_for(n)), dim3(kBlock), 0, s, in, out, n);
+  MFX_HIP(hipGetLastError());
+}
+
+void launch_to_float_free(const double *r, float *b, const uint32_t *mask, uint64_t n,
+                          hipStream_t s) {
+  if (n == 0) return;
+  hipLaunchKernelGGL(k_to_float_free, dim3(grid_for(n)), dim3(kBlock), 0, s, r, b, mask, n);
+  MFX_HIP(hipGetLastError());
+}
+
+void launch_to_double_free(const float *x, const double *r, double *z, const uint32_t *mask,
+                           uint64_t n, hipStream_t s) {
+  if (n == 0) return;
+  hipLaunchKernelGGL(k_to_double_free, dim3(grid_for(n)), dim3(kBlock), 0, s, x, r, z, mask, n);
   MFX_HIP(hipGetLastError());
 }
 

@@ -127,6 +127,9 @@ struct mfx_op {
   // CG scratch, allocated on first use
   DBuf<double> r, pdir, ap, part;
   DBuf<CgState> st;  // two (cg_run)
+  // scratch of mfx_chebyshev_f32 (which returns with its stream synchronized),
+  // allocated on first use
+  DBuf<float> cheb_t, cheb_d;
   int *h_done = nullptr;  // pinned
   ~mfx_op() {
     if (h_done) (void)hipHostFree(h_done);

@@ -14,10 +14,10 @@ namespace mfx {
 
 template <typename T>
 struct DevAxis {
-  DBuf<int> rowptr, col;
-  DBuf<T> val;
-  int rows = 0, cols = 0;
-  AxisMatrix<T> view() const { return {rows, cols, rowptr.ptr, col.ptr, val.ptr}; }
+  DBuf<int2> span;  // first column and entries of each row
+  DBuf<T> val;      // [rows][width]
+  int rows = 0, cols = 0, width = 0;
+  AxisMatrix<T> view() const { return {rows, cols, width, span.ptr, val.ptr}; }
 };
 
 struct HostCsr {
@@ -76,13 +76,28 @@ inline HostCsr transpose(const HostCsr &A) {
   return T;
 }
 
+// The rows as spans of consecutive columns (the entries between a row's first
+// and last column that the list leaves out are zeros).
 template <typename T>
 void upload(const HostCsr &h, DevAxis<T> &d) {
   d.rows = h.rows;
   d.cols = h.cols;
-  d.rowptr.upload(h.rowptr.data(), h.rowptr.size());
-  d.col.upload(h.col.data(), h.col.size());
-  std::vector<T> v(h.val.begin(), h.val.end());
+  std::vector<int2> span(h.rows);
+  d.width = 0;
+  for (int r = 0; r < h.rows; ++r) {
+    int lo = 0, hi = -1;
+    for (int k = h.rowptr[r]; k < h.rowptr[r + 1]; ++k) {
+      lo = k == h.rowptr[r] ? h.col[k] : std::min(lo, h.col[k]);
+      hi = std::max(hi, h.col[k]);
+    }
+    span[r] = make_int2(lo, hi - lo + 1 > 0 ? hi - lo + 1 : 0);
+    d.width = std::max(d.width, span[r].y);
+  }
+  std::vector<T> v((size_t)d.rows * d.width, T(0));
+  for (int r = 0; r < h.rows; ++r)
+    for (int k = h.rowptr[r]; k < h.rowptr[r + 1]; ++k)
+      v[(size_t)r * d.width + h.col[k] - span[r].x] = (T)h.val[k];
+  d.span.upload(span.data(), span.size());
   d.val.upload(v.data(), v.size());
 }
 
@@ -114,23 +129,47 @@ inline void build_transfer(const mfx_op &fine, const mfx_op &coarse, Transfer &t
   MFX_REQUIRE(fine.box.deform == coarse.box.deform, "transfer: operators on differently deformed meshes");
 }
 
-// prolongation: coarse (c0,c1,c2) -> x-pass (f0,c1,c2) -> y-pass (f0,f1,c2) -> z-pass (f0,f1,f2)
+// prolongation: coarse (c0,c1,c2) -> x-pass (f0,c1,c2) -> y-pass (f0,f1,c2) -> z-pass (f0,f1,f2).
+// add: dst += instead; start (may be tmp1): see AxisIO.
 template <typename T>
 void prolongate(const DevAxis<T> *P, const uint32_t f[3], const uint32_t c[3], const T *src, T *tmp1,
-                T *tmp2, T *dst, bool add, hipStream_t s) {
+                T *tmp2, T *dst, bool add, hipStream_t s, T *start = nullptr,
+                const uint32_t *start_rows = nullptr) {
   const uint32_t d1[3] = {f[0], c[1], c[2]}, d2[3] = {f[0], f[1], c[2]};
-  launch_axis_pass<T>(P[0].view(), 0, d1, src, tmp1, false, s);
-  launch_axis_pass<T>(P[1].view(), 1, d2, tmp1, tmp2, false, s);
-  launch_axis_pass<T>(P[2].view(), 2, f, tmp2, dst, add, s);
+  AxisIO<T> x, y, z;
+  x.in = src;
+  x.out = tmp1;
+  y.in = tmp1;
+  y.out = tmp2;
+  z.in = tmp2;
+  z.out = dst;
+  z.add = add;
+  z.start = start;
+  z.start_rows = start_rows;
+  launch_axis_pass<T>(P[0].view(), 0, d1, x, s);
+  launch_axis_pass<T>(P[1].view(), 1, d2, y, s);
+  launch_axis_pass<T>(P[2].view(), 2, f, z, s);
 }
-// restriction: fine (f0,f1,f2) -> z-pass (f0,f1,c2) -> y-pass (f0,c1,c2) -> x-pass (c0,c1,c2)
+// restriction: fine (f0,f1,f2) -> z-pass (f0,f1,c2) -> y-pass (f0,c1,c2) -> x-pass (c0,c1,c2) of src,
+// or of the residual minuend - src (tmp2 may then be src); zero_rows: coarse
+// rows set to zero
 template <typename T>
 void restrict_(const DevAxis<T> *R, const uint32_t f[3], const uint32_t c[3], const T *src, T *tmp1,
-               T *tmp2, T *dst, hipStream_t s) {
+               T *tmp2, T *dst, hipStream_t s, const T *minuend = nullptr,
+               const uint32_t *zero_rows = nullptr) {
   const uint32_t d1[3] = {f[0], f[1], c[2]}, d2[3] = {f[0], c[1], c[2]};
-  launch_axis_pass<T>(R[2].view(), 2, d1, src, tmp1, false, s);
-  launch_axis_pass<T>(R[1].view(), 1, d2, tmp1, tmp2, false, s);
-  launch_axis_pass<T>(R[0].view(), 0, c, tmp2, dst, false, s);
+  AxisIO<T> x, y, z;
+  z.in = src;
+  z.minuend = minuend;
+  z.out = tmp1;
+  y.in = tmp1;
+  y.out = tmp2;
+  x.in = tmp2;
+  x.out = dst;
+  x.zero_rows = zero_rows;
+  launch_axis_pass<T>(R[2].view(), 2, d1, z, s);
+  launch_axis_pass<T>(R[1].view(), 1, d2, y, s);
+  launch_axis_pass<T>(R[0].view(), 0, c, x, s);
 }
 
 }  // namespace mfx
