@@ -18,7 +18,38 @@ void set_error(const std::string &msg) { g_last_error = msg; }
 
 using namespace mfx;
 
+// Whether a box operator with the metric from the vertices runs the plane kernel
+// (plane_kernel.hpp) rather than the patch kernel or the per-column Gauss
+// kernel.  A wave of the plane kernel holds 64 / q cells and works a layer of
+// them off alone, so it needs a device full of waves (groups x layers) to
+// come ahead, the more the longer a layer takes (points, trilinear metric) and
+// the better the other kernel shares its work.  Below the lines the other
+// kernel is level to 2x faster (q >= 6 on a few thousand cells), above them
+// this one is: on 16M DoFs 1.0-2.1x (Gauss-Lobatto) and 1.1-3.0x (Gauss) in
+// FP64, 1.4-3.1x and 1.2-2.3x in FP32.  It has no instance where the planes do
+// not fit the registers (FP64 q >= 8, FP32 q >= 9).
+static bool plane_rule(const mfx_op &op, bool fp32) {
+  if (fp32 ? !plane_instance<float>(op.p, op.nq, op.colloc)
+           : !plane_instance<double>(op.p, op.nq, op.colloc))
+    return false;
+  const bool axes = op.box.deform == 0.0;
+  const int q = op.nq;
+  uint64_t need;
+  if (fp32)
+    need = axes || op.colloc ? 1024 : q <= 4 ? 2048 : 4096;
+  else if (axes)
+    need = op.colloc && q >= 6 ? 4096 : 2048;
+  else
+    need = q <= 3 ? 2048 : q <= 5 ? (op.colloc ? 4096 : 2048) : 8192;
+  return (uint64_t)op.plane_lay.groups * op.plane_lay.n[2] >= need;
+}
+
 static void finish_setup(mfx_op *op, int with_fp32, hipStream_t s) {
+  if (op->is_box && op->geometry == MFX_GEOM_ON_THE_FLY) {
+    op->plane_lay = plane_layout(op->nq, op->box.n);
+    op->plane64 = plane_rule(*op, false);
+    op->plane32 = with_fp32 && plane_rule(*op, true);
+  }
   op->cmask.alloc((op->N + 31) / 32 + 1);  // the last word: scratch of any_masked
   launch_bitmask(op->cons.ptr, op->n_cons, op->cmask.ptr, op->N, s);
   const uint64_t nq3 = (uint64_t)op->nq * op->nq * op->nq;
@@ -463,7 +494,7 @@ mfx_status mfx_op_vmult_add(mfx_op *op, double *dst, const double *src, void *st
   return guard([&] {
     MFX_REQUIRE(op && dst && src, "null pointer argument");
     MFX_REQUIRE(dst != src, "vmult_add: src and dst must not alias");
-    op->apply64(src, dst, as_stream(stream));
+    op->apply64(src, dst, as_stream(stream), nullptr, nullptr, false);
   });
 }
 

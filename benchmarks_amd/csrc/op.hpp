@@ -10,6 +10,7 @@
 #include "cg_state.hpp"
 #include "mfx_internal.hpp"
 #include "patch.hpp"
+#include "plane.hpp"
 
 namespace mfx {
 
@@ -170,14 +171,42 @@ struct mfx_op {
   uint32_t row_cells() const { return is_box && !colloc ? box.n[0] : 0; }
   // an undeformed box: every cell's Jacobian columns lie along x, y and z
   bool axis_cells() const { return is_box && !colloc && box.deform == 0.0; }
+  // Box operators with the metric from the vertices run the plane kernel where
+  // it is the faster one (plane_rule); the deterministic scatter is the patch
+  // kernel's.
+  bool plane64 = false, plane32 = false;
+  PlaneLayout plane_lay{};
+  template <typename T>
+  bool plane() const {
+    return (sizeof(T) == 8 ? plane64 : plane32) && !det;
+  }
+  template <typename T>
+  PlaneOp<T> plane_op(const T *eo_, const T *xq_, const T *wq_) const {
+    PlaneOp<T> o;
+    o.p = p;
+    o.nq = nq;
+    o.colloc = colloc;
+    o.axes = box.deform == 0.0;
+    o.lay = plane_lay;
+    o.eo = eo_;
+    o.xq = xq_;
+    o.wq = wq_;
+    o.cellX = cellX.ptr;
+    return o;
+  }
   uint32_t apply_blocks() const {
+    if (plane<double>()) return plane_lay.blocks();
     return patch ? (det ? grid64.det_dot : grid64.dot)
                  : apply_n_blocks(p, nq, colloc, E, row_cells());
   }
-  // dst += A_free src (no zeroing, no constrained rows)
+  // dst += A_free src (no zeroing, no constrained rows).  fresh: dst is zero on
+  // the free rows (the start of an apply), which every caller but vmult_add
+  // has it be.
   void apply64(const double *src, double *dst, hipStream_t s, double *partials = nullptr,
-               const int *skip = nullptr) const {
-    if (patch)
+               const int *skip = nullptr, bool fresh = true) const {
+    if (plane<double>())
+      launch_plane<double>(plane_op<double>(eo.ptr, xq.ptr, wq.ptr), src, dst, fresh, s, partials, skip);
+    else if (patch)
       launch_patch<double>(patch_op64(), src, dst, s, partials, skip);
     else if (geometry == MFX_GEOM_ON_THE_FLY)
       launch_apply_otf<double>(p, nq, B.ptr, D.ptr, eo.ptr, xq.ptr, wq.ptr, cellX.ptr, src, dst,
@@ -187,7 +216,9 @@ struct mfx_op {
                            skip, row_cells());
   }
   void apply32(const float *src, float *dst, hipStream_t s) const {
-    if (patch)
+    if (plane<float>())
+      launch_plane<float>(plane_op<float>(eo32.ptr, xq32.ptr, wq32.ptr), src, dst, true, s);
+    else if (patch)
       launch_patch<float>(patch_op32(), src, dst, s);
     else if (geometry == MFX_GEOM_ON_THE_FLY)
       launch_apply_otf<float>(p, nq, B32.ptr, D32.ptr, eo32.ptr, xq32.ptr, wq32.ptr, cellX.ptr,

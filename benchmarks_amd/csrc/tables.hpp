@@ -160,8 +160,8 @@ constexpr int eo_table_size(int O, int I) {
 
 // out = M in with M given by its even-odd tables (eo_table_size(O, I)
 // values at tab, read with compile-time offsets, so through the scalar cache)
-template <int O, int I, int S, typename T>
-__device__ __forceinline__ void eo_tab(const T *__restrict__ tab, const T *in, T *out) {
+template <int O, int I, int S, typename Tab, typename T>
+__device__ __forceinline__ void eo_tab(Tab tab, const T *in, T *out) {
   static_assert(S == 1 || S == -1, "centro-symmetry sign");
   constexpr int HI = I / 2, HO = O / 2, mi = I - 1, mo = O - 1;
   constexpr int CG = HO * HI, MC = 2 * HO * HI, MR = MC + ((I & 1) ? HO : 0), CT = MR + HI;
