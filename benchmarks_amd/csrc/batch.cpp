@@ -14,7 +14,9 @@
 // vertices (patch.hip), over the concatenated patches of all instances of
 // that degree.  At creation an autotuner may time the tile variants of the
 // collocation kernel (cells per workgroup, G prefetch) and the patch kernel
-// per degree on the batch's own cells and keep the fastest.
+// per degree on the batch's own cells and keep the fastest.  The CG steps of a
+// small batch use neither: they run in three launches, one of which applies the
+// operators of all degrees (small_batch).
 #include <algorithm>
 #include <chrono>
 #include <memory>
@@ -28,7 +30,7 @@
 namespace mfx {
 namespace {
 
-constexpr uint64_t kSegment = 8192;  // DoFs per vector-kernel workgroup
+constexpr uint64_t kSegment = 8192;  // DoFs per vector-kernel workgroup of a large batch
 constexpr int kGraphSteps = 8;       // CG steps per graph launch
 
 struct OpDeleter {
@@ -77,15 +79,23 @@ struct mfx_batch {
   // fused p.Ap: per instance its range of the patch kernel's partials
   DBuf<PapRange> pap_ranges;
   DBuf<double> part_c;  // constrained-row share of p.Ap per segment
+  // a small batch: tiles of all degrees for one launch, ordered by instance
+  bool small = false, chosen = false;  // chosen: a variant was set by the caller
+  DBuf<BatchTile> tiles;
+  DBuf<uint32_t> inst_tile;
+  DBuf<double> part_t;  // p.Ap per tile
   // CG scratch
-  DBuf<BatchCg> st;
+  DBuf<BatchCg> st;     // two states per instance: see steps()
   DBuf<double> r, p, ap, t, part, part2, ones;
-  DBuf<int> flags, n_active;
-  int *h_active = nullptr;
+  DBuf<int> flags;
+  int *n_active = nullptr;  // pinned host memory, written by the count kernel
+  hipEvent_t ev[2] = {nullptr, nullptr};
   hipStream_t cs = nullptr;
 
   ~mfx_batch() {
-    if (h_active) (void)hipHostFree(h_active);
+    for (hipEvent_t e : ev)
+      if (e) (void)hipEventDestroy(e);
+    if (n_active) (void)hipHostFree(n_active);
     if (cs) (void)hipStreamDestroy(cs);
   }
 
@@ -111,6 +121,29 @@ struct mfx_batch {
       if (!g.on_the_fly(g.variant)) return false;
     return true;
   }
+  // kGraphSteps CG steps; the states are st[0..n) before and after
+  void steps(double *x, const double *dinv, hipStream_t s) {
+    const uint32_t n = (uint32_t)ops.size();
+    if (!small || chosen) {
+      for (int k = 0; k < kGraphSteps; ++k) cg_step(x, dinv, s);
+      return;
+    }
+    BatchTiles t{};
+    t.tiles = tiles.ptr;
+    for (auto &g : groups)
+      t.degree[g.p - 2] = {g.cellX.ptr, g.w.ptr, g.xq.ptr};
+    BatchCg *cur = st.ptr, *other = st.ptr + n;
+    for (int k = 0; k < kGraphSteps; ++k) {
+      launch_b_direction_small(segs.ptr, n_segs, cur, k ? other : nullptr, inst_seg.ptr, part.ptr,
+                               part2.ptr, r.ptr, dinv, cmask.ptr, p.ptr, ap.ptr, x, part_c.ptr,
+                               flags.ptr, s);
+      if (k) std::swap(cur, other);
+      launch_b_apply(t, (uint32_t)tiles.n, p.ptr, ap.ptr, flags.ptr, part_t.ptr, s);
+      launch_b_update_small(segs.ptr, n_segs, cur, inst_seg.ptr, inst_tile.ptr, part_t.ptr,
+                            part_c.ptr, r.ptr, ap.ptr, dinv, part.ptr, part2.ptr, s);
+    }
+    launch_b_check(cur, st.ptr, inst_seg.ptr, n, part.ptr, part2.ptr, flags.ptr, n_active, s);
+  }
   void cg_step(double *x, const double *dinv, hipStream_t s) {
     // ap leaves the direction pass with the identity rows set
     launch_b_direction(segs.ptr, n_segs, st.ptr, r.ptr, dinv, cmask.ptr, p.ptr, ap.ptr, x,
@@ -125,8 +158,8 @@ struct mfx_batch {
       launch_b_alpha(st.ptr, inst_seg.ptr, (uint32_t)ops.size(), part.ptr, s);
     }
     launch_b_update(segs.ptr, n_segs, st.ptr, r.ptr, ap.ptr, dinv, part.ptr, part2.ptr, s);
-    launch_b_check(st.ptr, inst_seg.ptr, (uint32_t)ops.size(), part.ptr, part2.ptr, flags.ptr,
-                   n_active.ptr, s);
+    launch_b_check(st.ptr, st.ptr, inst_seg.ptr, (uint32_t)ops.size(), part.ptr, part2.ptr,
+                   flags.ptr, n_active, s);
   }
 };
 
@@ -168,6 +201,23 @@ void autotune(mfx_batch &b, hipStream_t s) {
       }
     }
   }
+}
+
+// Whether the CG steps run in three launches (k_b_direction_small and after in
+// batch_kernels.hip), unless the caller chose a variant.  A step then took, us
+// against the separate launches with tuned variants: 18 against 36 (one problem,
+// 36k rows), 28 against 53 (0.49M), 52 against 96 (five degrees, 1.2M), 136 against
+// 160 (7.8M points), 210 against 262 (64 problems, 11.4M points), 298 against 297
+// (16.6M points).  Every workgroup sums all partials of its instance, so one
+// large instance ends it too: with 5700 partials 102 -> 116 us at degree 6 (85 -> 76 at
+// degree 3).
+bool small_batch(const mfx_batch &b) {
+  uint64_t points = 0, partials = 0;
+  for (auto &op : b.ops) {
+    points += (uint64_t)op->E * (op->p + 1) * (op->p + 1) * (op->p + 1);
+    partials = std::max<uint64_t>(partials, op->E / batch_tile_cells(op->p) + op->N / kSegSmall);
+  }
+  return points <= 12000000 && partials <= 4096;
 }
 
 // The on-the-fly form of a degree group: every instance's patch map (the
@@ -339,13 +389,32 @@ mfx_status mfx_batch_create(const mfx_batch_instance *inst, int n, int tune, mfx
     b->cmask.alloc(b->N);
     MFX_HIP(hipMemsetAsync(b->cmask.ptr, 0, b->N, s));
     launch_mark_u8(b->cons.ptr, b->n_cons, b->cmask.ptr, s);
+    b->small = small_batch(*b);
+    if (b->small) {
+      std::vector<BatchTile> tiles;
+      std::vector<uint32_t> inst_tile(n + 1, 0), cells(7, 0);
+      for (int i = 0; i < n; ++i) {
+        const mfx_op &op = *b->ops[i];
+        const int p = op.p;
+        const uint32_t E = op.E, per = batch_tile_cells(p);
+        for (uint32_t e = 0; e < E; e += per)
+          tiles.push_back({(uint32_t)i, (uint32_t)p, e, std::min(per, E - e), cells[p] + e,
+                           (uint32_t)b->off[i], op.box.n[0], op.box.n[1], op.box.n[2], 0});
+        cells[p] += E;
+        inst_tile[i + 1] = (uint32_t)tiles.size();
+      }
+      b->tiles.upload(tiles.data(), tiles.size());
+      b->inst_tile.upload(inst_tile.data(), inst_tile.size());
+      b->part_t.alloc(tiles.size());
+    }
     // segments: contiguous DoF ranges of one instance
+    const uint64_t seg_rows = b->small ? kSegSmall : kSegment;
     std::vector<Seg> segs;
     std::vector<uint32_t> inst_seg(n + 1, 0);
     for (int i = 0; i < n; ++i) {
       inst_seg[i] = (uint32_t)segs.size();
-      for (uint64_t a = b->off[i]; a < b->off[i + 1]; a += kSegment)
-        segs.push_back({a, std::min(a + kSegment, b->off[i + 1]), (uint32_t)i, 0});
+      for (uint64_t a = b->off[i]; a < b->off[i + 1]; a += seg_rows)
+        segs.push_back({a, std::min(a + seg_rows, b->off[i + 1]), (uint32_t)i, 0});
     }
     inst_seg[n] = (uint32_t)segs.size();
     b->n_segs = (uint32_t)segs.size();
@@ -421,6 +490,7 @@ mfx_status mfx_batch_set_variant(mfx_batch *b, int degree, int variant) {
       if (g.p != degree) continue;
       MFX_REQUIRE(variant >= 0 && variant < g.n_variants(), "variant out of range");
       g.variant = variant;
+      b->chosen = true;
       return;
     }
     throw Error{MFX_ERR_INVALID_ARG, "no instance of degree " + std::to_string(degree)};
@@ -467,11 +537,12 @@ mfx_status mfx_batch_cg_solve(mfx_batch *b, double *x, const double *rhs, const 
       b->part2.alloc(b->n_segs);
     }
     if (!b->st.ptr) {
-      b->st.alloc(n);
+      b->st.alloc(2 * (size_t)n);
       b->flags.alloc(n);
-      b->n_active.alloc(1);
     }
-    if (!b->h_active) MFX_HIP(hipHostMalloc(reinterpret_cast<void **>(&b->h_active), sizeof(int)));
+    if (!b->n_active) MFX_HIP(hipHostMalloc(reinterpret_cast<void **>(&b->n_active), sizeof(int)));
+    for (hipEvent_t &e : b->ev)
+      if (!e) MFX_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
     const double *dinv = inv_diag;
     if (!dinv) {
       if (b->ones.n != b->N) {
@@ -487,9 +558,9 @@ mfx_status mfx_batch_cg_solve(mfx_batch *b, double *x, const double *rhs, const 
     launch_b_residual(b->segs.ptr, b->n_segs, b->r.ptr, rhs, b->t.ptr, dinv, b->part.ptr,
                       b->part2.ptr, s);
     launch_b_init(b->st.ptr, b->inst_seg.ptr, n, b->part.ptr, b->part2.ptr, abs_tol, rel_tol,
-                  max_steps, b->flags.ptr, b->n_active.ptr, s);
-    MFX_HIP(hipMemcpyAsync(b->h_active, b->n_active.ptr, sizeof(int), hipMemcpyDeviceToHost, s));
+                  max_steps, b->flags.ptr, b->n_active, s);
     MFX_HIP(hipStreamSynchronize(s));
+    volatile const int *active = b->n_active;
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
     struct GraphGuard {
@@ -500,21 +571,25 @@ mfx_status mfx_batch_cg_solve(mfx_batch *b, double *x, const double *rhs, const 
         if (g) (void)hipGraphDestroy(g);
       }
     } gg{graph, exec};
-    if (use_graph && *b->h_active > 0) {
+    if (use_graph && *active > 0) {
       MFX_HIP(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
-      for (int k = 0; k < kGraphSteps; ++k) b->cg_step(x, dinv, s);
+      b->steps(x, dinv, s);
       MFX_HIP(hipStreamEndCapture(s, &graph));
       MFX_HIP(hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0));
     }
+    // Two rounds are in flight: the count of one is read while the next runs
+    // (waiting for each before launching the next left the device idle for 33 us
+    // of a round's 250-400).  A round after the last finds every instance done and
+    // changes nothing; the one count both write only falls.
     const int max_rounds = max_steps / kGraphSteps + 2;
-    for (int round = 0; *b->h_active > 0 && round < max_rounds; ++round) {
+    for (int round = 0; *active > 0 && round < max_rounds; ++round) {
       if (exec) {
         MFX_HIP(hipGraphLaunch(exec, s));
       } else {
-        for (int k = 0; k < kGraphSteps; ++k) b->cg_step(x, dinv, s);
+        b->steps(x, dinv, s);
       }
-      MFX_HIP(hipMemcpyAsync(b->h_active, b->n_active.ptr, sizeof(int), hipMemcpyDeviceToHost, s));
-      MFX_HIP(hipStreamSynchronize(s));
+      MFX_HIP(hipEventRecord(b->ev[round & 1], s));
+      if (round > 0) MFX_HIP(hipEventSynchronize(b->ev[~round & 1]));
     }
     launch_b_finish(b->segs.ptr, b->n_segs, b->st.ptr, x, b->p.ptr, s);
     std::vector<BatchCg> fin(n);

@@ -63,9 +63,42 @@ void launch_mark_u8(const uint32_t *list, uint64_t n, uint8_t *mask, hipStream_t
 void launch_b_update(const Seg *segs, uint32_t n_segs, const BatchCg *st, double *r,
                      const double *ap, const double *dinv, double *part_rr, double *part_rz,
                      hipStream_t s);
-// convergence test, beta, gamma; flags and *n_active as in launch_b_init
-void launch_b_check(BatchCg *st, const uint32_t *inst_seg, uint32_t n_inst, const double *part_rr,
-                    const double *part_rz, int *flags, int *n_active, hipStream_t s);
+// convergence test, beta, gamma, from state sa to sb (which may be sa); flags
+// and *n_active as in launch_b_init
+void launch_b_check(const BatchCg *sa, BatchCg *sb, const uint32_t *inst_seg, uint32_t n_inst,
+                    const double *part_rr, const double *part_rz, int *flags, int *n_active,
+                    hipStream_t s);
+
+// ---- a step of a small batch in three launches (segments of <= kSegSmall rows) ----
+constexpr uint64_t kSegSmall = 1024;
+// cells first .. first + n of an instance of n0 x n1 x n2 cells and degree p,
+// which are cell .. cell + n of their degree; off: the instance's first row
+struct BatchTile {
+  uint32_t inst, p, first, n, cell, off, n0, n1, n2, pad;
+};
+struct BatchTiles {
+  const BatchTile *tiles;
+  struct Degree {
+    const double *cellX, *w, *xq;  // cell vertices, quadrature weights and points
+  } degree[5];                     // p = 2..6
+};
+// cells of a tile of degree p
+uint32_t batch_tile_cells(int p);
+// launch_b_check from sa to sb and launch_b_direction with the result; with
+// sb = nullptr, launch_b_direction with sa
+void launch_b_direction_small(const Seg *segs, uint32_t n_segs, const BatchCg *sa, BatchCg *sb,
+                              const uint32_t *inst_seg, const double *part_rr,
+                              const double *part_rz, const double *r, const double *dinv,
+                              const uint8_t *cmask, double *p, double *ap, double *x,
+                              double *part_c, int *flags, hipStream_t s);
+// dst += A src on the cells of the instances not done, p.Ap per tile to part
+void launch_b_apply(const BatchTiles &t, uint32_t n_tiles, const double *src, double *dst,
+                    const int *done, double *part, hipStream_t s);
+// alpha from an instance's tiles [inst_tile[i], inst_tile[i + 1]) and segments, then launch_b_update
+void launch_b_update_small(const Seg *segs, uint32_t n_segs, BatchCg *st, const uint32_t *inst_seg,
+                           const uint32_t *inst_tile, const double *part_t, const double *part_c,
+                           double *r, const double *ap, const double *dinv, double *part_rr,
+                           double *part_rz, hipStream_t s);
 // dst[i] = src[i] + offset for valid entries (invalid stays invalid)
 void launch_offset_map(const uint32_t *src, uint32_t *dst, uint64_t n, uint32_t offset,
                        hipStream_t s);
