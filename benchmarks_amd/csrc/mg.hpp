@@ -54,6 +54,29 @@ template <typename T>
 void launch_axis_pass(const AxisMatrix<T> &M, int axis, const uint32_t out_dims[3],
                       const AxisIO<T> &io, hipStream_t s);
 
+// All three axes in one launch (out = M_z x M_y x M_x in); false, and nothing
+// done, unless every row has 2 (or every row 3) entries at most.
+template <typename T>
+bool launch_axis_all(const AxisMatrix<T> M[3], const AxisIO<T> &io, hipStream_t s);
+
+// An assembled Q_1 operator on a node grid whose boundary rows are constrained
+// (identity rows, in the bitmask): 27 entries per row, val[k n + i].
+struct Stencil {
+  const float *val = nullptr;
+  const uint32_t *mask = nullptr;
+  uint32_t dims[3] = {0, 0, 0};
+};
+// x = 1 on the nodes of one of 27 colours, 0 elsewhere; y = A x to the stencil
+void launch_colour(double *x, const uint32_t dims[3], uint32_t colour, hipStream_t s);
+void launch_take_colour(const double *y, float *val, const uint32_t dims[3], uint32_t colour,
+                        hipStream_t s);
+// kStep: launch_cheb_step with t = A x, result in xo; kFromZero: the first two
+// steps from zero, with x = c0 dinv b after the first; kResidual: xo = b - A x
+enum class StencilMode { kStep, kFromZero, kResidual };
+void launch_stencil_step(const Stencil &A, StencilMode mode, const float *x, float *xo, float *d,
+                         const float *b, const float *dinv, float c0, float c1, float c2,
+                         hipStream_t s);
+
 // One Chebyshev step on FP32 vectors:
 //   r = b - t (r = b without has_t), d = c1 d + c2 dinv r, x = x + d
 // (x = d when x_zero: the iterate was zero).  c1 = 0 starts the recurrence.

@@ -67,6 +67,128 @@ k_axis_pass(AxisIO<T> io, uint32_t n0, uint32_t n1, uint32_t total, int axis, ui
   }
 }
 
+// All three axes in one launch, for rows of at most W entries: every thread
+// loads its W^3 inputs at once.  A pass costs a launch and a chain of loads
+// whatever its size (4.5 us of a V-cycle's each); the two launches saved
+// outweigh the loads the passes share up to the largest grids measured.  V-cycle of
+// Q_4 on 32^3 cells 698 -> 664 us, of Q_1 on 64^3 cells 197 -> 165, on 128^3
+// cells 750 -> 700.
+template <typename T, int W>
+__global__ void __launch_bounds__(kBlock)
+k_axis_all(AxisIO<T> io, AxisMatrix<T> X, AxisMatrix<T> Y, AxisMatrix<T> Z) {
+  const T *__restrict__ in = io.in;
+  const T *__restrict__ minuend = io.minuend;
+  const uint32_t total = (uint32_t)X.rows * Y.rows * Z.rows;
+  for (uint32_t t = blockIdx.x * kBlock + threadIdx.x; t < total; t += gridDim.x * kBlock) {
+    const uint32_t q = t / X.rows, i0 = t - q * X.rows, i2 = q / Y.rows, i1 = q - i2 * Y.rows;
+    const int2 sx = X.span[i0], sy = Y.span[i1], sz = Z.span[i2];
+    T v[W][W][W], wx[W], wy[W], wz[W];
+#pragma unroll
+    for (int k = 0; k < W; ++k) {
+      wx[k] = X.val[(size_t)i0 * W + k];
+      wy[k] = Y.val[(size_t)i1 * W + k];
+      wz[k] = Z.val[(size_t)i2 * W + k];
+    }
+#pragma unroll
+    for (int c = 0; c < W; ++c)
+#pragma unroll
+      for (int b = 0; b < W; ++b)
+#pragma unroll
+        for (int a = 0; a < W; ++a) {
+          v[c][b][a] = T(0);
+          if (a >= sx.y || b >= sy.y || c >= sz.y) continue;
+          const uint32_t at =
+              sx.x + a + (uint32_t)X.cols * (sy.x + b + (uint32_t)Y.cols * (sz.x + c));
+          v[c][b][a] = minuend ? minuend[at] - in[at] : in[at];
+        }
+    T acc = 0;
+#pragma unroll
+    for (int c = 0; c < W; ++c) {
+      T ay = 0;
+#pragma unroll
+      for (int b = 0; b < W; ++b) {
+        T ax = 0;
+#pragma unroll
+        for (int a = 0; a < W; ++a) ax += wx[a] * v[c][b][a];
+        ay += wy[b] * ax;
+      }
+      acc += wz[c] * ay;
+    }
+    if (io.zero_rows && (io.zero_rows[t >> 5] >> (t & 31) & 1)) acc = 0;
+    if (io.add) acc += io.out[t];
+    io.out[t] = acc;
+    if (io.start) io.start[t] = (io.start_rows[t >> 5] >> (t & 31) & 1) ? acc : T(0);
+  }
+}
+
+// ---- Q_1 levels with an assembled operator ----
+// Row i of A couples the 3 x 3 x 3 nodes around node i: entry k = 9 dz + 3 dy + dx
+// (each 0..2, offset -1) at st[k n + i].  The constrained rows (bitmask) are
+// identity rows; every node of the grid's boundary is one.
+
+// x = 1 on the nodes of one of the 27 colours (indices modulo 3), 0 elsewhere
+__global__ void k_colour(double *__restrict__ x, uint32_t n0, uint32_t n1, uint32_t total,
+                         uint32_t c) {
+  for (uint32_t i = blockIdx.x * kBlock + threadIdx.x; i < total; i += gridDim.x * kBlock) {
+    const uint32_t q = i / n0, ix = i - q * n0, iz = q / n1, iy = q - iz * n1;
+    x[i] = ix % 3 + 3 * (iy % 3) + 9 * (iz % 3) == c ? 1.0 : 0.0;
+  }
+}
+// y = A x for x of colour c: the entry of each row's only neighbour of the colour
+__global__ void k_take_colour(const double *__restrict__ y, float *__restrict__ st, uint32_t n0,
+                              uint32_t n1, uint32_t total, uint32_t c) {
+  for (uint32_t i = blockIdx.x * kBlock + threadIdx.x; i < total; i += gridDim.x * kBlock) {
+    const uint32_t q = i / n0, ix = i - q * n0, iz = q / n1, iy = q - iz * n1;
+    const uint32_t dx = (c % 3 + 4 - ix % 3) % 3, dy = (c / 3 % 3 + 4 - iy % 3) % 3,
+                   dz = (c / 9 + 4 - iz % 3) % 3;
+    st[(size_t)(9 * dz + 3 * dy + dx) * total + i] = (float)y[i];
+  }
+}
+
+// A Chebyshev step (launch_cheb_step) with r = b - A x formed in place:
+// xo = x + d.  FROM_ZERO: x is the first iterate, x = c0 dinv b (not stored),
+// and d_0 = x.  RESIDUAL: xo = r only.  At 33^3 rows it is bound by its launch
+// and one batch of loads, 3.2 us in place of a matrix-free apply (5.6 us) and a
+// step on vectors (4.5 us); at 2M rows by the bytes of the entries, which are
+// more than the apply's vertices but need no atomics and no zeroed result: V-cycle of
+// Q_1 on 64^3 cells 419 -> 197 us, on 128^3 cells 1746 -> 750.
+template <bool FROM_ZERO, bool RESIDUAL>
+__global__ void __launch_bounds__(kBlock)
+k_stencil_step(const float *__restrict__ st, const uint32_t *__restrict__ mask,
+               const float *__restrict__ x, float *__restrict__ xo, float *__restrict__ d,
+               const float *__restrict__ b, const float *__restrict__ dinv, float c0, float c1,
+               float c2, int n0, int n01, uint32_t total) {
+  const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
+  if (i >= total) return;
+  const bool cons = mask[i >> 5] >> (i & 31) & 1;
+  float s[3] = {0.0f, 0.0f, 0.0f};
+  const float xi = FROM_ZERO ? c0 * dinv[i] * b[i] : x[i];
+  if (cons) {
+    s[0] = xi;
+  } else {
+    // all loads before the first use
+    float a[27], v[27], w[FROM_ZERO ? 27 : 1];
+#pragma unroll
+    for (int k = 0; k < 27; ++k) {
+      const uint32_t j = (uint32_t)((int)i + (k / 9 - 1) * n01 + (k / 3 % 3 - 1) * n0 + k % 3 - 1);
+      a[k] = st[(size_t)k * total + i];
+      v[k] = FROM_ZERO ? b[j] : x[j];
+      if (FROM_ZERO) w[k] = dinv[j];
+    }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int k = 0; k < 27; ++k) s[k / 9] += a[k] * (FROM_ZERO ? c0 * w[k] * v[k] : v[k]);
+  }
+  const float r = b[i] - ((s[0] + s[1]) + s[2]);
+  if constexpr (RESIDUAL) {
+    xo[i] = r;
+  } else {
+    const float dn = (FROM_ZERO ? c1 * xi : c1 != 0.0f ? c1 * d[i] : 0.0f) + c2 * dinv[i] * r;
+    d[i] = dn;
+    xo[i] = xi + dn;
+  }
+}
+
 // start (optional): also the start value of the next A x in t -- the new x on
 // the rows of the bitmask (identity rows), 0 elsewhere -- which spares the
 // apply its own start pass over x and t.
@@ -203,6 +325,64 @@ template void launch_axis_pass<float>(const AxisMatrix<float> &, int, const uint
                                       const AxisIO<float> &, hipStream_t);
 template void launch_axis_pass<double>(const AxisMatrix<double> &, int, const uint32_t[3],
                                        const AxisIO<double> &, hipStream_t);
+
+template <typename T>
+bool launch_axis_all(const AxisMatrix<T> M[3], const AxisIO<T> &io, hipStream_t s) {
+  const int w = M[0].width;
+  if ((w != 2 && w != 3) || M[1].width != w || M[2].width != w) return false;
+  uint64_t n = 1, n_in = 1;
+  for (int a = 0; a < 3; ++a) {
+    MFX_REQUIRE(M[a].span && M[a].val, "transfer: null pointer");
+    n *= (uint64_t)M[a].rows;
+    n_in *= (uint64_t)M[a].cols;
+  }
+  MFX_REQUIRE(io.in && io.out && io.in != io.out, "transfer: bad input or output");
+  MFX_REQUIRE(!io.start || io.start_rows, "transfer: start value without its rows");
+  MFX_REQUIRE(n < (1ull << 31) && n_in < (1ull << 31), "transfer: grid too large");
+  if (n == 0) return true;
+  if (w == 2)
+    hipLaunchKernelGGL((k_axis_all<T, 2>), dim3(grid_for(n)), dim3(kBlock), 0, s, io, M[0], M[1],
+                       M[2]);
+  else
+    hipLaunchKernelGGL((k_axis_all<T, 3>), dim3(grid_for(n)), dim3(kBlock), 0, s, io, M[0], M[1],
+                       M[2]);
+  MFX_HIP(hipGetLastError());
+  return true;
+}
+template bool launch_axis_all<float>(const AxisMatrix<float>[3], const AxisIO<float> &, hipStream_t);
+
+void launch_colour(double *x, const uint32_t dims[3], uint32_t colour, hipStream_t s) {
+  const uint32_t n = dims[0] * dims[1] * dims[2];
+  hipLaunchKernelGGL(k_colour, dim3(grid_for(n)), dim3(kBlock), 0, s, x, dims[0], dims[1], n,
+                     colour);
+  MFX_HIP(hipGetLastError());
+}
+void launch_take_colour(const double *y, float *st, const uint32_t dims[3], uint32_t colour,
+                        hipStream_t s) {
+  const uint32_t n = dims[0] * dims[1] * dims[2];
+  hipLaunchKernelGGL(k_take_colour, dim3(grid_for(n)), dim3(kBlock), 0, s, y, st, dims[0], dims[1],
+                     n, colour);
+  MFX_HIP(hipGetLastError());
+}
+void launch_stencil_step(const Stencil &A, StencilMode mode, const float *x, float *xo, float *d,
+                         const float *b, const float *dinv, float c0, float c1, float c2,
+                         hipStream_t s) {
+  const uint32_t n = A.dims[0] * A.dims[1] * A.dims[2];
+  MFX_REQUIRE(A.val && A.mask && xo != x, "stencil step: bad arguments");
+  const dim3 grid((n + kBlock - 1) / kBlock), block(kBlock);
+  const int n0 = (int)A.dims[0], n01 = (int)(A.dims[0] * A.dims[1]);
+#define MFX_STEP(Z, R)                                                                          \
+  hipLaunchKernelGGL((k_stencil_step<Z, R>), grid, block, 0, s, A.val, A.mask, x, xo, d, b, dinv, \
+                     c0, c1, c2, n0, n01, n)
+  if (mode == StencilMode::kFromZero)
+    MFX_STEP(true, false);
+  else if (mode == StencilMode::kResidual)
+    MFX_STEP(false, true);
+  else
+    MFX_STEP(false, false);
+#undef MFX_STEP
+  MFX_HIP(hipGetLastError());
+}
 
 void launch_cheb_step(float *x, float *d, const float *b, float *t, const float *dinv, float c1,
                       float c2, bool has_t, bool x_zero, const uint32_t *start, uint64_t n,
