@@ -80,18 +80,16 @@ static void finish_setup(mfx_op *op, int with_fp32, hipStream_t s) {
         launch_patch_geometry<float>(op->p, op->lay, op->G32.ptr, op->Gp32.ptr, s);
       }
     }
-    op->B32.alloc(op->B.n);
-    launch_to_float(op->B.ptr, op->B32.ptr, op->B.n, s);
-    op->D32.alloc(op->D.n);
-    launch_to_float(op->D.ptr, op->D32.ptr, op->D.n, s);
-    if (op->eo.n) {
-      op->eo32.alloc(op->eo.n);
-      launch_to_float(op->eo.ptr, op->eo32.ptr, op->eo.n, s);
-    }
-    op->xq32.alloc(op->xq.n);
-    launch_to_float(op->xq.ptr, op->xq32.ptr, op->xq.n, s);
-    op->wq32.alloc(op->wq.n);
-    launch_to_float(op->wq.ptr, op->wq32.ptr, op->wq.n, s);
+    op->tables32.alloc(op->tables.n);
+    launch_to_float(op->tables.ptr, op->tables32.ptr, op->tables.n, s);
+    auto part = [&](const DView<double> &v) {
+      return DView<float>{op->tables32.ptr + (v.ptr - op->tables.ptr), v.n};
+    };
+    op->B32 = part(op->B);
+    op->D32 = part(op->D);
+    if (op->eo.n) op->eo32 = part(op->eo);
+    op->xq32 = part(op->xq);
+    op->wq32 = part(op->wq);
   }
   MFX_HIP(hipStreamSynchronize(s));
 }
@@ -116,13 +114,12 @@ static void common_init(mfx_op *op, int p, int nq, int quad, int geometry) {
     MFX_REQUIRE(gll_d_table_error(nq, D.data()) <= 1e-13 * mx,
                 "compile-time GLL derivative table disagrees with the basis tables");
   }
-  op->B.upload(B.data(), B.size());
-  op->D.upload(D.data(), D.size());
+  std::vector<double> eo;
   if (!op->colloc) {
     // even-odd tables of the line-form Gauss kernel: B and D on symmetric
     // points are centro-symmetric and centro-antisymmetric
     const int nm = p + 1;
-    std::vector<double> Bt((size_t)nm * nq), Dt((size_t)nq * nq), eo;
+    std::vector<double> Bt((size_t)nm * nq), Dt((size_t)nq * nq);
     for (int q = 0; q < nq; ++q)
       for (int m = 0; m < nm; ++m) Bt[(size_t)m * nq + q] = B[(size_t)q * nm + m];
     for (int i = 0; i < nq; ++i)
@@ -132,11 +129,24 @@ static void common_init(mfx_op *op, int p, int nq, int quad, int geometry) {
     dev = std::max(dev, eo_tables(D.data(), nq, nq, -1, eo));
     dev = std::max(dev, eo_tables(Dt.data(), nq, nq, -1, eo));
     MFX_REQUIRE(dev <= 1e-13, "basis tables are not centro-symmetric");
-    op->eo.upload(eo.data(), eo.size());
   }
-  op->xq.upload(xq.data(), xq.size());
-  op->wq.upload(wq.data(), wq.size());
-  op->support.upload(sup.data(), sup.size());
+  std::vector<double> all;
+  std::vector<std::pair<DView<double> *, size_t>> at;
+  auto add = [&](DView<double> &v, const std::vector<double> &t) {
+    v.n = t.size();
+    if (t.empty()) return;
+    at.push_back({&v, all.size()});
+    all.insert(all.end(), t.begin(), t.end());
+    all.resize((all.size() + 31) / 32 * 32, 0.0);  // each table on its own 256 bytes
+  };
+  add(op->B, B);
+  add(op->D, D);
+  add(op->eo, eo);
+  add(op->xq, xq);
+  add(op->wq, wq);
+  add(op->support, sup);
+  op->tables.upload(all.data(), all.size());
+  for (auto &[v, o] : at) v->ptr = op->tables.ptr + o;
 }
 
 // Metric terms of the lexicographic cell order: the stored array, or a

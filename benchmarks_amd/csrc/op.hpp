@@ -78,6 +78,13 @@ struct DBuf {
   }
 };
 
+// Part of a device buffer.
+template <typename T>
+struct DView {
+  T *ptr = nullptr;
+  size_t n = 0;
+};
+
 inline hipStream_t as_stream(void *s) { return reinterpret_cast<hipStream_t>(s); }
 
 // Process-wide creation count of operators.  Caches that belong to one
@@ -107,12 +114,15 @@ struct mfx_op {
   // a caller's map gathers constrained DoFs: their rows then receive the
   // cells' contributions, which vmult overwrites afterwards
   bool cons_in_map = false;
-  DBuf<double> G, B, D, xq, wq, support, cellX;
-  DBuf<float> G32, B32, D32, xq32, wq32;
-  // Gauss quadrature: the even-odd tables of B, B^T, D and D^T (eo_tab
-  // layout, in that order) for the line-form contractions
-  DBuf<double> eo;
-  DBuf<float> eo32;
+  DBuf<double> G, cellX;
+  DBuf<float> G32;
+  // the 1D tables, in one allocation and one upload.  eo: Gauss quadrature, the
+  // even-odd tables of B, B^T, D and D^T (eo_tab layout, in that order) for the
+  // line-form contractions
+  DBuf<double> tables;
+  DBuf<float> tables32;
+  DView<double> B, D, xq, wq, support, eo;
+  DView<float> B32, D32, xq32, wq32, eo32;
   // patch-of-cells kernels (box meshes, GLL collocation)
   bool patch = false;
   PatchLayout lay{};
