@@ -45,6 +45,24 @@ struct CollocTile {
   static constexpr bool PREFETCH = NQ <= 7;
 };
 
+// A metric term.  A row of nq^2 terms that does not end at a 128-byte line shares
+// its last line with the next row, which a wave reads later, so streaming it
+// past the caches fetches that line twice.  Short rows are therefore kept (the
+// default policy): vmult with stored terms, streamed -> kept, on 10M DoFs
+// p = 1, q = 2 1554 -> 994 us (FP32 1345 -> 649), p = 2, q = 3 638 -> 504 (404 -> 309),
+// p = 3, q = 5 610 -> 570 (391 -> 337), p = 4, q = 5 on 2M DoFs 77 -> 65 (51 -> 41).
+// Rows of whole lines are read once (FP64 q = 4 783 kept, 761 streamed), and of
+// long rows the shared line is too little to make up for what the stream
+// evicts (FP64 q = 6 441 kept, 427 streamed; q = 9 347, 328).
+template <typename T, int NQ>
+__device__ __forceinline__ T load_geo(const T *p) {
+  constexpr int kRow = NQ * NQ * sizeof(T);
+  if constexpr (kRow % 128 == 0 || kRow > 256)
+    return __builtin_nontemporal_load(p);
+  else
+    return *p;
+}
+
 __device__ __forceinline__ void atomic_add(double *p, double v) { unsafeAtomicAdd(p, v); }
 __device__ __forceinline__ void atomic_add(float *p, float v) { unsafeAtomicAdd(p, v); }
 
@@ -104,7 +122,7 @@ k_apply_colloc(const T *__restrict__ gD, const T *__restrict__ G,
 #pragma unroll
     for (int z = 0; z < NQ; ++z)
 #pragma unroll
-      for (int c = 0; c < 6; ++c) g[c][z] = __builtin_nontemporal_load(Ge + c * NQ3 + z * NQ2);
+      for (int c = 0; c < 6; ++c) g[c][z] = load_geo<T, NQ>(Ge + c * NQ3 + z * NQ2);
   }
 
   uint32_t idx[NQ];
@@ -135,12 +153,12 @@ k_apply_colloc(const T *__restrict__ gD, const T *__restrict__ G,
         gxx = g[0][z]; gxy = g[1][z]; gxz = g[2][z];
         gyy = g[3][z]; gyz = g[4][z]; gzz = g[5][z];
       } else {
-        gxx = __builtin_nontemporal_load(Ge + 0 * NQ3 + z * NQ2);
-        gxy = __builtin_nontemporal_load(Ge + 1 * NQ3 + z * NQ2);
-        gxz = __builtin_nontemporal_load(Ge + 2 * NQ3 + z * NQ2);
-        gyy = __builtin_nontemporal_load(Ge + 3 * NQ3 + z * NQ2);
-        gyz = __builtin_nontemporal_load(Ge + 4 * NQ3 + z * NQ2);
-        gzz = __builtin_nontemporal_load(Ge + 5 * NQ3 + z * NQ2);
+        gxx = load_geo<T, NQ>(Ge + 0 * NQ3 + z * NQ2);
+        gxy = load_geo<T, NQ>(Ge + 1 * NQ3 + z * NQ2);
+        gxz = load_geo<T, NQ>(Ge + 2 * NQ3 + z * NQ2);
+        gyy = load_geo<T, NQ>(Ge + 3 * NQ3 + z * NQ2);
+        gyz = load_geo<T, NQ>(Ge + 4 * NQ3 + z * NQ2);
+        gzz = load_geo<T, NQ>(Ge + 5 * NQ3 + z * NQ2);
       }
       T dx = 0, dy = 0, dz = 0;
 #pragma unroll
@@ -377,7 +395,7 @@ k_apply_interp(const T *__restrict__ gB, const T *__restrict__ gD,
 #pragma unroll
     for (int z = 0; z < NQ; ++z)
 #pragma unroll
-      for (int c = 0; c < 6; ++c) g[c][z] = __builtin_nontemporal_load(Ge + c * NQ3 + z * NQ2);
+      for (int c = 0; c < 6; ++c) g[c][z] = load_geo<T, NQ>(Ge + c * NQ3 + z * NQ2);
   }
   if constexpr (LINE) {
     // thread (qx, qy) interpolates the y-line x = qx, z = qy (< NM) into s0
@@ -536,12 +554,12 @@ k_apply_interp(const T *__restrict__ gB, const T *__restrict__ gD,
           gxx = g[0][z]; gxy = g[1][z]; gxz = g[2][z];
           gyy = g[3][z]; gyz = g[4][z]; gzz = g[5][z];
         } else {
-          gxx = __builtin_nontemporal_load(Ge + 0 * NQ3 + z * NQ2);
-          gxy = __builtin_nontemporal_load(Ge + 1 * NQ3 + z * NQ2);
-          gxz = __builtin_nontemporal_load(Ge + 2 * NQ3 + z * NQ2);
-          gyy = __builtin_nontemporal_load(Ge + 3 * NQ3 + z * NQ2);
-          gyz = __builtin_nontemporal_load(Ge + 4 * NQ3 + z * NQ2);
-          gzz = __builtin_nontemporal_load(Ge + 5 * NQ3 + z * NQ2);
+          gxx = load_geo<T, NQ>(Ge + 0 * NQ3 + z * NQ2);
+          gxy = load_geo<T, NQ>(Ge + 1 * NQ3 + z * NQ2);
+          gxz = load_geo<T, NQ>(Ge + 2 * NQ3 + z * NQ2);
+          gyy = load_geo<T, NQ>(Ge + 3 * NQ3 + z * NQ2);
+          gyz = load_geo<T, NQ>(Ge + 4 * NQ3 + z * NQ2);
+          gzz = load_geo<T, NQ>(Ge + 5 * NQ3 + z * NQ2);
         }
         const T fx = gxx * dx + gxy * dy + gxz * dz;
         const T fy = gxy * dx + gyy * dy + gyz * dz;
