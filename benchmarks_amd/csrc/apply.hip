@@ -131,7 +131,7 @@ k_apply_colloc(const T *__restrict__ gD, const T *__restrict__ G,
     if (GATHER) {
       const uint32_t *me = map + (size_t)e * NQ3 + col;
 #pragma unroll
-      for (int z = 0; z < NQ; ++z) idx[z] = __builtin_nontemporal_load(me + z * NQ2);
+      for (int z = 0; z < NQ; ++z) idx[z] = me[z * NQ2];
 #pragma unroll
       for (int z = 0; z < NQ; ++z) u[z] = (idx[z] != kInvalid) ? src[idx[z]] : T(0);
     } else {
@@ -214,7 +214,7 @@ k_apply_colloc(const T *__restrict__ gD, const T *__restrict__ G,
 // G = w det J J^-1 J^-T the stored form.  24 doubles per cell replace
 // 48 nq^3 bytes of G.
 //
-// ROW (box meshes, cells numbered x fastest, `row_cells` cells per x-row):
+// ROW (box meshes, cells and nodes numbered x fastest, boundary constrained; no map is read):
 // each workgroup takes up to EPB consecutive cells of one x-row.  The scatter
 // then first sums the cells' shared x-faces in LDS (the right face of cell
 // c and the left face of cell c+1, in that order) and adds each node of the
@@ -232,7 +232,7 @@ k_apply_interp(const T *__restrict__ gB, const T *__restrict__ gD,
                T *__restrict__ dst, const uint32_t *__restrict__ map,
                uint32_t n_cells, double *__restrict__ partials,
                const int *__restrict__ skip, const double *__restrict__ cellX,
-               const T *__restrict__ gxq, const T *__restrict__ gwq, uint32_t row_cells,
+               const T *__restrict__ gxq, const T *__restrict__ gwq, RowMesh rows,
                const T *__restrict__ geo) {
   constexpr int EPB = Tile<NQ>::EPB, NQ2 = NQ * NQ, NQ3 = NQ2 * NQ;
   static_assert(!AX || (OTF && ROW), "axis-aligned cells: a box-mesh form of the vertex metric");
@@ -255,10 +255,10 @@ k_apply_interp(const T *__restrict__ gB, const T *__restrict__ gD,
   // the workgroup's cells: e0 .. e0 + m - 1
   uint32_t e0, m;
   if constexpr (ROW) {
-    const uint32_t wpr = (row_cells + EPB - 1) / EPB;  // workgroups per x-row
+    const uint32_t wpr = (rows.n0 + EPB - 1) / EPB;  // workgroups per x-row
     const uint32_t row = blockIdx.x / wpr, xs = (blockIdx.x - row * wpr) * EPB;
-    e0 = row * row_cells + xs;
-    m = min((uint32_t)EPB, row_cells - xs);
+    e0 = row * rows.n0 + xs;
+    m = min((uint32_t)EPB, rows.n0 - xs);
   } else {
     e0 = blockIdx.x * EPB;
     m = min((uint32_t)EPB, n_cells - e0);
@@ -306,15 +306,39 @@ k_apply_interp(const T *__restrict__ gB, const T *__restrict__ gD,
     }
   }
 
+  // ROW: the segment's first node, the strides of the node grid, and which of its
+  // nodes are free: the boundary of the box is constrained
+  const uint32_t NX = rows.n0 * (NM - 1) + 1, NXY = NX * (rows.n1 * (NM - 1) + 1);
+  uint32_t base = 0, x_first = 0;
+  bool y0 = false, y1 = false, z0 = false, z1 = false;
+  if constexpr (ROW) {
+    const uint32_t row = e0 / rows.n0, ey = row % rows.n1, ez = row / rows.n1;
+    x_first = (NM - 1) * (e0 - row * rows.n0);
+    base = x_first + (NM - 1) * (ey * NX + ez * NXY);
+    y0 = ey == 0;
+    y1 = ey + 1 == rows.n1;
+    z0 = ez == 0;
+    z1 = ez + 1 == rows.n2;
+  }
+  auto row_free = [&](uint32_t X, int yn, int zn) {  // node X of the segment's row (yn, zn)
+    return !(x_first + X == 0 || x_first + X == NX - 1 || (y0 && yn == 0) || (y1 && yn == NM - 1) ||
+             (z0 && zn == 0) || (z1 && zn == NM - 1));
+  };
+
   // 1. gather the (x,y) node column
   uint32_t idx[NM];
   T uin[NM];
   if (node_col) {
     const int l0 = qy * NM + qx;
-    if (GATHER) {
+    if constexpr (ROW) {
+      const uint32_t X = el * (NM - 1) + qx;
+      const T *sc = src + base + X + qy * NX;
+#pragma unroll
+      for (int z = 0; z < NM; ++z) uin[z] = row_free(X, qy, z) ? sc[z * NXY] : T(0);
+    } else if (GATHER) {
       const uint32_t *me = map + (size_t)e * NM3 + l0;
 #pragma unroll
-      for (int z = 0; z < NM; ++z) idx[z] = __builtin_nontemporal_load(me + z * NM2);
+      for (int z = 0; z < NM; ++z) idx[z] = me[z * NM2];
 #pragma unroll
       for (int z = 0; z < NM; ++z) uin[z] = (idx[z] != kInvalid) ? src[idx[z]] : T(0);
     } else {
@@ -704,18 +728,15 @@ k_apply_interp(const T *__restrict__ gB, const T *__restrict__ gD,
   if constexpr (ROW) {
     __syncthreads();
     // node X of row r = zn NM + yn of the segment: its left-face value plus,
-    // on an inner face, the right face of the cell before it; the map entry
-    // of the cell that holds X as its left face or interior node (the last
-    // cell for the segment's end)
+    // on an inner face, the right face of the cell before it
     const int nx = (int)m * P + 1;
     for (int i = tid; i < NM * NM * nx; i += THREADS) {
       const int r = i / nx, X = i - r * nx;
       const int c = X / P;
       T v = acc[r * XW + X];
       if (X == c * P && c >= 1 && c < (int)m) v += rgt[r * EPB + c - 1];
-      const int co = min(c, (int)m - 1);
-      const uint32_t gi = map[(size_t)(e0 + co) * NM3 + r * NM + (X - co * P)];
-      if (gi != kInvalid) atomic_add(dst + gi, v);
+      const int zn = r / NM, yn = r - zn * NM;
+      if (row_free(X, yn, zn)) atomic_add(dst + base + X + yn * NX + zn * NXY, v);
     }
   }
   if (DOT) {
@@ -725,23 +746,22 @@ k_apply_interp(const T *__restrict__ gB, const T *__restrict__ gD,
 }
 
 // Workgroups of an apply: cells in batches of EPB, or (Gauss kernel on a box
-// mesh, row_cells > 0) EPB-cell segments of each x-row.
+// mesh) EPB-cell segments of each x-row.
 template <int NQ, bool COLLOC>
-uint32_t n_blocks_for(uint32_t n_cells, uint32_t row_cells = 0) {
+uint32_t n_blocks_for(uint32_t n_cells, RowMesh rows = {}) {
   constexpr int EPB = COLLOC ? CollocTile<NQ>::EPB : Tile<NQ>::EPB;
-  if (!COLLOC && row_cells)
-    return (n_cells / row_cells) * ((row_cells + EPB - 1) / EPB);
+  if (!COLLOC && rows.n0) return (n_cells / rows.n0) * ((rows.n0 + EPB - 1) / EPB);
   return (n_cells + EPB - 1) / EPB;
 }
 
 template <typename T, int NM, int NQ, bool COLLOC, bool GATHER>
 void launch_t(const T *B, const T *D, const T *G, const T *src, T *dst,
               const uint32_t *map, uint32_t n_cells, hipStream_t s,
-              double *partials, const int *skip, uint32_t row_cells) {
+              double *partials, const int *skip, RowMesh rows) {
   if (n_cells == 0) return;
-  const bool row = !COLLOC && GATHER && row_cells > 0;
-  MFX_REQUIRE(!row || n_cells % row_cells == 0, "row segments need whole x-rows of cells");
-  const dim3 grid(n_blocks_for<NQ, COLLOC>(n_cells, row ? row_cells : 0));
+  const bool row = !COLLOC && GATHER && rows.n0 > 0;
+  MFX_REQUIRE(!row || (uint64_t)rows.n0 * rows.n1 * rows.n2 == n_cells, "row segments: cells of another mesh");
+  const dim3 grid(n_blocks_for<NQ, COLLOC>(n_cells, row ? rows : RowMesh{}));
   if constexpr (COLLOC) {
     static_assert(NM == NQ, "collocation needs nm == nq");
     const dim3 block(CollocTile<NQ>::THREADS);
@@ -764,25 +784,25 @@ void launch_t(const T *B, const T *D, const T *G, const T *src, T *dst,
         if (row)
           hipLaunchKernelGGL((k_apply_interp<T, NM, NQ, GATHER, true, false, true>), grid, block,
                              0, s, B, D, G, src, dst, map, n_cells, partials, skip, nullptr,
-                             nullptr, nullptr, row_cells, (const T *)nullptr);
+                             nullptr, nullptr, rows, (const T *)nullptr);
         else
           hipLaunchKernelGGL((k_apply_interp<T, NM, NQ, GATHER, true>), grid, block, 0, s, B, D,
                              G, src, dst, map, n_cells, partials, skip, nullptr, nullptr, nullptr,
-                             0u, (const T *)nullptr);
+                             RowMesh{}, (const T *)nullptr);
       }
     } else {
       if constexpr (GATHER) {
         if (row) {
           hipLaunchKernelGGL((k_apply_interp<T, NM, NQ, GATHER, false, false, true>), grid,
                              block, 0, s, B, D, G, src, dst, map, n_cells, nullptr, nullptr,
-                             nullptr, nullptr, nullptr, row_cells, (const T *)nullptr);
+                             nullptr, nullptr, nullptr, rows, (const T *)nullptr);
           MFX_HIP(hipGetLastError());
           return;
         }
       }
       hipLaunchKernelGGL((k_apply_interp<T, NM, NQ, GATHER, false>), grid, block, 0, s,
                          B, D, G, src, dst, map, n_cells, nullptr, nullptr, nullptr, nullptr,
-                         nullptr, 0u, (const T *)nullptr);
+                         nullptr, RowMesh{}, (const T *)nullptr);
     }
   }
   MFX_HIP(hipGetLastError());
@@ -793,7 +813,7 @@ void launch_t(const T *B, const T *D, const T *G, const T *src, T *dst,
 template <typename T, bool GATHER>
 void dispatch(int p, int nq, bool colloc, const T *B, const T *D, const T *G,
               const T *src, T *dst, const uint32_t *map, uint32_t n,
-              hipStream_t s, double *partials, const int *skip, uint32_t rc) {
+              hipStream_t s, double *partials, const int *skip, RowMesh rc) {
 #define MFX_CASE_C(P)                                                         \
   case P:                                                                     \
     return launch_t<T, P + 1, P + 1, true, GATHER>(B, D, G, src, dst, map, n, s, partials, skip, rc);
@@ -886,14 +906,14 @@ void launch_colloc_variant(int p, int v, const double *D, const double *G, const
 template <typename T>
 void launch_apply(int p, int nq, bool colloc, const T *B, const T *D, const T *G,
                   const T *src, T *dst, const uint32_t *map, uint32_t n_cells,
-                  hipStream_t s, double *dot_partials, const int *skip, uint32_t row_cells) {
+                  hipStream_t s, double *dot_partials, const int *skip, RowMesh rows) {
   dispatch<T, true>(p, nq, colloc, B, D, G, src, dst, map, n_cells, s, dot_partials, skip,
-                    row_cells);
+                    rows);
 }
 template <typename T>
 void launch_evec(int p, int nq, bool colloc, const T *B, const T *D, const T *G,
                  const T *in, T *out, uint32_t n_cells, hipStream_t s) {
-  dispatch<T, false>(p, nq, colloc, B, D, G, in, out, nullptr, n_cells, s, nullptr, nullptr, 0u);
+  dispatch<T, false>(p, nq, colloc, B, D, G, in, out, nullptr, n_cells, s, nullptr, nullptr, RowMesh{});
 }
 
 // Gauss (non-collocated) apply with the metric terms computed from the cell
@@ -902,24 +922,25 @@ template <typename T, int NM, int NQ>
 void launch_interp_otf(const T *B, const T *D, const T *eo, const T *xq, const T *wq,
                        const double *cellX, const T *src, T *dst, const uint32_t *map,
                        uint32_t n_cells, hipStream_t s, double *partials, const int *skip,
-                       uint32_t row_cells, bool axes) {
-  MFX_REQUIRE(!axes || row_cells, "axis-aligned cells are a box-mesh form");
+                       RowMesh rows, bool axes) {
+  MFX_REQUIRE(!axes || rows.n0, "axis-aligned cells are a box-mesh form");
   if (n_cells == 0) return;
-  MFX_REQUIRE(!row_cells || n_cells % row_cells == 0, "row segments need whole x-rows of cells");
-  const dim3 grid(n_blocks_for<NQ, false>(n_cells, row_cells)), block(Tile<NQ>::THREADS);
+  MFX_REQUIRE(!rows.n0 || (uint64_t)rows.n0 * rows.n1 * rows.n2 == n_cells,
+              "row segments: cells of another mesh");
+  const dim3 grid(n_blocks_for<NQ, false>(n_cells, rows)), block(Tile<NQ>::THREADS);
   if (partials) {
     if constexpr (std::is_same<T, double>::value) {
       if (axes)
         hipLaunchKernelGGL((k_apply_interp<T, NM, NQ, true, true, true, true, true>), grid, block,
                            0, s, B, D, nullptr, src, dst, map, n_cells, partials, skip, cellX, xq,
-                           wq, row_cells, eo);
-      else if (row_cells)
+                           wq, rows, eo);
+      else if (rows.n0)
         hipLaunchKernelGGL((k_apply_interp<T, NM, NQ, true, true, true, true>), grid, block, 0, s,
                            B, D, nullptr, src, dst, map, n_cells, partials, skip, cellX, xq, wq,
-                           row_cells, eo);
+                           rows, eo);
       else
         hipLaunchKernelGGL((k_apply_interp<T, NM, NQ, true, true, true>), grid, block, 0, s, B, D,
-                           nullptr, src, dst, map, n_cells, partials, skip, cellX, xq, wq, 0u,
+                           nullptr, src, dst, map, n_cells, partials, skip, cellX, xq, wq, RowMesh{},
                            eo);
     } else {
       throw Error{MFX_ERR_UNSUPPORTED, "p.Ap partials are computed in FP64 only"};
@@ -927,14 +948,14 @@ void launch_interp_otf(const T *B, const T *D, const T *eo, const T *xq, const T
   } else if (axes) {
     hipLaunchKernelGGL((k_apply_interp<T, NM, NQ, true, false, true, true, true>), grid, block, 0,
                        s, B, D, nullptr, src, dst, map, n_cells, nullptr, nullptr, cellX, xq, wq,
-                       row_cells, eo);
-  } else if (row_cells) {
+                       rows, eo);
+  } else if (rows.n0) {
     hipLaunchKernelGGL((k_apply_interp<T, NM, NQ, true, false, true, true>), grid, block, 0, s, B,
                        D, nullptr, src, dst, map, n_cells, nullptr, nullptr, cellX, xq, wq,
-                       row_cells, eo);
+                       rows, eo);
   } else {
     hipLaunchKernelGGL((k_apply_interp<T, NM, NQ, true, false, true>), grid, block, 0, s, B, D,
-                       nullptr, src, dst, map, n_cells, nullptr, nullptr, cellX, xq, wq, 0u,
+                       nullptr, src, dst, map, n_cells, nullptr, nullptr, cellX, xq, wq, RowMesh{},
                        eo);
   }
   MFX_HIP(hipGetLastError());
@@ -944,16 +965,16 @@ template <typename T>
 void launch_apply_otf(int p, int nq, const T *B, const T *D, const T *eo, const T *xq,
                       const T *wq, const double *cellX, const T *src, T *dst,
                       const uint32_t *map, uint32_t n_cells, hipStream_t s, double *partials,
-                      const int *skip, uint32_t row_cells, bool axes) {
+                      const int *skip, RowMesh rows, bool axes) {
   MFX_REQUIRE(B && D && eo && xq && wq && cellX, "on-the-fly apply: missing tables or vertices");
 #define MFX_CASE_O(P)                                                                         \
   case P:                                                                                    \
     if (nq == P + 1)                                                                         \
       return launch_interp_otf<T, P + 1, P + 1>(B, D, eo, xq, wq, cellX, src, dst, map,      \
-                                                n_cells, s, partials, skip, row_cells, axes); \
+                                                n_cells, s, partials, skip, rows, axes); \
     if (nq == P + 2)                                                                         \
       return launch_interp_otf<T, P + 1, P + 2>(B, D, eo, xq, wq, cellX, src, dst, map,      \
-                                                n_cells, s, partials, skip, row_cells, axes); \
+                                                n_cells, s, partials, skip, rows, axes); \
     break;
   switch (p) {
     MFX_CASE_O(1) MFX_CASE_O(2) MFX_CASE_O(3) MFX_CASE_O(4)
@@ -968,29 +989,29 @@ void launch_apply_otf(int p, int nq, const T *B, const T *D, const T *eo, const 
 template void launch_apply_otf<double>(int, int, const double *, const double *, const double *,
                                        const double *, const double *, const double *,
                                        const double *, double *, const uint32_t *, uint32_t,
-                                       hipStream_t, double *, const int *, uint32_t, bool);
+                                       hipStream_t, double *, const int *, RowMesh, bool);
 template void launch_apply_otf<float>(int, int, const float *, const float *, const float *,
                                       const float *, const float *, const double *, const float *,
                                       float *, const uint32_t *, uint32_t, hipStream_t, double *,
-                                      const int *, uint32_t, bool);
+                                      const int *, RowMesh, bool);
 
 template void launch_apply<double>(int, int, bool, const double *, const double *,
                                    const double *, const double *, double *,
                                    const uint32_t *, uint32_t, hipStream_t, double *,
-                                   const int *, uint32_t);
+                                   const int *, RowMesh);
 template void launch_apply<float>(int, int, bool, const float *, const float *,
                                   const float *, const float *, float *,
                                   const uint32_t *, uint32_t, hipStream_t, double *,
-                                  const int *, uint32_t);
+                                  const int *, RowMesh);
 template void launch_evec<double>(int, int, bool, const double *, const double *,
                                   const double *, const double *, double *, uint32_t,
                                   hipStream_t);
 
-uint32_t apply_n_blocks(int p, int nq, bool colloc, uint32_t n_cells, uint32_t row_cells) {
+uint32_t apply_n_blocks(int p, int nq, bool colloc, uint32_t n_cells, RowMesh rows) {
   (void)p;
 #define MFX_NB(Q)                                                                    \
   case Q:                                                                           \
-    return colloc ? n_blocks_for<Q, true>(n_cells) : n_blocks_for<Q, false>(n_cells, row_cells);
+    return colloc ? n_blocks_for<Q, true>(n_cells) : n_blocks_for<Q, false>(n_cells, rows);
   switch (nq) {
     MFX_NB(2) MFX_NB(3) MFX_NB(4) MFX_NB(5) MFX_NB(6) MFX_NB(7) MFX_NB(8) MFX_NB(9) MFX_NB(10)
     default: return 0;

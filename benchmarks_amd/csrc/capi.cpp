@@ -19,28 +19,36 @@ void set_error(const std::string &msg) { g_last_error = msg; }
 using namespace mfx;
 
 // Whether a box operator with the metric from the vertices runs the plane kernel
-// (plane_kernel.hpp) rather than the patch kernel or the per-column Gauss
-// kernel.  A wave of the plane kernel holds 64 / q cells and works a layer of
-// them off alone, so it needs a device full of waves (groups x layers) to
-// come ahead, the more the longer a layer takes (points, trilinear metric) and
-// the better the other kernel shares its work.  Below the lines the other
-// kernel is level to 2x faster (q >= 6 on a few thousand cells), above them
-// this one is: on 16M DoFs 1.0-2.1x (Gauss-Lobatto) and 1.1-3.0x (Gauss) in
-// FP64, 1.4-3.1x and 1.2-2.3x in FP32.  It has no instance where the planes do
-// not fit the registers (FP64 q >= 8, FP32 q >= 9).
+// (plane_kernel.hpp) rather than the patch kernel (Gauss-Lobatto) or the
+// per-column Gauss kernel.  A wave of the plane kernel holds 64 / q cells and works
+// a layer of them off alone, so it needs a device full of waves (groups x
+// layers) to come ahead, the more the longer a layer takes (points, trilinear
+// metric) and the better the other kernel shares its work.  Below the lines the
+// other kernel is level to 2x faster (q >= 6 on a few thousand cells), above them
+// this one is: at the lines 1.0-1.2x, on 16-20M DoFs 1.0-2.1x (Gauss-Lobatto) and
+// 1.0-3.1x (Gauss) in FP64, 1.4-3.1x and 1.0-2.5x in FP32.  The Gauss kernel with
+// the trilinear metric holds out longest where its cells fill the lanes best:
+// FP64 p = 4, q = 6 is level at any size, FP32 p = 4, q = 5 3% ahead up to 20M DoFs.
+// There is no instance where the planes do not fit the registers (FP64 q >= 8,
+// FP32 q >= 9).
 static bool plane_rule(const mfx_op &op, bool fp32) {
   if (fp32 ? !plane_instance<float>(op.p, op.nq, op.colloc)
            : !plane_instance<double>(op.p, op.nq, op.colloc))
     return false;
   const bool axes = op.box.deform == 0.0;
   const int q = op.nq;
+  const bool over = q == op.p + 2;  // more points than the stiffness of affine cells needs
   uint64_t need;
-  if (fp32)
-    need = axes || op.colloc ? 1024 : q <= 4 ? 2048 : 4096;
+  if (op.colloc)
+    need = fp32   ? 1024
+           : axes ? (q >= 6 ? 4096 : 2048)
+                  : (q <= 3 ? 2048 : q <= 5 ? 4096 : 8192);
   else if (axes)
-    need = op.colloc && q >= 6 ? 4096 : 2048;
+    need = fp32 ? (q <= 5 ? 1536 : over ? 4096 : 2048) : (q <= 5 ? 1024 : q == 6 ? 2048 : 5120);
+  else if (fp32)
+    need = q <= 3 ? 1024 : q == 4 ? 4096 : q == 5 ? (over ? 12288 : ~0ull) : over && q >= 7 ? 8192 : 6144;
   else
-    need = q <= 3 ? 2048 : q <= 5 ? (op.colloc ? 4096 : 2048) : 8192;
+    need = q <= 4 ? 1024 : q == 5 ? (over ? 1024 : 6144) : q == 6 ? 16384 : 8192;
   return (uint64_t)op.plane_lay.groups * op.plane_lay.n[2] >= need;
 }
 

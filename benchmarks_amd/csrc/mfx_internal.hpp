@@ -33,29 +33,34 @@ struct Error {
 
 constexpr uint32_t kInvalid = MFX_INVALID_DOF;
 
+// Cells per direction of a box mesh whose cells and nodes are numbered x fastest
+// and whose boundary nodes are constrained; n0 = 0: any other mesh.
+struct RowMesh {
+  uint32_t n0 = 0, n1 = 0, n2 = 0;
+};
+
 // Launch wrappers implemented in the .hip translation units.  Each checks
 // its arguments against what the kernel assumes and throws mfx::Error.
 template <typename T>
 void launch_apply(int p, int nq, bool collocation, const T *B, const T *D,
                   const T *G, const T *src, T *dst, const uint32_t *map,
                   uint32_t n_cells, hipStream_t s, double *dot_partials = nullptr,
-                  const int *skip = nullptr, uint32_t row_cells = 0);
+                  const int *skip = nullptr, RowMesh rows = {});
 // Non-collocated (Gauss) apply with the metric terms of the trilinear cells
 // computed per quadrature point from their vertices (cellX [E][8][3]), xq and
-// wq the 1D quadrature points and weights on [0,1].  row_cells > 0 (both
-// Gauss applies): the cells form x-rows of row_cells cells numbered x
-// fastest, and the map gives neighbours along x their shared face nodes (a
-// box mesh); the scatter then sums shared x-faces in LDS first.
+// wq the 1D quadrature points and weights on [0,1].  rows (both Gauss applies):
+// the cells are those of a box mesh; the kernel then computes the DoFs itself
+// (the map is not read) and the scatter sums shared x-faces in LDS first.
 // eo: the even-odd tables of B, B^T, D, D^T (tables.hpp eo_tables) for the
 // line-form contractions.
 // axes: the cells are those of an undeformed box (Jacobian columns along x,
-// y and z; row_cells > 0), whose diagonal metric is formed once per column.
+// y and z; on a box mesh), whose diagonal metric is formed once per column.
 template <typename T>
 void launch_apply_otf(int p, int nq, const T *B, const T *D, const T *eo, const T *xq,
                       const T *wq, const double *cellX, const T *src, T *dst,
                       const uint32_t *map, uint32_t n_cells, hipStream_t s,
                       double *dot_partials = nullptr, const int *skip = nullptr,
-                      uint32_t row_cells = 0, bool axes = false);
+                      RowMesh rows = {}, bool axes = false);
 template <typename T>
 void launch_evec(int p, int nq, bool collocation, const T *B, const T *D,
                  const T *G, const T *in, T *out, uint32_t n_cells,
@@ -73,7 +78,7 @@ void launch_colloc_variant(int p, int v, const double *D, const double *G, const
                            int *epb = nullptr, int *prefetch = nullptr);
 // number of partial sums written by launch_apply(..., dot_partials)
 uint32_t apply_n_blocks(int p, int nq, bool collocation, uint32_t n_cells,
-                        uint32_t row_cells = 0);
+                        RowMesh rows = {});
 
 // set-up kernels (setup.hip)
 struct BoxGeom {

@@ -176,9 +176,10 @@ struct mfx_op {
     o.pbuf = det ? pbuf32.ptr : nullptr;
     return o;
   }
-  // Gauss applies on a box: x-rows of cells (their shared faces are summed
-  // before the scatter); 0 for other meshes and collocation
-  uint32_t row_cells() const { return is_box && !colloc ? box.n[0] : 0; }
+  // Gauss applies on a box: its cells per direction
+  RowMesh rows() const {
+    return is_box && !colloc ? RowMesh{box.n[0], box.n[1], box.n[2]} : RowMesh{};
+  }
   // an undeformed box: every cell's Jacobian columns lie along x, y and z
   bool axis_cells() const { return is_box && !colloc && box.deform == 0.0; }
   // Box operators with the metric from the vertices run the plane kernel where
@@ -207,7 +208,7 @@ struct mfx_op {
   uint32_t apply_blocks() const {
     if (plane<double>()) return plane_lay.blocks();
     return patch ? (det ? grid64.det_dot : grid64.dot)
-                 : apply_n_blocks(p, nq, colloc, E, row_cells());
+                 : apply_n_blocks(p, nq, colloc, E, rows());
   }
   // dst += A_free src (no zeroing, no constrained rows).  fresh: dst is zero on
   // the free rows (the start of an apply), which every caller but vmult_add
@@ -220,10 +221,10 @@ struct mfx_op {
       launch_patch<double>(patch_op64(), src, dst, s, partials, skip);
     else if (geometry == MFX_GEOM_ON_THE_FLY)
       launch_apply_otf<double>(p, nq, B.ptr, D.ptr, eo.ptr, xq.ptr, wq.ptr, cellX.ptr, src, dst,
-                               map.ptr, E, s, partials, skip, row_cells(), axis_cells());
+                               map.ptr, E, s, partials, skip, rows(), axis_cells());
     else
       launch_apply<double>(p, nq, colloc, B.ptr, D.ptr, G.ptr, src, dst, map.ptr, E, s, partials,
-                           skip, row_cells());
+                           skip, rows());
   }
   void apply32(const float *src, float *dst, hipStream_t s) const {
     if (plane<float>())
@@ -232,11 +233,11 @@ struct mfx_op {
       launch_patch<float>(patch_op32(), src, dst, s);
     else if (geometry == MFX_GEOM_ON_THE_FLY)
       launch_apply_otf<float>(p, nq, B32.ptr, D32.ptr, eo32.ptr, xq32.ptr, wq32.ptr, cellX.ptr,
-                              src, dst, map.ptr, E, s, nullptr, nullptr, row_cells(),
+                              src, dst, map.ptr, E, s, nullptr, nullptr, rows(),
                               axis_cells());
     else
       launch_apply<float>(p, nq, colloc, B32.ptr, D32.ptr, G32.ptr, src, dst, map.ptr, E, s,
-                          nullptr, nullptr, row_cells());
+                          nullptr, nullptr, rows());
   }
   // dst = A src with identity on the constrained rows
   void vmult64(const double *src, double *dst, hipStream_t s) const {
