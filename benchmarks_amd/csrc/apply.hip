@@ -38,11 +38,14 @@ struct Tile {
   static constexpr int EPB = (256 / (NQ * NQ)) > 0 ? 256 / (NQ * NQ) : 1;
   static constexpr int THREADS = EPB * NQ * NQ;
 };
+// Without the prefetch of G (its registers) nq = 6 and 7 run 112 and 104 us instead of
+// 134 and 126 on 4M DoFs, nq = 6 with 7 cells (3 with the prefetch); nq = 5 is faster
+// with it, 5 cells (142, 174 without) and 10 cells 173.
 template <int NQ>
 struct CollocTile {
-  static constexpr int EPB = NQ <= 6 ? 128 / (NQ * NQ) : (NQ == 7 ? 1 : (NQ == 8 ? 2 : 3));
+  static constexpr int EPB = NQ <= 5 ? 128 / (NQ * NQ) : NQ == 6 ? 7 : NQ == 7 ? 1 : NQ == 8 ? 2 : 3;
   static constexpr int THREADS = EPB * NQ * NQ;
-  static constexpr bool PREFETCH = NQ <= 7;
+  static constexpr bool PREFETCH = NQ <= 5;
 };
 
 // A metric term.  A row of nq^2 terms that does not end at a 128-byte line shares
@@ -103,6 +106,10 @@ k_apply_colloc(const T *__restrict__ gD, const T *__restrict__ G,
   __shared__ T sfx[EPB][NQ3];
   __shared__ T sfy[EPB][NQ3];
   __shared__ double red[(THREADS + 63) / 64];
+  // the DoFs of the cells' left and right x faces (see k_apply_interp's JOIN; at
+  // nq = 5 its registers beside the prefetched G cost more: 68 -> 72 us)
+  constexpr bool JOIN = GATHER && EPB > 2 && !(PREF && NQ >= 5);
+  __shared__ uint32_t sL[JOIN ? EPB * NQ2 : 1], sR[JOIN ? EPB * NQ2 : 1];
 
   if (skip && *skip) return;  // converged CG: nothing left to do
   const int tid = threadIdx.x;
@@ -142,6 +149,13 @@ k_apply_colloc(const T *__restrict__ gD, const T *__restrict__ G,
 #pragma unroll
     for (int z = 0; z < NQ; ++z) su[el][z * NQ2 + col] = u[z];
   }
+  if constexpr (JOIN) {  // (cells left out give no DoF)
+#pragma unroll
+    for (int z = 0; z < NQ; ++z) {
+      if (qx == 0) sL[el * NQ2 + z * NQ + qy] = active ? idx[z] : kInvalid;
+      if (qx == NQ - 1) sR[el * NQ2 + z * NQ + qy] = active ? idx[z] : kInvalid;
+    }
+  }
   __syncthreads();
 
   T fz[NQ];
@@ -175,6 +189,11 @@ k_apply_colloc(const T *__restrict__ gD, const T *__restrict__ G,
   __syncthreads();
 
   double dot = 0.0;
+  T vj[JOIN ? NQ : 1];
+  T *lft = &su[0][0];  // [cell][z][y]: left faces that the cell before adds
+  auto joined = [&](int z) {
+    return qx == 0 && el > 0 && sR[(el - 1) * NQ2 + z * NQ + qy] == idx[z];
+  };
   if (active) {
 #pragma unroll
     for (int z = 0; z < NQ; ++z) {
@@ -186,10 +205,26 @@ k_apply_colloc(const T *__restrict__ gD, const T *__restrict__ G,
         v += sD[a * NQ + z] * fz[a];
       }
       if (DOT) dot += (double)u[z] * (double)v;
-      if (GATHER) {
+      if constexpr (JOIN) {
+        vj[z] = v;
+        if (joined(z)) lft[el * NQ2 + z * NQ + qy] = v;
+      } else if (GATHER) {
         if (idx[z] != kInvalid) atomic_add(dst + idx[z], v);
       } else {
         dst[(size_t)e * NQ3 + z * NQ2 + col] = v;
+      }
+    }
+  }
+  if constexpr (JOIN) {
+    __syncthreads();
+    if (active) {
+#pragma unroll
+      for (int z = 0; z < NQ; ++z) {
+        if (idx[z] == kInvalid || joined(z)) continue;
+        T v = vj[z];
+        if (qx == NQ - 1 && el + 1 < EPB && sL[(el + 1) * NQ2 + z * NQ + qy] == idx[z])
+          v += lft[(el + 1) * NQ2 + z * NQ + qy];
+        atomic_add(dst + idx[z], v);
       }
     }
   }
@@ -246,6 +281,16 @@ k_apply_interp(const T *__restrict__ gB, const T *__restrict__ gD,
   __shared__ T sXv[OTF ? EPB * 24 : 1];  // cell vertices, then
   __shared__ T sKc[OTF ? EPB * 21 : 1];  // per cell 7 Jacobian coefficient vectors
   __shared__ double red[(Tile<NQ>::THREADS + 63) / 64];
+  // JOIN (a DoF map, any mesh): the DoFs of the cells' left and right x faces.  A
+  // face node that the map gives to both of two consecutive cells is added once,
+  // with the first cell's column: in an adapter's numbering a cell's left face lies
+  // strided in its neighbour's DoFs, a request per node or two.  On 1.75M DoFs,
+  // Gauss: p = 2, q = 3 143 -> 94 us, p = 4, q = 6 107 -> 91; p = 1 collocated
+  // 257 -> 143.  Not
+  // where the node columns are under half of the lanes (p = 1, q = 3: 374 -> 453 us
+  // with the metric from the vertices) or with few cells (q = 9 64 -> 66, q = 10 78 -> 84).
+  constexpr bool JOIN = GATHER && !ROW && EPB > 3 && 2 * NM2 >= NQ2;
+  __shared__ uint32_t sL[JOIN ? EPB * NM2 : 1], sR[JOIN ? EPB * NM2 : 1];
 
   if (skip && *skip) return;  // converged CG: nothing left to do
   const int tid = threadIdx.x;
@@ -341,6 +386,13 @@ k_apply_interp(const T *__restrict__ gB, const T *__restrict__ gD,
       for (int z = 0; z < NM; ++z) idx[z] = me[z * NM2];
 #pragma unroll
       for (int z = 0; z < NM; ++z) uin[z] = (idx[z] != kInvalid) ? src[idx[z]] : T(0);
+      if constexpr (JOIN) {
+#pragma unroll
+        for (int z = 0; z < NM; ++z) {
+          if (qx == 0) sL[el * NM2 + z * NM + qy] = idx[z];
+          if (qx == NM - 1) sR[el * NM2 + z * NM + qy] = idx[z];
+        }
+      }
     } else {
       const T *se = src + (size_t)e * NM3 + l0;
 #pragma unroll
@@ -685,6 +737,13 @@ k_apply_interp(const T *__restrict__ gB, const T *__restrict__ gD,
   constexpr int P = NM - 1, XW = EPB * P + 1;  // ROW: nodes of a full segment row
   T *acc = &s1[0][0];  // ROW: [zn][yn][X], X = c P + xn, the left faces
   T *rgt = &s2[0][0];  // ROW: [zn][yn][c], right faces of all but the last cell
+  T *lft = &s2[0][0];  // JOIN: [c][zn][yn], left faces that the cell before adds
+  static_assert(!JOIN || NM * NM <= NQ3, "left faces do not fit s2");
+  T vj[JOIN ? NM : 1];  // JOIN: the column's sums
+  // JOIN: node zn of this column is the right face node of the cell before
+  auto joined = [&](int zn) {
+    return qx == 0 && el > 0 && sR[(el - 1) * NM2 + zn * NM + qy] == idx[zn];
+  };
   static_assert(!ROW || NM * NM * XW <= EPB * NQ3, "row segment does not fit s1");
   static_assert(!ROW || NM * NM * EPB <= EPB * NQ3, "right faces do not fit s2");
   if constexpr (LINE && ROW) {
@@ -718,10 +777,28 @@ k_apply_interp(const T *__restrict__ gB, const T *__restrict__ gD,
           acc[(zn * NM + qy) * XW + el * P + qx] = v;
         else
           rgt[(zn * NM + qy) * EPB + el] = v;
+      } else if constexpr (JOIN) {
+        vj[zn] = v;
+        if (joined(zn)) lft[el * NM2 + zn * NM + qy] = v;
       } else if (GATHER) {
         if (idx[zn] != kInvalid) atomic_add(dst + idx[zn], v);
       } else {
         dst[(size_t)e * NM3 + zn * NM2 + qy * NM + qx] = v;
+      }
+    }
+  }
+  if constexpr (JOIN) {
+    // a face node that the map gives to two consecutive cells goes out with the
+    // first one's column
+    __syncthreads();
+    if (node_col) {
+#pragma unroll
+      for (int zn = 0; zn < NM; ++zn) {
+        if (idx[zn] == kInvalid || joined(zn)) continue;
+        T v = vj[zn];
+        if (qx == NM - 1 && (uint32_t)el + 1 < m && sL[(el + 1) * NM2 + zn * NM + qy] == idx[zn])
+          v += lft[(el + 1) * NM2 + zn * NM + qy];
+        atomic_add(dst + idx[zn], v);
       }
     }
   }
