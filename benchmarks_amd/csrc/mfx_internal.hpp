@@ -136,6 +136,8 @@ struct SineModes {
 void launch_sine_modes(const double *xyz, uint64_t n, const SineModes &m, double *out,
                        hipStream_t s);
 // deterministic two-stage dot: partials[nb] then final sum into *result
+// *result = the sum of n partial sums, in a fixed order
+void launch_sum(const double *part, uint32_t n, double *result, hipStream_t s);
 uint32_t dot_n_blocks(uint64_t n);
 void launch_dot(const double *x, const double *y, uint64_t n, double *partials,
                 double *result, hipStream_t s);

@@ -598,27 +598,48 @@ mfx_status mfx_mg_solve(mfx_mg *mg, double *x, const double *b, int max_steps, d
     bool converged = res_norm <= tol;
     bool breakdown = false;
     if (!converged && max_steps > 0) {
-      mg->precondition(mg->z.ptr, mg->r.ptr, s);
-      MFX_HIP(hipMemcpyAsync(mg->p.ptr, mg->z.ptr, N * sizeof(double), hipMemcpyDeviceToDevice, s));
-      double gamma = dot(mg->r.ptr, mg->z.ptr, N, mg->part, s);
+      // each scalar is the sum of its passes' partials, read back
+      // (p.Ap from the apply's partials where one workgroup sums them quickly; the
+      // cell-wise Gauss apply writes 3e5 at 135M rows)
+      const uint32_t nv = pcg_blocks(N);
+      const bool fused = A.apply_blocks() <= 8192;
+      const uint32_t na = fused ? A.apply_blocks() : 0;
+      const size_t need = std::max<size_t>((size_t)na + nv, dot_n_blocks(N)) + 1;
+      if (mg->part.n < need) mg->part.alloc(need);
+      double *part = mg->part.ptr;
+      auto sum = [&](uint32_t n) {
+        double h = 0.0;
+        launch_sum(part, n, part + n, s);
+        MFX_HIP(hipMemcpyAsync(&h, part + n, sizeof(double), hipMemcpyDeviceToHost, s));
+        MFX_HIP(hipStreamSynchronize(s));
+        return h;
+      };
+      mfx_mg::Level &L = mg->lv[0];
+      const uint32_t *mask = A.cmask.ptr;
+      launch_to_float_free(mg->r.ptr, L.b.ptr, mask, N, s);
+      mg->vcycle(0, s);
+      launch_to_double_free(L.x.ptr, mg->r.ptr, mg->z.ptr, mask, N, s, part);
+      double gamma = sum(nv), beta = 0.0;
       while (steps < max_steps) {
-        vmult64(A, mg->ap.ptr, mg->p.ptr, s);
-        const double pap = dot(mg->p.ptr, mg->ap.ptr, N, mg->part, s);
+        launch_pcg_direction_start(mg->p.ptr, mg->z.ptr, beta, mg->ap.ptr, mask, N, part + na, s);
+        A.apply64(mg->p.ptr, mg->ap.ptr, s, fused ? part : nullptr);
+        const double pap = fused ? sum(na + nv) : dot(mg->p.ptr, mg->ap.ptr, N, mg->part, s);
         if (!(pap > 0.0) || !(gamma > 0.0)) {
           breakdown = true;
           break;
         }
-        const double alpha = gamma / pap;
-        launch_pcg_update(x, mg->r.ptr, mg->p.ptr, mg->ap.ptr, alpha, N, s);
+        launch_pcg_update_fused(x, mg->r.ptr, mg->p.ptr, mg->ap.ptr, gamma / pap, L.b.ptr, mask, N,
+                                part, s);
         ++steps;
-        res_norm = std::sqrt(dot(mg->r.ptr, mg->r.ptr, N, mg->part, s));
+        res_norm = std::sqrt(sum(nv));
         if (res_norm <= tol) {
           converged = true;
           break;
         }
-        mg->precondition(mg->z.ptr, mg->r.ptr, s);
-        const double gn = dot(mg->r.ptr, mg->z.ptr, N, mg->part, s);
-        launch_pcg_direction(mg->p.ptr, mg->z.ptr, gn / gamma, N, s);
+        mg->vcycle(0, s);
+        launch_to_double_free(L.x.ptr, mg->r.ptr, mg->z.ptr, mask, N, s, part);
+        const double gn = sum(nv);
+        beta = gn / gamma;
         gamma = gn;
       }
     }

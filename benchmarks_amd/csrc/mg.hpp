@@ -87,8 +87,19 @@ void launch_cheb_step(float *x, float *d, const float *b, float *t, const float 
 // b = r, 0 on the rows of the bitmask; z = x, r on the rows of the bitmask
 void launch_to_float_free(const double *r, float *b, const uint32_t *mask, uint64_t n,
                           hipStream_t s);
+// (part, optional: pcg_blocks(n) partial sums of r z)
 void launch_to_double_free(const float *x, const double *r, double *z, const uint32_t *mask,
-                           uint64_t n, hipStream_t s);
+                           uint64_t n, hipStream_t s, double *part = nullptr);
+// x += alpha p, r -= alpha ap, b = r on the free rows and 0 on the masked ones;
+// pcg_blocks(n) partial sums of r r
+void launch_pcg_update_fused(double *x, double *r, const double *p, const double *ap, double alpha,
+                             float *b, const uint32_t *mask, uint64_t n, double *part,
+                             hipStream_t s);
+// p = z + beta p; ap = p on the masked rows and 0 elsewhere (the start of A p);
+// pcg_blocks(n) partial sums of p p over the masked rows
+void launch_pcg_direction_start(double *p, const double *z, double beta, double *ap,
+                                const uint32_t *mask, uint64_t n, double *part, hipStream_t s);
+uint32_t pcg_blocks(uint64_t n);
 // r = b - t
 void launch_residual_f32(float *r, const float *b, const float *t, uint64_t n, hipStream_t s);
 void launch_to_double(const float *in, double *out, uint64_t n, hipStream_t s);

@@ -645,6 +645,11 @@ void launch_dot(const double *x, const double *y, uint64_t n, double *partials, 
   MFX_HIP(hipGetLastError());
 }
 
+void launch_sum(const double *part, uint32_t n, double *result, hipStream_t s) {
+  hipLaunchKernelGGL(k_dot_final, dim3(1), dim3(kBlock), 0, s, part, n, result);
+  MFX_HIP(hipGetLastError());
+}
+
 // ---- CG launchers ----
 uint32_t cg_vec_blocks(uint64_t n) { return vec_grid(n); }
 uint32_t cg_cons_blocks(uint64_t nc) { return nc ? std::min<uint32_t>(vec_grid(nc), 256) : 0; }
