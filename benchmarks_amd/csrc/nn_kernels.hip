@@ -488,8 +488,18 @@ struct WgradArgs {
 // 2-byte and 4-byte loads: 38 us for all eight layers on a 33^3 grid, against
 // 430 us in one launch per layer with one tap per workgroup, the loads of each
 // tap by themselves and a 64-bit index division per point.
+//
+// The FP32 sums are taken in blocks of kSumChunks chunks, then over the blocks:
+// on large grids a unit has hundreds of chunks, and one chain over all of them
+// would round that often (257 x 129 x 129 nodes: 1044 chunks, 16 + 66 roundings
+// instead).  The sums over the blocks wait in the LDS: in registers they cost the
+// fourth wave per SIMD (33^3 grid 201 -> 205 us, 129^3 3781 -> 3927).
+constexpr uint32_t kSumChunks = 16;
+constexpr int kWgradSums = 24;  // of a lane: 3 taps x 2 channel tiles x 4
 template <int CIN, int COUT, int STRIDE, bool UP, int CTW>
-__device__ __forceinline__ void wgrad_mfma(const WgradLayer &L, uint32_t unit) {
+__device__ __forceinline__ void wgrad_mfma(const WgradLayer &L, uint32_t unit,
+                                           float (*blocks)[kBlock]) {
+  static_assert(3 * CTW * 4 <= kWgradSums, "block sums");
   static_assert(CIN % (16 * CTW) == 0 && COUT % 16 == 0, "channel tiles");
   static_assert(UP == (STRIDE == 1), "the stride-1 layers read an up-sampled input");
   constexpr int OT = COUT / 16, CG = CIN / 16 / CTW;
@@ -510,6 +520,18 @@ __device__ __forceinline__ void wgrad_mfma(const WgradLayer &L, uint32_t unit) {
 #pragma unroll
     for (int b = 0; b < CTW; ++b) acc[t][b] = v4f{0.f, 0.f, 0.f, 0.f};
   for (uint32_t k = k0; k < k1; ++k) {
+    if (k > k0 && (k - k0) % kSumChunks == 0) {
+#pragma unroll
+      for (int t = 0; t < 3; ++t)
+#pragma unroll
+        for (int b = 0; b < CTW; ++b)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            float &s = blocks[(t * CTW + b) * 4 + r][threadIdx.x];
+            s = k - k0 == kSumChunks ? acc[t][b][r] : s + acc[t][b][r];
+            acc[t][b][r] = 0.f;
+          }
+    }
     const uint32_t p0 = k * 32 + 8 * g;
     int x, y, z;
     decode(p0 < P ? p0 : 0, L.od, x, y, z);
@@ -586,7 +608,9 @@ __device__ __forceinline__ void wgrad_mfma(const WgradLayer &L, uint32_t unit) {
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const int o = ot * 16 + 4 * g + r, c = (cg * CTW + b) * 16 + li;
-        L.part[(((uint64_t)pi * COUT + o) * 27 + zy * 3 + t) * CIN + c] = acc[t][b][r];
+        float v = acc[t][b][r];
+        if (k1 - k0 > kSumChunks) v += blocks[(t * CTW + b) * 4 + r][threadIdx.x];
+        L.part[(((uint64_t)pi * COUT + o) * 27 + zy * 3 + t) * CIN + c] = v;
       }
 }
 
@@ -646,16 +670,17 @@ constexpr int kWgradOrder[8] = {6, 5, 1, 4, 2, 3, 7, 0};
 
 __global__ void __launch_bounds__(kBlock) k_wgrad(WgradArgs a) {
   __shared__ float red[kBlock / 64][16];
+  __shared__ float blocks[kWgradSums][kBlock];
   const uint32_t b = blockIdx.x;
   auto wave_unit = [&](int l) {
     return (b - a.l[l].block0) * (kBlock / 64) + (threadIdx.x >> 6);
   };
-  if (b < a.l[5].block0) return wgrad_mfma<32, 16, 1, true, 2>(a.l[6], wave_unit(6));
-  if (b < a.l[1].block0) return wgrad_mfma<64, 32, 1, true, 2>(a.l[5], wave_unit(5));
-  if (b < a.l[4].block0) return wgrad_mfma<16, 32, 2, false, 1>(a.l[1], wave_unit(1));
-  if (b < a.l[2].block0) return wgrad_mfma<64, 64, 1, true, 2>(a.l[4], wave_unit(4));
-  if (b < a.l[3].block0) return wgrad_mfma<32, 64, 2, false, 2>(a.l[2], wave_unit(2));
-  if (b < a.l[7].block0) return wgrad_mfma<64, 64, 2, false, 2>(a.l[3], wave_unit(3));
+  if (b < a.l[5].block0) return wgrad_mfma<32, 16, 1, true, 2>(a.l[6], wave_unit(6), blocks);
+  if (b < a.l[1].block0) return wgrad_mfma<64, 32, 1, true, 2>(a.l[5], wave_unit(5), blocks);
+  if (b < a.l[4].block0) return wgrad_mfma<16, 32, 2, false, 1>(a.l[1], wave_unit(1), blocks);
+  if (b < a.l[2].block0) return wgrad_mfma<64, 64, 1, true, 2>(a.l[4], wave_unit(4), blocks);
+  if (b < a.l[3].block0) return wgrad_mfma<32, 64, 2, false, 2>(a.l[2], wave_unit(2), blocks);
+  if (b < a.l[7].block0) return wgrad_mfma<64, 64, 2, false, 2>(a.l[3], wave_unit(3), blocks);
   if (b < a.l[0].block0) return wgrad_thin<true>(a.l[7], nullptr, b - a.l[7].block0, red);
   wgrad_thin<false>(a.l[0], a.x32, b - a.l[0].block0, red);
 }
