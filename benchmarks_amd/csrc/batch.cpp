@@ -14,9 +14,10 @@
 // vertices (patch.hip), over the concatenated patches of all instances of
 // that degree.  At creation an autotuner may time the tile variants of the
 // collocation kernel (cells per workgroup, G prefetch) and the patch kernel
-// per degree on the batch's own cells and keep the fastest.  The CG steps of a
-// small batch use neither: they run in three launches, one of which applies the
-// operators of all degrees (small_batch).
+// per degree on the batch's own cells and keep the fastest.  The variants are
+// those of the vmult and of a large batch's CG steps; the steps of a small batch
+// run in three launches, one of which applies the operators of all degrees, whatever
+// the variants (small_batch).
 #include <algorithm>
 #include <chrono>
 #include <memory>
@@ -80,7 +81,7 @@ struct mfx_batch {
   DBuf<PapRange> pap_ranges;
   DBuf<double> part_c;  // constrained-row share of p.Ap per segment
   // a small batch: tiles of all degrees for one launch, ordered by instance
-  bool small = false, chosen = false;  // chosen: a variant was set by the caller
+  bool small = false;
   DBuf<BatchTile> tiles;
   DBuf<uint32_t> inst_tile;
   DBuf<double> part_t;  // p.Ap per tile
@@ -124,7 +125,7 @@ struct mfx_batch {
   // kGraphSteps CG steps; the states are st[0..n) before and after
   void steps(double *x, const double *dinv, hipStream_t s) {
     const uint32_t n = (uint32_t)ops.size();
-    if (!small || chosen) {
+    if (!small) {
       for (int k = 0; k < kGraphSteps; ++k) cg_step(x, dinv, s);
       return;
     }
@@ -204,7 +205,7 @@ void autotune(mfx_batch &b, hipStream_t s) {
 }
 
 // Whether the CG steps run in three launches (k_b_direction_small and after in
-// batch_kernels.hip), unless the caller chose a variant.  A step then took, us
+// batch_kernels.hip).  A step then took, us
 // against the separate launches with tuned variants: 18 against 36 (one problem,
 // 36k rows), 28 against 53 (0.49M), 52 against 96 (five degrees, 1.2M), 136 against
 // 160 (7.8M points), 210 against 262 (64 problems, 11.4M points), 298 against 297
@@ -490,7 +491,6 @@ mfx_status mfx_batch_set_variant(mfx_batch *b, int degree, int variant) {
       if (g.p != degree) continue;
       MFX_REQUIRE(variant >= 0 && variant < g.n_variants(), "variant out of range");
       g.variant = variant;
-      b->chosen = true;
       return;
     }
     throw Error{MFX_ERR_INVALID_ARG, "no instance of degree " + std::to_string(degree)};

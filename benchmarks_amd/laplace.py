@@ -462,7 +462,8 @@ class BatchedLaplace:
                 "geometry": [geo[g] for g in list(t.geometry)[:nv]], "ms": list(t.ms)[:nv]}
 
     def set_variant(self, degree: int, variant: int) -> None:
-        """Use tuning variant `variant` for the instances of `degree`."""
+        """Use tuning variant `variant` for the instances of `degree`, in vmult and in
+        the CG steps of a large batch (a small batch's steps have their own kernel)."""
         check(lib().mfx_batch_set_variant(self._h, degree, variant))
 
     def solve(self, x: torch.Tensor, b: torch.Tensor, inverse_diagonal=None, max_steps=100000,

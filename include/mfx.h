@@ -369,7 +369,12 @@ typedef struct {
   int degree;
   uint32_t n_cells;            /* cells of this degree over all instances */
   int n_variants;              /* tile variants of the collocation kernel */
-  int variant;                 /* the one in use */
+  int variant;                 /* the one in use: by mfx_batch_vmult, and by the steps of
+                                  mfx_batch_cg_solve on a large batch.  The steps of a small
+                                  one (at most 12M cell points (p+1)^3 n_cells over all
+                                  instances, none larger than about 0.75M DoFs at degree 2
+                                  to 2.1M at degree 6) apply all degrees in one launch of
+                                  their own kernel, whichever variants are in use */
   int default_variant;         /* the library's default tile */
   int cells_per_workgroup[8];  /* per variant (cells per patch for the patch kernel) */
   int prefetch[8];             /* per variant: metric terms loaded ahead */
@@ -392,7 +397,7 @@ mfx_status mfx_batch_offsets(const mfx_batch *batch, uint64_t *offsets /* n + 1 
 mfx_op *mfx_batch_instance_operator(mfx_batch *batch, int instance);
 mfx_status mfx_batch_get_tuning(const mfx_batch *batch, int degree, mfx_batch_tuning *tuning);
 /* use variant `variant` (0 .. n_variants - 1 of the tuning record) for the
- * instances of `degree` */
+ * instances of `degree`, where variants are used (see the record) */
 mfx_status mfx_batch_set_variant(mfx_batch *batch, int degree, int variant);
 mfx_status mfx_batch_vmult(mfx_batch *batch, double *dst, const double *src, void *stream);
 mfx_status mfx_batch_inverse_diagonal(mfx_batch *batch, double *inv, void *stream);
