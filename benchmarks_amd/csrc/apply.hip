@@ -927,14 +927,42 @@ void launch_cv(const double *D, const double *G, const double *src, double *dst,
                      src, dst, map, n_cells, nullptr, nullptr, cell_inst, inst_done);
   MFX_HIP(hipGetLastError());
 }
-template <int NQ, int E0, int E1, int E2>
+template <int NQ>
+constexpr int kVariantCells[3] = {0, 0, 0};
+template <>
+constexpr int kVariantCells<3>[3] = {7, 14, 28};
+template <>
+constexpr int kVariantCells<4>[3] = {4, 8, 16};
+template <>
+constexpr int kVariantCells<5>[3] = {2, 5, 10};
+template <>
+constexpr int kVariantCells<6>[3] = {1, 3, 7};
+template <>
+constexpr int kVariantCells<7>[3] = {1, 2, 5};
+// variant v: cells [v / 2], with the prefetch for even v
+constexpr bool variant_prefetch(int v) { return v % 2 == 0; }
+
+// the variant that is the default tile of launch_apply
+template <int NQ>
+constexpr int default_variant() {
+  for (int v = 0; v < 6; ++v)
+    if (kVariantCells<NQ>[v / 2] == CollocTile<NQ>::EPB &&
+        variant_prefetch(v) == CollocTile<NQ>::PREFETCH)
+      return v;
+  return -1;
+}
+static_assert(default_variant<3>() >= 0 && default_variant<4>() >= 0 && default_variant<5>() >= 0 &&
+                  default_variant<6>() >= 0 && default_variant<7>() >= 0,
+              "the default tile is among the variants");
+
+template <int NQ>
 void launch_cv_sel(int v, int *epb, int *pref, const double *D, const double *G, const double *src,
                    double *dst, const uint32_t *map, uint32_t n, const uint16_t *ci,
                    const int *done, hipStream_t s) {
-  const int e[3] = {E0, E1, E2};
+  constexpr int E0 = kVariantCells<NQ>[0], E1 = kVariantCells<NQ>[1], E2 = kVariantCells<NQ>[2];
   MFX_REQUIRE(v >= 0 && v < 6, "tile variant out of range");
-  *epb = e[v / 2];
-  *pref = (v % 2 == 0);
+  *epb = kVariantCells<NQ>[v / 2];
+  *pref = variant_prefetch(v);
   if (!src) return;  // description only
   if (n == 0) return;
   switch (v) {
@@ -952,13 +980,12 @@ void launch_cv_sel(int v, int *epb, int *pref, const double *D, const double *G,
 int colloc_variant_count(int p) { return (p >= 2 && p <= 6) ? 6 : 0; }
 
 int colloc_default_variant(int p) {
-  // the variant equal to the default tile (CollocTile) of launch_apply
   switch (p) {
-    case 2: return 2;  // 14 cells, prefetch
-    case 3: return 2;  // 8 cells, prefetch
-    case 4: return 2;  // 5 cells, prefetch
-    case 5: return 2;  // 3 cells, prefetch
-    case 6: return 0;  // 1 cell, prefetch
+    case 2: return default_variant<3>();
+    case 3: return default_variant<4>();
+    case 4: return default_variant<5>();
+    case 5: return default_variant<6>();
+    case 6: return default_variant<7>();
     default: return 0;
   }
 }
@@ -969,11 +996,11 @@ void launch_colloc_variant(int p, int v, const double *D, const double *G, const
                            int *epb, int *prefetch) {
   int e = 0, pf = 0;
   switch (p) {
-    case 2: launch_cv_sel<3, 7, 14, 28>(v, &e, &pf, D, G, src, dst, map, n_cells, cell_inst, inst_done, s); break;
-    case 3: launch_cv_sel<4, 4, 8, 16>(v, &e, &pf, D, G, src, dst, map, n_cells, cell_inst, inst_done, s); break;
-    case 4: launch_cv_sel<5, 2, 5, 10>(v, &e, &pf, D, G, src, dst, map, n_cells, cell_inst, inst_done, s); break;
-    case 5: launch_cv_sel<6, 1, 3, 7>(v, &e, &pf, D, G, src, dst, map, n_cells, cell_inst, inst_done, s); break;
-    case 6: launch_cv_sel<7, 1, 2, 5>(v, &e, &pf, D, G, src, dst, map, n_cells, cell_inst, inst_done, s); break;
+    case 2: launch_cv_sel<3>(v, &e, &pf, D, G, src, dst, map, n_cells, cell_inst, inst_done, s); break;
+    case 3: launch_cv_sel<4>(v, &e, &pf, D, G, src, dst, map, n_cells, cell_inst, inst_done, s); break;
+    case 4: launch_cv_sel<5>(v, &e, &pf, D, G, src, dst, map, n_cells, cell_inst, inst_done, s); break;
+    case 5: launch_cv_sel<6>(v, &e, &pf, D, G, src, dst, map, n_cells, cell_inst, inst_done, s); break;
+    case 6: launch_cv_sel<7>(v, &e, &pf, D, G, src, dst, map, n_cells, cell_inst, inst_done, s); break;
     default: throw Error{MFX_ERR_UNSUPPORTED, "tile variants exist for degrees 2..6"};
   }
   if (epb) *epb = e;
