@@ -30,12 +30,12 @@ using namespace mfx;
 // the trilinear metric holds out longest where its cells fill the lanes best:
 // FP64 p = 4, q = 6 is level at any size, FP32 p = 4, q = 5 3% ahead up to 20M DoFs.
 // There is no instance where the planes do not fit the registers (FP64 q >= 8,
-// FP32 q >= 9).
+// FP32 q >= 9), nor for FP32 p = 4, q = 5 with the trilinear metric.
 static bool plane_rule(const mfx_op &op, bool fp32) {
-  if (fp32 ? !plane_instance<float>(op.p, op.nq, op.colloc)
-           : !plane_instance<double>(op.p, op.nq, op.colloc))
-    return false;
   const bool axes = op.box.deform == 0.0;
+  if (fp32 ? !plane_instance<float>(op.p, op.nq, op.colloc, axes)
+           : !plane_instance<double>(op.p, op.nq, op.colloc, axes))
+    return false;
   const int q = op.nq;
   const bool over = q == op.p + 2;  // more points than the stiffness of affine cells needs
   uint64_t need;
@@ -46,7 +46,7 @@ static bool plane_rule(const mfx_op &op, bool fp32) {
   else if (axes)
     need = fp32 ? (q <= 5 ? 1536 : over ? 4096 : 2048) : (q <= 5 ? 1024 : q == 6 ? 2048 : 5120);
   else if (fp32)
-    need = q <= 3 ? 1024 : q == 4 ? 4096 : q == 5 ? (over ? 12288 : ~0ull) : over && q >= 7 ? 8192 : 6144;
+    need = q <= 3 ? 1024 : q == 4 ? 4096 : q == 5 ? 12288 : over && q >= 7 ? 8192 : 6144;
   else
     need = q <= 4 ? 1024 : q == 5 ? (over ? 1024 : 6144) : q == 6 ? 16384 : 8192;
   return (uint64_t)op.plane_lay.groups * op.plane_lay.n[2] >= need;

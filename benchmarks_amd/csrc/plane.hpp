@@ -30,7 +30,7 @@ struct PlaneOp {
 
 // whether the kernel has an instance for the operator's form
 template <typename T>
-bool plane_instance(int p, int nq, bool colloc);
+bool plane_instance(int p, int nq, bool colloc, bool axes);
 // dst += A src over the free rows; fresh: dst is zero on the free rows, so that
 // sums only one wave forms may be stored instead of added
 template <typename T>

@@ -3,7 +3,7 @@
 
 namespace mfx {
 
-template bool plane_instance<float>(int, int, bool);
+template bool plane_instance<float>(int, int, bool, bool);
 template void launch_plane<float>(const PlaneOp<float> &, const float *, float *, bool, hipStream_t,
                                   double *, const int *);
 

@@ -6,7 +6,7 @@
 
 namespace mfx {
 
-template bool plane_instance<double>(int, int, bool);
+template bool plane_instance<double>(int, int, bool, bool);
 template void launch_plane<double>(const PlaneOp<double> &, const double *, double *, bool,
                                    hipStream_t, double *, const int *);
 
