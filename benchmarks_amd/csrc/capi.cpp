@@ -423,7 +423,13 @@ mfx_status mfx_op_create(const mfx_op_desc *d, mfx_op **out) {
                 "collocation kernel works on patches of a box mesh)");
     const uint64_t nm3 = (uint64_t)(d->degree + 1) * (d->degree + 1) * (d->degree + 1);
     const uint64_t nmap = (uint64_t)d->n_cells * nm3;
-    for (uint64_t i = 0; i < nmap; ++i)
+    // (MFX_INVALID_DOF + 1 is 0.)  Without a branch per entry the compiler vectorizes
+    // the check, a third of a creation: Q_2 on 190k cells 3.8 -> 2.7 ms, Q_4 on
+    // 22.7k cells 1.4-1.7 -> 1.0
+    uint32_t bad = 0;
+    const uint32_t n_dofs = (uint32_t)d->n_dofs;
+    for (uint64_t i = 0; i < nmap; ++i) bad |= (uint32_t)(d->map[i] + 1u > n_dofs);
+    for (uint64_t i = 0; bad && i < nmap; ++i)
       MFX_REQUIRE(d->map[i] == MFX_INVALID_DOF || d->map[i] < d->n_dofs,
                   "map entry out of range at " + std::to_string(i));
     for (uint64_t i = 0; i < d->n_constrained; ++i)
