@@ -493,10 +493,12 @@ struct WgradArgs {
 // on large grids a unit has hundreds of chunks, and one chain over all of them
 // would round that often (257 x 129 x 129 nodes: 1044 chunks, 16 + 66 roundings
 // instead).  The sums over the blocks wait in the LDS: in registers they cost the
-// fourth wave per SIMD (33^3 grid 201 -> 205 us, 129^3 3781 -> 3927).
+// fourth wave per SIMD (33^3 grid 201 -> 205 us, 129^3 3781 -> 3927).  LONG: some unit
+// has more than one block; the launch without it keeps the small grids' time (33^3 201 us,
+// 202-203 with it).
 constexpr uint32_t kSumChunks = 16;
 constexpr int kWgradSums = 24;  // of a lane: 3 taps x 2 channel tiles x 4
-template <int CIN, int COUT, int STRIDE, bool UP, int CTW>
+template <bool LONG, int CIN, int COUT, int STRIDE, bool UP, int CTW>
 __device__ __forceinline__ void wgrad_mfma(const WgradLayer &L, uint32_t unit,
                                            float (*blocks)[kBlock]) {
   static_assert(3 * CTW * 4 <= kWgradSums, "block sums");
@@ -520,7 +522,7 @@ __device__ __forceinline__ void wgrad_mfma(const WgradLayer &L, uint32_t unit,
 #pragma unroll
     for (int b = 0; b < CTW; ++b) acc[t][b] = v4f{0.f, 0.f, 0.f, 0.f};
   for (uint32_t k = k0; k < k1; ++k) {
-    if (k > k0 && (k - k0) % kSumChunks == 0) {
+    if (LONG && k > k0 && (k - k0) % kSumChunks == 0) {
 #pragma unroll
       for (int t = 0; t < 3; ++t)
 #pragma unroll
@@ -609,7 +611,7 @@ __device__ __forceinline__ void wgrad_mfma(const WgradLayer &L, uint32_t unit,
       for (int r = 0; r < 4; ++r) {
         const int o = ot * 16 + 4 * g + r, c = (cg * CTW + b) * 16 + li;
         float v = acc[t][b][r];
-        if (k1 - k0 > kSumChunks) v += blocks[(t * CTW + b) * 4 + r][threadIdx.x];
+        if (LONG && k1 - k0 > kSumChunks) v += blocks[(t * CTW + b) * 4 + r][threadIdx.x];
         L.part[(((uint64_t)pi * COUT + o) * 27 + zy * 3 + t) * CIN + c] = v;
       }
 }
@@ -668,19 +670,20 @@ __device__ __forceinline__ void wgrad_thin(const WgradLayer &L, const float *x32
 // block ranges in the order of the layers below (longest units first)
 constexpr int kWgradOrder[8] = {6, 5, 1, 4, 2, 3, 7, 0};
 
+template <bool LONG>
 __global__ void __launch_bounds__(kBlock) k_wgrad(WgradArgs a) {
   __shared__ float red[kBlock / 64][16];
-  __shared__ float blocks[kWgradSums][kBlock];
+  __shared__ float blocks[LONG ? kWgradSums : 1][kBlock];
   const uint32_t b = blockIdx.x;
   auto wave_unit = [&](int l) {
     return (b - a.l[l].block0) * (kBlock / 64) + (threadIdx.x >> 6);
   };
-  if (b < a.l[5].block0) return wgrad_mfma<32, 16, 1, true, 2>(a.l[6], wave_unit(6), blocks);
-  if (b < a.l[1].block0) return wgrad_mfma<64, 32, 1, true, 2>(a.l[5], wave_unit(5), blocks);
-  if (b < a.l[4].block0) return wgrad_mfma<16, 32, 2, false, 1>(a.l[1], wave_unit(1), blocks);
-  if (b < a.l[2].block0) return wgrad_mfma<64, 64, 1, true, 2>(a.l[4], wave_unit(4), blocks);
-  if (b < a.l[3].block0) return wgrad_mfma<32, 64, 2, false, 2>(a.l[2], wave_unit(2), blocks);
-  if (b < a.l[7].block0) return wgrad_mfma<64, 64, 2, false, 2>(a.l[3], wave_unit(3), blocks);
+  if (b < a.l[5].block0) return wgrad_mfma<LONG, 32, 16, 1, true, 2>(a.l[6], wave_unit(6), blocks);
+  if (b < a.l[1].block0) return wgrad_mfma<LONG, 64, 32, 1, true, 2>(a.l[5], wave_unit(5), blocks);
+  if (b < a.l[4].block0) return wgrad_mfma<LONG, 16, 32, 2, false, 1>(a.l[1], wave_unit(1), blocks);
+  if (b < a.l[2].block0) return wgrad_mfma<LONG, 64, 64, 1, true, 2>(a.l[4], wave_unit(4), blocks);
+  if (b < a.l[3].block0) return wgrad_mfma<LONG, 32, 64, 2, false, 2>(a.l[2], wave_unit(2), blocks);
+  if (b < a.l[7].block0) return wgrad_mfma<LONG, 64, 64, 2, false, 2>(a.l[3], wave_unit(3), blocks);
   if (b < a.l[0].block0) return wgrad_thin<true>(a.l[7], nullptr, b - a.l[7].block0, red);
   wgrad_thin<false>(a.l[0], a.x32, b - a.l[0].block0, red);
 }
@@ -917,8 +920,11 @@ void nn_wgrad(const NnWgrad (&l)[8], const float *x32, float *grad, hipStream_t 
   ReduceArgs r;
   a.x32 = x32;
   uint32_t block = 0;
+  bool long_units = false;
   for (int k : kWgradOrder) {
     const bool thin = k == 0 || k == 7;
+    const uint64_t chunks = ((uint64_t)l[k].od[0] * l[k].od[1] * l[k].od[2] + 31) / 32;
+    long_units = long_units || (!thin && chunks > (uint64_t)kSumChunks * l[k].n_parts);
     a.l[k] = WgradLayer{l[k].in, l[k].G, l[k].part, D3(l[k].od), D3(l[k].id), l[k].n_parts, block};
     block += thin ? 27 * l[k].n_parts
                   : (units[k] * l[k].n_parts + kBlock / 64 - 1) / (kBlock / 64);
@@ -931,7 +937,10 @@ void nn_wgrad(const NnWgrad (&l)[8], const float *x32, float *grad, hipStream_t 
     w += l[k].n_weights;
   }
   r.w0[8] = w;
-  hipLaunchKernelGGL(k_wgrad, dim3(block), dim3(kBlock), 0, s, a);
+  if (long_units)
+    hipLaunchKernelGGL(k_wgrad<true>, dim3(block), dim3(kBlock), 0, s, a);
+  else
+    hipLaunchKernelGGL(k_wgrad<false>, dim3(block), dim3(kBlock), 0, s, a);
   hipLaunchKernelGGL(k_wgrad_reduce, dim3((w + 63) / 64), dim3(kBlock), 0, s, r, grad);
   MFX_HIP(hipGetLastError());
 }
