@@ -16,13 +16,14 @@
 //   * the map and G are read with the column index fastest, so every load
 //     instruction of a wavefront touches contiguous 8-byte runs (G layout
 //     [cell][6][q^3], x fastest);
-//   * collocation kernel: the 6 q-columns of G a thread needs are loaded into
-//     registers before the first barrier, so the geometry stream is in flight
-//     while the dependent map -> src gather completes;
+//   * collocation kernel: where the registers allow (CollocTile), the 6 q-columns
+//     of G a thread needs are loaded into them before the first barrier, so the
+//     geometry stream is in flight while the dependent map -> src gather completes;
 //   * scatter: hardware FP64/FP32 atomic add in L2 (global_atomic_add_f64).
-// Cells per workgroup and the prefetch switch were chosen per nq by timing
-// the p = 2/4/6/8 BP5 operators at ~32M DoFs (a remap of workgroups onto
-// XCD-contiguous cell ranges was measured too and did not pay).
+// Cells per workgroup and the prefetch switch were chosen per nq by timing, at nq =
+// 5 on 32M DoFs and at nq = 6 and 7 on 1.5M to 6M of general meshes in FP64, FP32 and the
+// E-vector form (a remap of workgroups onto XCD-contiguous cell ranges was
+// measured too and did not pay).
 #include <type_traits>
 
 #include "mfx_internal.hpp"
@@ -40,12 +41,20 @@ struct Tile {
 };
 // Without the prefetch of G (its registers) nq = 6 and 7 run 112 and 104 us instead of
 // 134 and 126 on 4M DoFs, nq = 6 with 7 cells (3 with the prefetch); nq = 5 is faster
-// with it, 5 cells (142, 174 without) and 10 cells 173.
-template <int NQ>
+// with it, 5 cells (142, 174 without) and 10 cells 173.  FP32 needs half the
+// registers: nq = 7 is faster with the prefetch (1.5M DoFs 35.0, 38.0 without; 6M 113,
+// 122).  The E-vector form keeps it at nq = 6 too, with 3 cells (32.9 / 35.2, 109 / 127):
+// it has no faces to join, which is what 7 cells are better for.
+template <typename T, int NQ, bool GATHER = true>
 struct CollocTile {
-  static constexpr int EPB = NQ <= 5 ? 128 / (NQ * NQ) : NQ == 6 ? 7 : NQ == 7 ? 1 : NQ == 8 ? 2 : 3;
+  static constexpr int EPB = NQ <= 5   ? 128 / (NQ * NQ)
+                             : NQ == 6 ? (GATHER ? 7 : 3)
+                             : NQ == 7 ? 1
+                             : NQ == 8 ? 2
+                                       : 3;
   static constexpr int THREADS = EPB * NQ * NQ;
-  static constexpr bool PREFETCH = NQ <= 5;
+  static constexpr bool PREFETCH =
+      NQ <= 5 || (NQ == 6 && !GATHER) || (NQ == 7 && sizeof(T) == 4);
 };
 
 // A metric term.  A row of nq^2 terms that does not end at a 128-byte line shares
@@ -57,10 +66,11 @@ struct CollocTile {
 // Rows of whole lines are read once (FP64 q = 4 783 kept, 761 streamed), and of
 // long rows the shared line is too little to make up for what the stream
 // evicts (FP64 q = 6 441 kept, 427 streamed; q = 9 347, 328).
-template <typename T, int NQ>
+// STREAM: stream whatever the length (kCollocStream).
+template <typename T, int NQ, bool STREAM = false>
 __device__ __forceinline__ T load_geo(const T *p) {
   constexpr int kRow = NQ * NQ * sizeof(T);
-  if constexpr (kRow % 128 == 0 || kRow > 256)
+  if constexpr (STREAM || kRow % 128 == 0 || kRow > 256)
     return __builtin_nontemporal_load(p);
   else
     return *p;
@@ -92,7 +102,19 @@ __device__ __forceinline__ double block_sum(double v, double *red) {
 // EPB cells per workgroup; PREF: G columns loaded into registers before the
 // first barrier.  cell_inst / inst_done (optional): cells whose instance is
 // flagged done are skipped (batched solves).
-template <typename T, int NQ, int EPB, bool PREF, bool GATHER, bool DOT>
+// JOIN: a face node that the map gives to two consecutive cells is added once (see
+// k_apply_interp).  Not at nq = 5, where its registers beside the prefetched G cost
+// more (68 -> 72 us); at nq = 9 by join_colloc.
+template <int NQ, int EPB, bool PREF>
+constexpr bool kCollocJoin = EPB > 2 && !(PREF && NQ >= 5);
+// The prefetched rows of about 200 bytes, FP32 nq = 7, are streamed at any size (kept:
+// 1.5M DoFs 35.7 -> 35.0 us, 3M 61.1 -> 62.5, 6M 109 -> 113); FP64 nq = 5 by stream_colloc.
+template <typename T, int NQ>
+constexpr bool kCollocStream = sizeof(T) == 4 && NQ == 7;
+constexpr uint64_t kMemorySideCache = 256ull << 20;
+template <typename T, int NQ, int EPB, bool PREF, bool GATHER, bool DOT,
+          bool JOIN = GATHER && kCollocJoin<NQ, EPB, PREF>,
+          bool STREAM = kCollocStream<T, NQ>>
 __global__ void __launch_bounds__(EPB * NQ * NQ)
 k_apply_colloc(const T *__restrict__ gD, const T *__restrict__ G,
                const T *__restrict__ src, T *__restrict__ dst,
@@ -106,9 +128,7 @@ k_apply_colloc(const T *__restrict__ gD, const T *__restrict__ G,
   __shared__ T sfx[EPB][NQ3];
   __shared__ T sfy[EPB][NQ3];
   __shared__ double red[(THREADS + 63) / 64];
-  // the DoFs of the cells' left and right x faces (see k_apply_interp's JOIN; at
-  // nq = 5 its registers beside the prefetched G cost more: 68 -> 72 us)
-  constexpr bool JOIN = GATHER && EPB > 2 && !(PREF && NQ >= 5);
+  // JOIN: the DoFs of the cells' left and right x faces
   __shared__ uint32_t sL[JOIN ? EPB * NQ2 : 1], sR[JOIN ? EPB * NQ2 : 1];
 
   if (skip && *skip) return;  // converged CG: nothing left to do
@@ -129,7 +149,7 @@ k_apply_colloc(const T *__restrict__ gD, const T *__restrict__ G,
 #pragma unroll
     for (int z = 0; z < NQ; ++z)
 #pragma unroll
-      for (int c = 0; c < 6; ++c) g[c][z] = load_geo<T, NQ>(Ge + c * NQ3 + z * NQ2);
+      for (int c = 0; c < 6; ++c) g[c][z] = load_geo<T, NQ, STREAM>(Ge + c * NQ3 + z * NQ2);
   }
 
   uint32_t idx[NQ];
@@ -167,12 +187,12 @@ k_apply_colloc(const T *__restrict__ gD, const T *__restrict__ G,
         gxx = g[0][z]; gxy = g[1][z]; gxz = g[2][z];
         gyy = g[3][z]; gyz = g[4][z]; gzz = g[5][z];
       } else {
-        gxx = load_geo<T, NQ>(Ge + 0 * NQ3 + z * NQ2);
-        gxy = load_geo<T, NQ>(Ge + 1 * NQ3 + z * NQ2);
-        gxz = load_geo<T, NQ>(Ge + 2 * NQ3 + z * NQ2);
-        gyy = load_geo<T, NQ>(Ge + 3 * NQ3 + z * NQ2);
-        gyz = load_geo<T, NQ>(Ge + 4 * NQ3 + z * NQ2);
-        gzz = load_geo<T, NQ>(Ge + 5 * NQ3 + z * NQ2);
+        gxx = load_geo<T, NQ, STREAM>(Ge + 0 * NQ3 + z * NQ2);
+        gxy = load_geo<T, NQ, STREAM>(Ge + 1 * NQ3 + z * NQ2);
+        gxz = load_geo<T, NQ, STREAM>(Ge + 2 * NQ3 + z * NQ2);
+        gyy = load_geo<T, NQ, STREAM>(Ge + 3 * NQ3 + z * NQ2);
+        gyz = load_geo<T, NQ, STREAM>(Ge + 4 * NQ3 + z * NQ2);
+        gzz = load_geo<T, NQ, STREAM>(Ge + 5 * NQ3 + z * NQ2);
       }
       T dx = 0, dy = 0, dz = 0;
 #pragma unroll
@@ -259,8 +279,18 @@ k_apply_colloc(const T *__restrict__ gD, const T *__restrict__ G,
 // FP atomics execute beyond the per-XCD L2s, and their request count bounds
 // the per-cell scatter (measured: plain stores in their place made the FP32
 // q = p+1 apply at 135M DoFs 2.1x faster).
+//
+// JOIN (a DoF map, any mesh): a face node that the map gives to both of two consecutive
+// cells is added once, with the first cell's column: in an adapter's numbering a
+// cell's left face lies strided in its neighbour's DoFs, a request per node or two.  On
+// 1.75M DoFs, Gauss: p = 2, q = 3 143 -> 94 us, p = 4, q = 6 107 -> 91; p = 1 collocated
+// 257 -> 143.  Not where the node columns are under half of the lanes (p = 1, q = 3:
+// 374 -> 453 us with the metric from the vertices) or with few cells (q = 9 64 -> 66,
+// q = 10 78 -> 84).  It costs a barrier and a pass through the LDS: join_faces.
+template <int NM, int NQ>
+constexpr bool kJoin = Tile<NQ>::EPB > 3 && 2 * NM * NM >= NQ * NQ;
 template <typename T, int NM, int NQ, bool GATHER, bool DOT, bool OTF = false, bool ROW = false,
-          bool AX = false>
+          bool AX = false, bool JOIN = GATHER && !ROW && kJoin<NM, NQ>>
 __global__ void __launch_bounds__(Tile<NQ>::THREADS)
 k_apply_interp(const T *__restrict__ gB, const T *__restrict__ gD,
                const T *__restrict__ G, const T *__restrict__ src,
@@ -281,15 +311,8 @@ k_apply_interp(const T *__restrict__ gB, const T *__restrict__ gD,
   __shared__ T sXv[OTF ? EPB * 24 : 1];  // cell vertices, then
   __shared__ T sKc[OTF ? EPB * 21 : 1];  // per cell 7 Jacobian coefficient vectors
   __shared__ double red[(Tile<NQ>::THREADS + 63) / 64];
-  // JOIN (a DoF map, any mesh): the DoFs of the cells' left and right x faces.  A
-  // face node that the map gives to both of two consecutive cells is added once,
-  // with the first cell's column: in an adapter's numbering a cell's left face lies
-  // strided in its neighbour's DoFs, a request per node or two.  On 1.75M DoFs,
-  // Gauss: p = 2, q = 3 143 -> 94 us, p = 4, q = 6 107 -> 91; p = 1 collocated
-  // 257 -> 143.  Not
-  // where the node columns are under half of the lanes (p = 1, q = 3: 374 -> 453 us
-  // with the metric from the vertices) or with few cells (q = 9 64 -> 66, q = 10 78 -> 84).
-  constexpr bool JOIN = GATHER && !ROW && EPB > 3 && 2 * NM2 >= NQ2;
+  // JOIN: the DoFs of the cells' left and right x faces
+  static_assert(!JOIN || (GATHER && !ROW && kJoin<NM, NQ>), "faces are joined through a map");
   __shared__ uint32_t sL[JOIN ? EPB * NM2 : 1], sR[JOIN ? EPB * NM2 : 1];
 
   if (skip && *skip) return;  // converged CG: nothing left to do
@@ -824,63 +847,134 @@ k_apply_interp(const T *__restrict__ gB, const T *__restrict__ gD,
 
 // Workgroups of an apply: cells in batches of EPB, or (Gauss kernel on a box
 // mesh) EPB-cell segments of each x-row.
-template <int NQ, bool COLLOC>
+template <int NQ, bool COLLOC, bool GATHER = true>
 uint32_t n_blocks_for(uint32_t n_cells, RowMesh rows = {}) {
-  constexpr int EPB = COLLOC ? CollocTile<NQ>::EPB : Tile<NQ>::EPB;
+  constexpr int EPB = COLLOC ? CollocTile<double, NQ, GATHER>::EPB : Tile<NQ>::EPB;
   if (!COLLOC && rows.n0) return (n_cells / rows.n0) * ((rows.n0 + EPB - 1) / EPB);
   return (n_cells + EPB - 1) / EPB;
+}
+
+// Whether the Gauss kernel joins faces, where it can, at nq >= 6.  Without / with it:
+// - with at most a workgroup per CU its latency counts: raw applies of 60k DoFs, FP64, p = 4,
+//   q = 6 9.8 / 10.5 us, p = 7, q = 8 9.8 / 11.4;
+// - at q = 8 (few cells in a workgroup) it pays only where the adds it saves are a request
+//   each, not where a cell's x-lines are consecutive DoFs (scattered = false).  In the
+//   mesh's order, 6M DoFs: p = 6 FP64 211 / 228 us, FP32 130 / 136, p = 7 166 / 175; in an
+//   adapter's order, 1.5M: 75 / 73, 41 / 37, 50 / 47;
+// - with stored FP64 terms and q = p + 2 (lanes without a node) not once G's stream bounds
+//   the kernel: p = 5, q = 7 in the mesh's order 400k DoFs 20.3 / 18.6, 1.5M 63 / 65, in
+//   an adapter's 1.5M 69 / 67, 2.5M 100 / 102, 20M 723 / 747; p = 6, q = 8 4M 160 / 155, 6M
+//   228 / 227, 9M 347 / 353, 20M 716 / 743.
+// Everywhere else it gains in either order (p = 6, q = 7 170 / 152, p = 5, q = 7 with the
+// metric from the vertices 179 / 164, FP32 6M DoFs 142 / 121).
+template <typename T, int NM, int NQ, bool OTF>
+bool join_faces(uint32_t blocks, bool scattered) {
+  if (blocks <= 256 || (NQ == 8 && !scattered)) return false;
+  if (OTF || sizeof(T) == 4 || NM == NQ || NQ == 6) return true;
+  if (NQ == 7) return blocks <= (scattered ? 2816 : 1024);
+  return blocks <= 8192;
+}
+
+// The same for the collocation kernel at nq = 9.  FP64: not on a few CUs (27 cells 10.6 ->
+// 11.2 us, 125 cells 12.5 -> 11.6).  FP32: on many workgroups in an adapter's order while
+// G fits the memory-side cache (1.5M DoFs 30.8 -> 29.4 us; 400k 12.4 -> 14.2, 12M 197 -> 205;
+// in the mesh's order 27.9 -> 30.4).
+template <typename T, int NQ>
+bool join_colloc(uint32_t n_cells, bool scattered) {
+  const uint32_t blocks = n_blocks_for<NQ, true>(n_cells);
+  if (sizeof(T) == 8) return blocks > 16;
+  return scattered && blocks > 512 && (uint64_t)n_cells * 24 * NQ * NQ * NQ <= kMemorySideCache;
+}
+
+// Whether the collocation kernel streams G at nq = 5 in FP64: where G exceeds the
+// memory-side cache and the vectors do not, which then stay in it.  Kept / streamed: 3M
+// DoFs 107.6 / 104.9 us, 6M 197 / 190 (E-vectors 133 / 129); below 1.5M 50 / 52, above
+// 18M 488 / 490 (E-vectors of 10M 229 / 258).
+template <int NQ, bool GATHER>
+bool stream_colloc(uint32_t n_cells) {
+  constexpr int NV = GATHER ? NQ - 1 : NQ;  // DoFs of a cell per direction
+  return (uint64_t)n_cells * 48 * NQ * NQ * NQ > kMemorySideCache &&
+         (uint64_t)n_cells * 16 * NV * NV * NV <= kMemorySideCache;
+}
+
+template <typename T, int NQ, bool GATHER, bool DOT, bool JOIN, bool STREAM>
+void launch_colloc(const T *D, const T *G, const T *src, T *dst, const uint32_t *map,
+                   uint32_t n_cells, hipStream_t s, double *partials, const int *skip) {
+  using C = CollocTile<T, NQ, GATHER>;
+  const dim3 grid(n_blocks_for<NQ, true, GATHER>(n_cells)), block(C::THREADS);
+  hipLaunchKernelGGL((k_apply_colloc<T, NQ, C::EPB, C::PREFETCH, GATHER, DOT, JOIN, STREAM>), grid,
+                     block, 0, s, D, G, src, dst, map, n_cells, partials, skip, nullptr, nullptr);
+}
+
+template <typename T, int NM, int NQ, bool GATHER, bool DOT, bool OTF>
+void launch_mapped(const dim3 grid, const T *B, const T *D, const T *G, const T *src, T *dst,
+                   const uint32_t *map, uint32_t n_cells, hipStream_t s, double *partials,
+                   const int *skip, const double *cellX, const T *xq, const T *wq, const T *eo,
+                   bool scattered) {
+  constexpr bool CAN = GATHER && kJoin<NM, NQ>, ALWAYS = CAN && NQ <= 5;
+  const dim3 block(Tile<NQ>::THREADS);
+  if constexpr (CAN) {
+    if (ALWAYS || join_faces<T, NM, NQ, OTF>(grid.x, scattered)) {
+      hipLaunchKernelGGL((k_apply_interp<T, NM, NQ, true, DOT, OTF, false, false, true>), grid,
+                         block, 0, s, B, D, G, src, dst, map, n_cells, partials, skip, cellX, xq,
+                         wq, RowMesh{}, eo);
+      return;
+    }
+  }
+  if constexpr (!ALWAYS)
+    hipLaunchKernelGGL((k_apply_interp<T, NM, NQ, GATHER, DOT, OTF, false, false, false>), grid,
+                       block, 0, s, B, D, G, src, dst, map, n_cells, partials, skip, cellX, xq, wq,
+                       RowMesh{}, eo);
 }
 
 template <typename T, int NM, int NQ, bool COLLOC, bool GATHER>
 void launch_t(const T *B, const T *D, const T *G, const T *src, T *dst,
               const uint32_t *map, uint32_t n_cells, hipStream_t s,
-              double *partials, const int *skip, RowMesh rows) {
+              double *partials, const int *skip, RowMesh rows, bool scattered) {
   if (n_cells == 0) return;
   const bool row = !COLLOC && GATHER && rows.n0 > 0;
   MFX_REQUIRE(!row || (uint64_t)rows.n0 * rows.n1 * rows.n2 == n_cells, "row segments: cells of another mesh");
-  const dim3 grid(n_blocks_for<NQ, COLLOC>(n_cells, row ? rows : RowMesh{}));
   if constexpr (COLLOC) {
     static_assert(NM == NQ, "collocation needs nm == nq");
-    const dim3 block(CollocTile<NQ>::THREADS);
-    if (partials) {
-      if constexpr (std::is_same<T, double>::value && GATHER)
-        hipLaunchKernelGGL((k_apply_colloc<T, NQ, CollocTile<NQ>::EPB, CollocTile<NQ>::PREFETCH,
-                                           GATHER, true>),
-                           grid, block, 0, s, D, G, src, dst, map, n_cells, partials, skip,
-                           nullptr, nullptr);
-    } else {
-      hipLaunchKernelGGL((k_apply_colloc<T, NQ, CollocTile<NQ>::EPB, CollocTile<NQ>::PREFETCH,
-                                         GATHER, false>),
-                         grid, block, 0, s, D, G, src, dst, map, n_cells, nullptr, nullptr,
-                         nullptr, nullptr);
-    }
+    using C = CollocTile<T, NQ, GATHER>;
+    constexpr bool JOIN = GATHER && kCollocJoin<NQ, C::EPB, C::PREFETCH>;
+    auto with = [&](auto dot) {
+      constexpr bool DOT = decltype(dot)::value;
+      if constexpr (JOIN && NQ == 9)
+        if (!join_colloc<T, NQ>(n_cells, scattered))
+          return launch_colloc<T, NQ, GATHER, DOT, false, false>(D, G, src, dst, map, n_cells, s,
+                                                                 partials, skip);
+      if constexpr (NQ == 5 && sizeof(T) == 8)
+        if (stream_colloc<NQ, GATHER>(n_cells))
+          return launch_colloc<T, NQ, GATHER, DOT, JOIN, true>(D, G, src, dst, map, n_cells, s,
+                                                               partials, skip);
+      launch_colloc<T, NQ, GATHER, DOT, JOIN, kCollocStream<T, NQ>>(D, G, src, dst, map, n_cells,
+                                                                    s, partials, skip);
+    };
+    if (!partials)
+      with(std::false_type{});
+    else if constexpr (std::is_same<T, double>::value && GATHER)
+      with(std::true_type{});
   } else {
-    const dim3 block(Tile<NQ>::THREADS);
-    if (partials) {
-      if constexpr (std::is_same<T, double>::value && GATHER) {
-        if (row)
-          hipLaunchKernelGGL((k_apply_interp<T, NM, NQ, GATHER, true, false, true>), grid, block,
-                             0, s, B, D, G, src, dst, map, n_cells, partials, skip, nullptr,
-                             nullptr, nullptr, rows, (const T *)nullptr);
-        else
-          hipLaunchKernelGGL((k_apply_interp<T, NM, NQ, GATHER, true>), grid, block, 0, s, B, D,
-                             G, src, dst, map, n_cells, partials, skip, nullptr, nullptr, nullptr,
-                             RowMesh{}, (const T *)nullptr);
-      }
-    } else {
-      if constexpr (GATHER) {
+    const dim3 grid(n_blocks_for<NQ, false>(n_cells, row ? rows : RowMesh{})),
+        block(Tile<NQ>::THREADS);
+    auto with = [&](auto dot) {
+      constexpr bool DOT = decltype(dot)::value;
+      if constexpr (GATHER)
         if (row) {
-          hipLaunchKernelGGL((k_apply_interp<T, NM, NQ, GATHER, false, false, true>), grid,
-                             block, 0, s, B, D, G, src, dst, map, n_cells, nullptr, nullptr,
-                             nullptr, nullptr, nullptr, rows, (const T *)nullptr);
-          MFX_HIP(hipGetLastError());
+          hipLaunchKernelGGL((k_apply_interp<T, NM, NQ, GATHER, DOT, false, true>), grid, block, 0,
+                             s, B, D, G, src, dst, map, n_cells, partials, skip, nullptr, nullptr,
+                             nullptr, rows, (const T *)nullptr);
           return;
         }
-      }
-      hipLaunchKernelGGL((k_apply_interp<T, NM, NQ, GATHER, false>), grid, block, 0, s,
-                         B, D, G, src, dst, map, n_cells, nullptr, nullptr, nullptr, nullptr,
-                         nullptr, RowMesh{}, (const T *)nullptr);
-    }
+      launch_mapped<T, NM, NQ, GATHER, DOT, false>(grid, B, D, G, src, dst, map, n_cells, s,
+                                                   partials, skip, nullptr, nullptr, nullptr,
+                                                   nullptr, scattered);
+    };
+    if (!partials)
+      with(std::false_type{});
+    else if constexpr (std::is_same<T, double>::value && GATHER)
+      with(std::true_type{});
   }
   MFX_HIP(hipGetLastError());
 }
@@ -890,16 +984,16 @@ void launch_t(const T *B, const T *D, const T *G, const T *src, T *dst,
 template <typename T, bool GATHER>
 void dispatch(int p, int nq, bool colloc, const T *B, const T *D, const T *G,
               const T *src, T *dst, const uint32_t *map, uint32_t n,
-              hipStream_t s, double *partials, const int *skip, RowMesh rc) {
+              hipStream_t s, double *partials, const int *skip, RowMesh rc, bool scattered) {
 #define MFX_CASE_C(P)                                                         \
   case P:                                                                     \
-    return launch_t<T, P + 1, P + 1, true, GATHER>(B, D, G, src, dst, map, n, s, partials, skip, rc);
+    return launch_t<T, P + 1, P + 1, true, GATHER>(B, D, G, src, dst, map, n, s, partials, skip, rc, scattered);
 #define MFX_CASE_I(P)                                                         \
   case P:                                                                     \
     if (nq == P + 1)                                                          \
-      return launch_t<T, P + 1, P + 1, false, GATHER>(B, D, G, src, dst, map, n, s, partials, skip, rc); \
+      return launch_t<T, P + 1, P + 1, false, GATHER>(B, D, G, src, dst, map, n, s, partials, skip, rc, scattered); \
     if (nq == P + 2)                                                          \
-      return launch_t<T, P + 1, P + 2, false, GATHER>(B, D, G, src, dst, map, n, s, partials, skip, rc); \
+      return launch_t<T, P + 1, P + 2, false, GATHER>(B, D, G, src, dst, map, n, s, partials, skip, rc, scattered); \
     break;
   if (colloc) {
     MFX_REQUIRE(nq == p + 1, "collocation requires nq == p+1");
@@ -946,8 +1040,8 @@ constexpr bool variant_prefetch(int v) { return v % 2 == 0; }
 template <int NQ>
 constexpr int default_variant() {
   for (int v = 0; v < 6; ++v)
-    if (kVariantCells<NQ>[v / 2] == CollocTile<NQ>::EPB &&
-        variant_prefetch(v) == CollocTile<NQ>::PREFETCH)
+    if (kVariantCells<NQ>[v / 2] == CollocTile<double, NQ>::EPB &&
+        variant_prefetch(v) == CollocTile<double, NQ>::PREFETCH)
       return v;
   return -1;
 }
@@ -1010,14 +1104,16 @@ void launch_colloc_variant(int p, int v, const double *D, const double *G, const
 template <typename T>
 void launch_apply(int p, int nq, bool colloc, const T *B, const T *D, const T *G,
                   const T *src, T *dst, const uint32_t *map, uint32_t n_cells,
-                  hipStream_t s, double *dot_partials, const int *skip, RowMesh rows) {
+                  hipStream_t s, double *dot_partials, const int *skip, RowMesh rows,
+                  bool scattered) {
   dispatch<T, true>(p, nq, colloc, B, D, G, src, dst, map, n_cells, s, dot_partials, skip,
-                    rows);
+                    rows, scattered);
 }
 template <typename T>
 void launch_evec(int p, int nq, bool colloc, const T *B, const T *D, const T *G,
                  const T *in, T *out, uint32_t n_cells, hipStream_t s) {
-  dispatch<T, false>(p, nq, colloc, B, D, G, in, out, nullptr, n_cells, s, nullptr, nullptr, RowMesh{});
+  dispatch<T, false>(p, nq, colloc, B, D, G, in, out, nullptr, n_cells, s, nullptr, nullptr, RowMesh{},
+                     false);
 }
 
 // Gauss (non-collocated) apply with the metric terms computed from the cell
@@ -1026,42 +1122,32 @@ template <typename T, int NM, int NQ>
 void launch_interp_otf(const T *B, const T *D, const T *eo, const T *xq, const T *wq,
                        const double *cellX, const T *src, T *dst, const uint32_t *map,
                        uint32_t n_cells, hipStream_t s, double *partials, const int *skip,
-                       RowMesh rows, bool axes) {
+                       RowMesh rows, bool axes, bool scattered) {
   MFX_REQUIRE(!axes || rows.n0, "axis-aligned cells are a box-mesh form");
   if (n_cells == 0) return;
   MFX_REQUIRE(!rows.n0 || (uint64_t)rows.n0 * rows.n1 * rows.n2 == n_cells,
               "row segments: cells of another mesh");
   const dim3 grid(n_blocks_for<NQ, false>(n_cells, rows)), block(Tile<NQ>::THREADS);
-  if (partials) {
-    if constexpr (std::is_same<T, double>::value) {
-      if (axes)
-        hipLaunchKernelGGL((k_apply_interp<T, NM, NQ, true, true, true, true, true>), grid, block,
-                           0, s, B, D, nullptr, src, dst, map, n_cells, partials, skip, cellX, xq,
-                           wq, rows, eo);
-      else if (rows.n0)
-        hipLaunchKernelGGL((k_apply_interp<T, NM, NQ, true, true, true, true>), grid, block, 0, s,
-                           B, D, nullptr, src, dst, map, n_cells, partials, skip, cellX, xq, wq,
-                           rows, eo);
-      else
-        hipLaunchKernelGGL((k_apply_interp<T, NM, NQ, true, true, true>), grid, block, 0, s, B, D,
-                           nullptr, src, dst, map, n_cells, partials, skip, cellX, xq, wq, RowMesh{},
-                           eo);
-    } else {
-      throw Error{MFX_ERR_UNSUPPORTED, "p.Ap partials are computed in FP64 only"};
-    }
-  } else if (axes) {
-    hipLaunchKernelGGL((k_apply_interp<T, NM, NQ, true, false, true, true, true>), grid, block, 0,
-                       s, B, D, nullptr, src, dst, map, n_cells, nullptr, nullptr, cellX, xq, wq,
-                       rows, eo);
-  } else if (rows.n0) {
-    hipLaunchKernelGGL((k_apply_interp<T, NM, NQ, true, false, true, true>), grid, block, 0, s, B,
-                       D, nullptr, src, dst, map, n_cells, nullptr, nullptr, cellX, xq, wq,
-                       rows, eo);
-  } else {
-    hipLaunchKernelGGL((k_apply_interp<T, NM, NQ, true, false, true>), grid, block, 0, s, B, D,
-                       nullptr, src, dst, map, n_cells, nullptr, nullptr, cellX, xq, wq, RowMesh{},
-                       eo);
-  }
+  auto with = [&](auto dot) {
+    constexpr bool DOT = decltype(dot)::value;
+    if (axes)
+      hipLaunchKernelGGL((k_apply_interp<T, NM, NQ, true, DOT, true, true, true>), grid, block, 0,
+                         s, B, D, nullptr, src, dst, map, n_cells, partials, skip, cellX, xq, wq,
+                         rows, eo);
+    else if (rows.n0)
+      hipLaunchKernelGGL((k_apply_interp<T, NM, NQ, true, DOT, true, true>), grid, block, 0, s, B,
+                         D, nullptr, src, dst, map, n_cells, partials, skip, cellX, xq, wq, rows,
+                         eo);
+    else
+      launch_mapped<T, NM, NQ, true, DOT, true>(grid, B, D, nullptr, src, dst, map, n_cells, s,
+                                                partials, skip, cellX, xq, wq, eo, scattered);
+  };
+  if (!partials)
+    with(std::false_type{});
+  else if constexpr (std::is_same<T, double>::value)
+    with(std::true_type{});
+  else
+    throw Error{MFX_ERR_UNSUPPORTED, "p.Ap partials are computed in FP64 only"};
   MFX_HIP(hipGetLastError());
 }
 
@@ -1069,16 +1155,18 @@ template <typename T>
 void launch_apply_otf(int p, int nq, const T *B, const T *D, const T *eo, const T *xq,
                       const T *wq, const double *cellX, const T *src, T *dst,
                       const uint32_t *map, uint32_t n_cells, hipStream_t s, double *partials,
-                      const int *skip, RowMesh rows, bool axes) {
+                      const int *skip, RowMesh rows, bool axes, bool scattered) {
   MFX_REQUIRE(B && D && eo && xq && wq && cellX, "on-the-fly apply: missing tables or vertices");
 #define MFX_CASE_O(P)                                                                         \
   case P:                                                                                    \
     if (nq == P + 1)                                                                         \
       return launch_interp_otf<T, P + 1, P + 1>(B, D, eo, xq, wq, cellX, src, dst, map,      \
-                                                n_cells, s, partials, skip, rows, axes); \
+                                                n_cells, s, partials, skip, rows, axes,  \
+                                                scattered);                              \
     if (nq == P + 2)                                                                         \
       return launch_interp_otf<T, P + 1, P + 2>(B, D, eo, xq, wq, cellX, src, dst, map,      \
-                                                n_cells, s, partials, skip, rows, axes); \
+                                                n_cells, s, partials, skip, rows, axes,  \
+                                                scattered);                              \
     break;
   switch (p) {
     MFX_CASE_O(1) MFX_CASE_O(2) MFX_CASE_O(3) MFX_CASE_O(4)
@@ -1093,20 +1181,20 @@ void launch_apply_otf(int p, int nq, const T *B, const T *D, const T *eo, const 
 template void launch_apply_otf<double>(int, int, const double *, const double *, const double *,
                                        const double *, const double *, const double *,
                                        const double *, double *, const uint32_t *, uint32_t,
-                                       hipStream_t, double *, const int *, RowMesh, bool);
+                                       hipStream_t, double *, const int *, RowMesh, bool, bool);
 template void launch_apply_otf<float>(int, int, const float *, const float *, const float *,
                                       const float *, const float *, const double *, const float *,
                                       float *, const uint32_t *, uint32_t, hipStream_t, double *,
-                                      const int *, RowMesh, bool);
+                                      const int *, RowMesh, bool, bool);
 
 template void launch_apply<double>(int, int, bool, const double *, const double *,
                                    const double *, const double *, double *,
                                    const uint32_t *, uint32_t, hipStream_t, double *,
-                                   const int *, RowMesh);
+                                   const int *, RowMesh, bool);
 template void launch_apply<float>(int, int, bool, const float *, const float *,
                                   const float *, const float *, float *,
                                   const uint32_t *, uint32_t, hipStream_t, double *,
-                                  const int *, RowMesh);
+                                  const int *, RowMesh, bool);
 template void launch_evec<double>(int, int, bool, const double *, const double *,
                                   const double *, const double *, double *, uint32_t,
                                   hipStream_t);

@@ -437,6 +437,16 @@ mfx_status mfx_op_create(const mfx_op_desc *d, mfx_op **out) {
     op->E = d->n_cells;
     op->N = d->n_dofs;
     op->n_cons = d->n_constrained;
+    // the cells whose middle x-line begins with consecutive DoFs
+    uint32_t lines = 0, lined = 0;
+    const uint64_t nm = d->degree + 1, middle = (nm / 2 * nm + nm / 2) * nm;
+    for (uint64_t e = 0; e < d->n_cells; ++e) {
+      const uint32_t *x = d->map + e * nm3 + middle;
+      if (x[0] == MFX_INVALID_DOF || x[1] == MFX_INVALID_DOF) continue;
+      ++lines;
+      lined += x[1] == x[0] + 1;
+    }
+    op->scattered = 2 * (uint64_t)lined < lines;
     op->map.upload(d->map, nmap);
     op->cellX.upload(d->cell_vertices, (uint64_t)d->n_cells * 24);
     op->cons.upload(d->constrained, d->n_constrained);

@@ -41,11 +41,13 @@ struct RowMesh {
 
 // Launch wrappers implemented in the .hip translation units.  Each checks
 // its arguments against what the kernel assumes and throws mfx::Error.
+// scattered (both applies): the nodes of a cell's x-lines are not consecutive DoFs
+// (for the choice of the scatter; false where it is not known).
 template <typename T>
 void launch_apply(int p, int nq, bool collocation, const T *B, const T *D,
                   const T *G, const T *src, T *dst, const uint32_t *map,
                   uint32_t n_cells, hipStream_t s, double *dot_partials = nullptr,
-                  const int *skip = nullptr, RowMesh rows = {});
+                  const int *skip = nullptr, RowMesh rows = {}, bool scattered = false);
 // Non-collocated (Gauss) apply with the metric terms of the trilinear cells
 // computed per quadrature point from their vertices (cellX [E][8][3]), xq and
 // wq the 1D quadrature points and weights on [0,1].  rows (both Gauss applies):
@@ -60,7 +62,7 @@ void launch_apply_otf(int p, int nq, const T *B, const T *D, const T *eo, const 
                       const T *wq, const double *cellX, const T *src, T *dst,
                       const uint32_t *map, uint32_t n_cells, hipStream_t s,
                       double *dot_partials = nullptr, const int *skip = nullptr,
-                      RowMesh rows = {}, bool axes = false);
+                      RowMesh rows = {}, bool axes = false, bool scattered = false);
 template <typename T>
 void launch_evec(int p, int nq, bool collocation, const T *B, const T *D,
                  const T *G, const T *in, T *out, uint32_t n_cells,
@@ -135,9 +137,9 @@ struct SineModes {
 };
 void launch_sine_modes(const double *xyz, uint64_t n, const SineModes &m, double *out,
                        hipStream_t s);
-// deterministic two-stage dot: partials[nb] then final sum into *result
 // *result = the sum of n partial sums, in a fixed order
 void launch_sum(const double *part, uint32_t n, double *result, hipStream_t s);
+// deterministic two-stage dot: partials[nb] then final sum into *result
 uint32_t dot_n_blocks(uint64_t n);
 void launch_dot(const double *x, const double *y, uint64_t n, double *partials,
                 double *result, hipStream_t s);

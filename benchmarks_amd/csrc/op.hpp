@@ -114,6 +114,7 @@ struct mfx_op {
   // a caller's map gathers constrained DoFs: their rows then receive the
   // cells' contributions, which vmult overwrites afterwards
   bool cons_in_map = false;
+  bool scattered = false;  // a caller's map: see launch_apply
   DBuf<double> G, cellX;
   DBuf<float> G32;
   // the 1D tables, in one allocation and one upload.  eo: Gauss quadrature, the
@@ -221,10 +222,10 @@ struct mfx_op {
       launch_patch<double>(patch_op64(), src, dst, s, partials, skip);
     else if (geometry == MFX_GEOM_ON_THE_FLY)
       launch_apply_otf<double>(p, nq, B.ptr, D.ptr, eo.ptr, xq.ptr, wq.ptr, cellX.ptr, src, dst,
-                               map.ptr, E, s, partials, skip, rows(), axis_cells());
+                               map.ptr, E, s, partials, skip, rows(), axis_cells(), scattered);
     else
       launch_apply<double>(p, nq, colloc, B.ptr, D.ptr, G.ptr, src, dst, map.ptr, E, s, partials,
-                           skip, rows());
+                           skip, rows(), scattered);
   }
   void apply32(const float *src, float *dst, hipStream_t s) const {
     if (plane<float>())
@@ -234,10 +235,10 @@ struct mfx_op {
     else if (geometry == MFX_GEOM_ON_THE_FLY)
       launch_apply_otf<float>(p, nq, B32.ptr, D32.ptr, eo32.ptr, xq32.ptr, wq32.ptr, cellX.ptr,
                               src, dst, map.ptr, E, s, nullptr, nullptr, rows(),
-                              axis_cells());
+                              axis_cells(), scattered);
     else
       launch_apply<float>(p, nq, colloc, B32.ptr, D32.ptr, G32.ptr, src, dst, map.ptr, E, s,
-                          nullptr, nullptr, rows());
+                          nullptr, nullptr, rows(), scattered);
   }
   // dst = A src with identity on the constrained rows
   void vmult64(const double *src, double *dst, hipStream_t s) const {
