@@ -10,8 +10,8 @@ cell counts have enough factors of two for the multigrid hierarchy to reach a
 directly solvable coarse mesh.)
 
 Each degree is measured with the metric terms stored (G, 48 q^3 B per cell,
-per-cell kernel) and computed on the fly from the cell vertices (patch
-kernel); the faster mode per degree enters the aggregate.  Also reported
+patch kernel) and computed on the fly from the cell vertices (plane kernel
+at p = 2, 4, 6, patch kernel at p = 8); the faster mode per degree enters the aggregate.  Also reported
 per degree: the apply kernel's time (HIP events on the launch stream), its
 algorithmic bytes and FLOPs, Jacobi-CG and mixed-precision multigrid CG
 time-to-1e-8 relative residual on the same operator and right-hand side, the

@@ -14,7 +14,7 @@ void vmult64(mfx_op &op, double *dst, const double *src, hipStream_t s);
 void vmult32(mfx_op &op, float *dst, const float *src, hipStream_t s);
 // `degree` Chebyshev(Jacobi) steps towards A x = b in FP32 on [lmin, lmax]
 // (t, d: scratch vectors of the operator's size).  started: t already holds
-// the start value of A x (chebyshev_start's rows); leave_start: t is left as the
+// the start value of A x (x on the constrained rows, 0 elsewhere); leave_start: t is left as the
 // start value of A x for the final x.  Both only where
 // cheb_starts(op): the apply then adds to t without a start pass of its own.
 void chebyshev(mfx_op &op, float *x, const float *b, const float *dinv, float *t, float *d,

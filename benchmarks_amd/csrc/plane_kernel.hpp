@@ -8,9 +8,9 @@
 // the y-lines z = k.  No workgroup barrier: the exchanges order within the
 // wave.  Against one lane per (x, y) column with its x and y contractions
 // through the LDS (the patch kernel and the per-column Gauss kernel) this halves
-// the LDS accesses per point (10-11 instead of 16-24) and drops the 5-9 barriers
+// the LDS instructions per point (7.5-8.7 instead of 16-20) and drops the 5-9 barriers
 // per batch of cells, which bounded those kernels.  It is bound by the vector
-// units where the metric is trilinear (busy 80% in FP32, 54% in FP64 at p = 4
+// units where the metric is trilinear (busy 76% in FP32, 51% in FP64 at p = 4
 // with two waves per SIMD), by the scatter where it is diagonal (without its
 // atomics 310 -> 253 us in FP64, 204 -> 123 in FP32).  33M DoFs, collocated
 // p = 4: FP64 undeformed 486 -> 310 us, deformed 476 -> 397; FP32 518 -> 204 and
@@ -507,7 +507,7 @@ k_plane(const T *__restrict__ eo_, const T *__restrict__ gxq, const T *__restric
     __syncthreads();  // the staging has been read
   }
   if constexpr (DOT) {
-    dot = active ? dot : 0.0;  // idle lanes have no metric
+    dot = active ? dot : 0.0;  // idle lanes repeat other lanes' or cells' work
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) dot += __shfl_xor(dot, o, 64);
     if (lane == 0) partials[blockIdx.x] = dot;

@@ -1,5 +1,5 @@
 // transfer.hpp -- grid transfers between two box operators of one box:
-// tensor products of 1D nodal-interpolation matrices (CSR, on the device),
+// tensor products of 1D nodal-interpolation matrices (spans of columns, on the device),
 // applied by the axis passes of mg_kernels.hip.  Used by the multigrid
 // (mg.cpp) and by the learned preconditioner's coarse correction (nn.cpp).
 #pragma once

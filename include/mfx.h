@@ -386,7 +386,8 @@ typedef struct {
 /* autotune != 0: time every variant per degree (the collocation kernel's
  * tiles with stored metric terms, and the patch kernel with metric terms
  * from the cell vertices) on the batch's cells and keep the fastest;
- * otherwise the default tile */
+ * otherwise the default tile.  The solves of a small batch do not use the
+ * variants, so 0 saves the timing where only they matter */
 mfx_status mfx_batch_create(const mfx_batch_instance *instances, int n_instances,
                             int autotune, mfx_batch **out);
 mfx_status mfx_batch_destroy(mfx_batch *batch);

@@ -73,3 +73,34 @@ def test_metric_larger_than_the_cache(gpu):
     y = torch.empty(P.N, dtype=torch.float64, device="cuda")
     op.vmult(y, torch.from_numpy(x).cuda())
     assert np.linalg.norm(y.cpu().numpy() - ref) <= 1e-12 * np.linalg.norm(ref)
+
+
+def _joins(op, N):
+    """Whether the apply's kernel joins faces (its last template argument)."""
+    import torch
+    from torch.profiler import ProfilerActivity, profile
+    x = torch.zeros(N, dtype=torch.float64, device="cuda")
+    y = torch.empty_like(x)
+    with profile(activities=[ProfilerActivity.CUDA]) as prof:
+        op.vmult(y, x)
+        torch.cuda.synchronize()
+    names = [e.key for e in prof.key_averages() if "k_apply_interp<" in e.key]
+    assert len(names) == 1, names
+    args = names[0].split("k_apply_interp<")[1].split(">")[0].split(",")
+    return args[8].strip() == "true"
+
+
+@pytest.mark.parametrize("p,q,n,ordered,shuffled", [
+    (4, 6, (3, 3, 3), False, False), (4, 6, (13, 12, 12), True, True),
+    (6, 8, (11, 10, 10), False, True), (7, 8, (11, 10, 10), False, True),
+    (5, 7, (11, 11, 11), True, True), (5, 7, (18, 17, 17), False, True)])
+def test_which_form_runs(gpu, p, q, n, ordered, shuffled):
+    from benchmarks_amd.laplace import LaplaceOperator
+    P = O.make_problem(p, q, O.GAUSS, n)
+    cons = np.flatnonzero(P.constrained).astype(np.uint32)
+    m = np.asarray(P.map, dtype=np.uint32)
+    perm = np.random.RandomState(1).permutation(P.N).astype(np.uint32)
+    t = np.where(m == NONE, NONE, perm[np.where(m == NONE, 0, m)]).astype(np.uint32)
+    for mm, cc, want in ((m, cons, ordered), (t, perm[cons], shuffled)):
+        op = LaplaceOperator.from_arrays(p, q, O.GAUSS, mm, P.cellX, cc, P.N)
+        assert _joins(op, P.N) == want
